@@ -30,6 +30,7 @@ SOURCES = {
     "bmi_server.hip": [],
     "bmi_space_dev.cpp": ["-x", "hip"],
     "bmi_potential.hip": [],
+    "bmi_rows.hip": [],
 }
 
 

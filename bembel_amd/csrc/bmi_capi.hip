@@ -306,12 +306,10 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
                       hipStream_t st) {
   const bmi_space* s = h->s;
   const bool C = h->cplx;
-  const int S = C ? 2 : 1;
   const int64_t N = s->nsuper;
   const int rows = h->cd;
   const int64_t vcs = static_cast<int64_t>(s->nel) * s->I2;  // super DOFs per component
   const CouplingOperand co = coupling_operand(h, reduced);
-  const int64_t cblk = co.blk;
   for (int cc = 0; cc < h->vd; ++cc) {
     TimedScope ts("matvec_forward", st);
     launch_forward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[cc].ptr, h->d_T.ptr, xs, N, cc * vcs,
@@ -332,16 +330,13 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
     }
     return;
   }
-  for (int rc = 0; rc < h->vd; ++rc) {
-    device_fill(w.bw, S * h->lvl_total * nrhs, 0.0, st);
-    for (int cc = 0; cc < h->vd; ++cc)
-      launch_coupling_apply(C, co.fp32, std::max(h->cpl_variant, 0), h->ntgt, nrhs, rows, h->d_tgt.ptr,
-                            h->d_crp.ptr, h->d_csrc.ptr, co.F, h->vd * h->vd * cblk, (rc * h->vd + cc) * cblk,
-                            h->d_lvl_off.ptr, w.fw[cc], w.bw, 1, st, co.Fc, co.ncoarse, co.ld);
-    TimedScope ts("matvec_backward", st);
-    launch_backward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[rc].ptr, h->d_T.ptr, w.bw,
-                    h->d_lvl_off.ptr, yf, N, rc * vcs, st);
-  }
+  // every cluster of every level is a target (zero where there are no blocks)
+  launch_coupling_apply(C, co.fp32, std::max(h->cpl_variant, 0), h->ntgt_all, nrhs, rows, h->d_tgt_all.ptr,
+                        h->d_crp_all.ptr, h->d_csrc.ptr, co.F, co.blk, 0, h->d_lvl_off.ptr, w.fw[0], w.bw, 0, st,
+                        co.Fc, co.ncoarse, co.ld);
+  TimedScope ts("matvec_backward", st);
+  launch_backward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[0].ptr, h->d_T.ptr, w.bw,
+                  h->d_lvl_off.ptr, yf, N, 0, st);
 }
 
 // near-field sweep: ys = A_near xs
@@ -349,12 +344,8 @@ static void apply_near(bmi_h2* h, int nrhs, const double* xs, double* ys, hipStr
   const bmi_space* s = h->s;
   const int64_t N = s->nsuper;
   const int64_t vcs = static_cast<int64_t>(s->nel) * s->I2;
-  const int64_t dblk = static_cast<int64_t>(h->dd) * h->dd;
-  for (int rc = 0; rc < h->vd; ++rc)
-    for (int cc = 0; cc < h->vd; ++cc)
-      launch_leaf(h->cplx, std::max(h->leaf_variant, 0), h->ncl_leaf, nrhs, h->dd, h->d_drp.ptr, h->d_dsrc.ptr,
-                  h->d_dense.ptr, h->vd * h->vd * dblk, (rc * h->vd + cc) * dblk, xs, N, cc * vcs, ys, N, rc * vcs,
-                  cc > 0 ? 1 : 0, st);
+  launch_leaf(h->cplx, std::max(h->leaf_variant, 0), h->ncl_leaf, nrhs, h->dd, h->vd, h->d_drp.ptr, h->d_dsrc.ptr,
+              h->d_dense.ptr, xs, N, vcs, ys, N, vcs, st);
 }
 
 // time both variants of the two sweeps once (1 RHS) and keep the faster; the variants give

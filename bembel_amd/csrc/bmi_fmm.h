@@ -13,6 +13,27 @@ constexpr int MULTI_MIN_RHS = 8;
 
 constexpr int CP_STRIDE = 12;  // doubles per cluster node: x(3) kappa ds(3) dt(3) pad(2)
 
+// block rows of up to 64 columns, any block size (bmi_rows.hip): target own (cluster own of one level,
+// or tgt[own] = (level, cluster)) takes the blocks rp[own] .. rp[own + 1], each n x n per component
+// pair (column stride ld, fblk entries apart, vd x vd of them per entry).  Scalar (row r, column
+// k) of cluster c and component m: x[level offset * nrhs + m * xseg + c * xcs + k * xks + r * xrs].
+struct RowsArgs {
+  int nown, nrhs, n, ld, vd;
+  const int2* tgt;
+  const int64_t* lvl_off;
+  const int* rp;
+  const int* src;
+  const void* F;
+  int64_t fblk;
+  const double* x;
+  int64_t xseg, xcs, xks, xrs;
+  double* y;
+  int64_t yseg, ycs, yks, yrs;
+  int accumulate;
+  int slabs, ncw;  // set by the launch: row slabs, column groups per workgroup
+};
+void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st);
+
 void launch_cluster_points(const bmi_space* s, int level, int np, const double* d_cheb, double* out,
                            hipStream_t st);
 void launch_coupling_assemble(int kind, const int4* d_leaves, int nleaves, int np2,
@@ -71,9 +92,9 @@ void launch_forward(bool cplx, int npatch, int L, int rows, int np2, int dd, int
 void launch_backward(bool cplx, int npatch, int L, int rows, int np2, int dd, int nrhs, const double* mom,
                      const double* T, double* bw, const int64_t* lvl_off, double* yf, int64_t ldy, int64_t yseg,
                      hipStream_t st);
-void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, const int* rp, const int* src, const double* F,
-                 int64_t fstride, int64_t fcomp, const double* xs, int64_t ldxs, int64_t xseg, double* ys, int64_t ldys,
-                 int64_t yseg, int accumulate, hipStream_t st);
+void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, int vd, const int* rp, const int* src,
+                 const double* F, const double* xs, int64_t ldxs, int64_t xseg, double* ys, int64_t ldys,
+                 int64_t yseg, hipStream_t st);
 // near-field sweep and coupling sweep of a single-RHS, single-component product in one launch
 // (ys written, bw written); false when no fused kernel exists for these sizes
 // near32: the near-field blocks dF are the FP32 copy (with FP32 coupling blocks)

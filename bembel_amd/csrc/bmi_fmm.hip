@@ -514,45 +514,6 @@ __global__ __launch_bounds__(256) void k_backward_tree(int top, int bot, int to_
   }
 }
 
-// ------------------------------------------------------------------ coupling apply
-// bw[t][k][i] += sum over blocks (t, s): F (cd x cd) * fw[s][k][:]  for all levels at once;
-// targets are (level, cluster) pairs listed in `tgt`, their blocks in CSR `rp`/`src`.
-template <bool C, typename FT>
-__global__ void k_coupling_apply(int ntgt, int nrhs, int cd, int ld, const int2* __restrict__ tgt,
-                                 const int* __restrict__ rp, const int* __restrict__ src,
-                                 const FT* __restrict__ F, int64_t fstride, int64_t fcomp,
-                                 const int64_t* __restrict__ lvl_off, const double* __restrict__ fw,
-                                 double* bw, int accumulate) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= static_cast<int64_t>(ntgt) * nrhs * cd) return;
-  const int i = static_cast<int>(gid % cd);
-  const int64_t tk = gid / cd;
-  const int k = static_cast<int>(tk % nrhs), t = static_cast<int>(tk / nrhs);
-  const int2 T = tgt[t];  // level, cluster
-  const int64_t off = lvl_off[T.x] * nrhs;  // level start in [level][cluster][rhs][row]
-  Val<C> acc;
-  for (int p = rp[t]; p < rp[t + 1]; ++p) {
-    const FT* f = F + (C ? 2 : 1) * (static_cast<int64_t>(p) * fstride + fcomp);
-    const int64_t xb = off + (static_cast<int64_t>(src[p]) * nrhs + k) * cd;
-    for (int j = 0; j < cd; ++j) {
-      Val<C> a;
-      if constexpr (C) {
-        a.r = static_cast<double>(f[2 * (static_cast<int64_t>(j) * ld + i)]);
-        a.i = static_cast<double>(f[2 * (static_cast<int64_t>(j) * ld + i) + 1]);
-      } else {
-        a.r = static_cast<double>(f[static_cast<int64_t>(j) * ld + i]);
-      }
-      acc.fma(a, Val<C>::load(fw, xb + j));
-    }
-  }
-  const int64_t o = off + (static_cast<int64_t>(T.y) * nrhs + k) * cd + i;
-  if (accumulate) {
-    Val<C> prev = Val<C>::load(bw, o);
-    acc.fma_real(1.0, prev);
-  }
-  acc.store(bw, o);
-}
-
 // ------------------------------------------------------------------ Maxwell far field
 // The Maxwell coupling leaf (level, t, s) is K_ts (np2 x np2 kernel values at the Chebyshev nodes
 // of clusters t and s), and its component block (r, c) in the reference is
@@ -662,37 +623,6 @@ __global__ __launch_bounds__(GS* NG) void k_mx_coupling(int nrhs, int np2, int c
   bw1[2 * (o + i)] = r1, bw1[2 * (o + i) + 1] = i1;
   bw0[2 * (o + np2 + i)] = dr, bw0[2 * (o + np2 + i) + 1] = di;
   bw1[2 * (o + np2 + i)] = dr, bw1[2 * (o + np2 + i) + 1] = di;
-}
-
-// ------------------------------------------------------------------ backward transformation
-// leaf rows: ys[seg + c*dd + i, k] = sum_dense F (dd x dd) xs[cseg + c2*dd .., k]
-//                                    + sum_r Mom(r, i) bw_L[c][k][r]
-template <bool C>
-__global__ void k_leaf(int ncl, int nrhs, int dd, const int* __restrict__ rp, const int* __restrict__ src,
-                       const double* __restrict__ F, int64_t fstride, int64_t fcomp,
-                       const double* __restrict__ xs, int64_t ldxs, int64_t xseg,
-                       const double* __restrict__ mom, int rows, const double* __restrict__ bw,
-                       double* ys, int64_t ldys, int64_t yseg, int accumulate) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= static_cast<int64_t>(ncl) * nrhs * dd) return;
-  const int i = static_cast<int>(gid % dd);
-  const int64_t ck = gid / dd;
-  const int c = static_cast<int>(ck % ncl), k = static_cast<int>(ck / ncl);
-  Val<C> acc;
-  const double* xk = xs + (C ? 2 : 1) * (static_cast<int64_t>(k) * ldxs + xseg);
-  for (int p = rp[c]; p < rp[c + 1]; ++p) {
-    const double* f = F + (C ? 2 : 1) * (static_cast<int64_t>(p) * fstride + fcomp);
-    const int64_t xb = static_cast<int64_t>(src[p]) * dd;
-    for (int j = 0; j < dd; ++j) acc.fma(Val<C>::load(f, static_cast<int64_t>(j) * dd + i), Val<C>::load(xk, xb + j));
-  }
-  if (bw) {
-    const int64_t bb = (static_cast<int64_t>(c) * nrhs + k) * rows;
-    for (int r = 0; r < rows; ++r) acc.fma_real(mom[static_cast<int64_t>(i) * rows + r], Val<C>::load(bw, bb + r));
-  }
-  double* yk = ys + (C ? 2 : 1) * (static_cast<int64_t>(k) * ldys + yseg);
-  const int64_t o = static_cast<int64_t>(c) * dd + i;
-  if (accumulate) acc.fma_real(1.0, Val<C>::load(yk, o));
-  acc.store(yk, o);
 }
 
 // ------------------------------------------------------------------ wave-per-cluster sweeps
@@ -1804,10 +1734,7 @@ __global__ __launch_bounds__(256) void k_sweep_fused_sym(LeafArgs la, CplArgs ca
 }
 
 // ------------------------------------------------------------------ many right-hand sides
-// Block rows for many right-hand sides: one wave per row owner (leaf cluster or coupling target)
-// and 64 columns, lane k owns column k and keeps all ROWS rows of its column in registers.  The
-// blocks are wave-uniform and read through the scalar cache, each once per 64 columns, so the
-// products run at the arithmetic rate instead of re-reading every block per few columns.
+// Block rows of row owners (leaf clusters or coupling targets), 64 columns per workgroup.
 // Addresses: X(s, j, k) = x[S * (xoff + s * xcs + k * xks + j)], Y(r, i, k) likewise with the
 // owner's cluster; coupling owners shift both by their level's start.
 struct MultiArgs {
@@ -1830,92 +1757,6 @@ struct MultiArgs {
   // 3 = one block on source r, block index 0 (leaf moments and leaf rows)
   int mode;
 };
-
-// One wave covers RPW of the ROWS rows (blockIdx.z picks which): fewer accumulators per lane and
-// several waves per owner keep enough waves resident to hide the latency of the scalar block loads.
-template <bool C, typename FT, int ROWS, int RPW>
-__global__ __launch_bounds__(64) void k_multi_rows(MultiArgs a) {
-  constexpr int S = C ? 2 : 1;
-  constexpr bool F32 = std::is_same<FT, float>::value;
-  const int r = blockIdx.x;
-  const int k = static_cast<int>(blockIdx.y) * 64 + static_cast<int>(threadIdx.x);
-  const int i0 = RPW == ROWS ? 0 : static_cast<int>(blockIdx.z) * RPW;
-  const bool valid = k < a.nrhs;
-  const int kk = valid ? k : 0;
-  int cl = r;
-  int64_t xo = a.xoff, yo = a.yoff;
-  if (a.tgt) {
-    const int2 T = a.tgt[r];
-    cl = T.y;
-    const int64_t lo = a.lvl_off[T.x] * a.nrhs;  // level start of [level][cluster][rhs][row]
-    xo += lo;
-    yo += lo;
-  }
-  double ar[RPW], ai[C ? RPW : 1];
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    ar[i] = 0.0;
-    if constexpr (C) ai[i] = 0.0;
-  }
-  const FT* __restrict__ F = static_cast<const FT*>(a.F);
-  const int p0 = a.rp[r], p1 = a.rp[r + 1];
-  for (int p = p0; p < p1; ++p) {
-    const FT* f = F + S * (static_cast<int64_t>(p) * a.fstride + a.fcomp + i0);
-    const double* x = a.x + S * (xo + static_cast<int64_t>(a.src[p]) * a.xcs + static_cast<int64_t>(kk) * a.xks);
-    if constexpr (F32) {
-      // FP32 blocks, FP64 sums
-      for (int j = 0; j < ROWS; ++j) {
-        const double xr = x[S * j * a.xrs];
-        const double xi = C ? x[S * j * a.xrs + 1] : 0.0;
-        const float* fj = reinterpret_cast<const float*>(f) + S * j * a.ldf;
-#pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-          const int ii = RPW == ROWS ? i : (i0 + i < ROWS ? i : ROWS - 1 - i0);
-          const double fr = static_cast<double>(fj[S * ii]);
-          if constexpr (C) {
-            const double fi = static_cast<double>(fj[S * ii + 1]);
-            ar[i] += fr * xr - fi * xi;
-            ai[i] += fr * xi + fi * xr;
-          } else {
-            ar[i] += fr * xr;
-          }
-        }
-      }
-    } else {
-      for (int j = 0; j < ROWS; ++j) {
-        const double xr = x[S * j * a.xrs];
-        const double xi = C ? x[S * j * a.xrs + 1] : 0.0;
-        const double* fj = reinterpret_cast<const double*>(f) + S * j * a.ldf;
-#pragma unroll
-        for (int i = 0; i < RPW; ++i) {
-          const int ii = RPW == ROWS ? i : (i0 + i < ROWS ? i : ROWS - 1 - i0);
-          const double fr = fj[S * ii];
-          if constexpr (C) {
-            const double fi = fj[S * ii + 1];
-            ar[i] += fr * xr - fi * xi;
-            ai[i] += fr * xi + fi * xr;
-          } else {
-            ar[i] += fr * xr;
-          }
-        }
-      }
-    }
-  }
-  if (!valid) return;
-  double* y = a.y + S * (yo + static_cast<int64_t>(cl) * a.ycs + static_cast<int64_t>(k) * a.yks + i0 * a.yrs);
-#pragma unroll
-  for (int i = 0; i < RPW; ++i) {
-    if (RPW != ROWS && i0 + i >= ROWS) continue;
-    double vr = ar[i], vi = C ? ai[i] : 0.0;
-    double* yi_ = y + S * i * a.yrs;
-    if (a.accumulate) {
-      vr += yi_[0];
-      if constexpr (C) vi += yi_[1];
-    }
-    yi_[0] = vr;
-    if constexpr (C) yi_[1] = vi;
-  }
-}
 
 // ------------------------------------------------------------------ block rows staged in LDS (many RHS)
 // One workgroup (4 waves) per owner and 64 right-hand sides: y_owner (ROUT x 64) = sum over the
@@ -2784,32 +2625,18 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   const int64_t n = static_cast<int64_t>(ntgt) * nrhs * cd;
   if (n == 0) return;
   TimedScope ts("coupling_apply", st);
-  if (nrhs >= MULTI_MIN_RHS && (!Fc || ncoarse == 0)) {
-    const MultiArgs ma{ntgt, nrhs, tgt, lvl_off, rp, src, F, fstride, fcomp, ld, fw, 0,
-                       static_cast<int64_t>(nrhs) * cd, cd, 1, bw, 0, static_cast<int64_t>(nrhs) * cd, cd, 1, accumulate};
-#define BMI_CPL_M(CC, FTT, CDD)                                                                       \
-  if (cplx == CC && fp32 == std::is_same<FTT, float>::value && cd == CDD) {                           \
-    constexpr int RPW = CDD;                                                                          \
-    const dim3 grid(static_cast<unsigned>(ntgt), static_cast<unsigned>((nrhs + 63) / 64),             \
-                    static_cast<unsigned>((CDD + RPW - 1) / RPW));                                    \
-    hipLaunchKernelGGL((k_multi_rows<CC, FTT, CDD, RPW>), grid, dim3(64), 0, st, ma);                 \
-    BMI_CHECK_HIP(hipGetLastError());                                                                 \
-    return;                                                                                           \
-  }
-    BMI_CPL_M(false, double, 16)
-    BMI_CPL_M(false, float, 16)
-    BMI_CPL_M(true, double, 16)
-    BMI_CPL_M(true, float, 16)
-    BMI_CPL_M(false, double, 25)
-    BMI_CPL_M(false, float, 25)
-    BMI_CPL_M(true, double, 25)
-    BMI_CPL_M(true, float, 25)
-    BMI_CPL_M(true, double, 32)
-    BMI_CPL_M(true, float, 32)
-#undef BMI_CPL_M
-  }
+  // several columns, and single columns of block sizes without a wave-per-target kernel (the BF16
+  // blocks of the coarsest levels are read by the wave kernels only)
+  auto rows = [&] {
+    launch_block_rows(cplx, fp32,
+                      RowsArgs{ntgt, nrhs, cd, ld, 1, tgt, lvl_off, rp, src, F, fstride, fw, 0,
+                               static_cast<int64_t>(nrhs) * cd, cd, 1, bw, 0, static_cast<int64_t>(nrhs) * cd, cd, 1,
+                               accumulate, 1, 1},
+                      st);
+  };
+  if (nrhs > 1 && (!Fc || ncoarse == 0)) return rows();
   const dim3 wgrid(static_cast<unsigned>((ntgt + 3) / 4));
-  // wave-per-target kernels for the block sizes of the configurations (np 4, 5; Maxwell np 4)
+  // wave-per-target kernels for the block sizes of the configurations (np 4, 5)
 #define BMI_CPL_W(CC, FTT, CDD)                                                                              \
   if (cplx == CC && fp32 == std::is_same<FTT, float>::value && cd == CDD) {                                  \
     const CplArgs ca{ntgt, nrhs, tgt, rp, src, F, fstride, fcomp, lvl_off, fw, bw, accumulate, Fc, ncoarse, ld}; \
@@ -2833,19 +2660,7 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   BMI_CPL_W(true, double, 32)
   BMI_CPL_W(true, float, 32)
 #undef BMI_CPL_W
-  if (cplx && !fp32)
-    hipLaunchKernelGGL((k_coupling_apply<true, double>), dim3(nblk(n)), dim3(256), 0, st, ntgt, nrhs, cd, ld, tgt, rp,
-                       src, static_cast<const double*>(F), fstride, fcomp, lvl_off, fw, bw, accumulate);
-  else if (!cplx && !fp32)
-    hipLaunchKernelGGL((k_coupling_apply<false, double>), dim3(nblk(n)), dim3(256), 0, st, ntgt, nrhs, cd, ld, tgt,
-                       rp, src, static_cast<const double*>(F), fstride, fcomp, lvl_off, fw, bw, accumulate);
-  else if (cplx)
-    hipLaunchKernelGGL((k_coupling_apply<true, float>), dim3(nblk(n)), dim3(256), 0, st, ntgt, nrhs, cd, ld, tgt, rp,
-                       src, static_cast<const float*>(F), fstride, fcomp, lvl_off, fw, bw, accumulate);
-  else
-    hipLaunchKernelGGL((k_coupling_apply<false, float>), dim3(nblk(n)), dim3(256), 0, st, ntgt, nrhs, cd, ld, tgt, rp,
-                       src, static_cast<const float*>(F), fstride, fcomp, lvl_off, fw, bw, accumulate);
-  BMI_CHECK_HIP(hipGetLastError());
+  rows();
 }
 
 // deepest subtree (at most three levels below its root) whose level buffers fit in 64 KB of LDS
@@ -2941,55 +2756,37 @@ void launch_backward(bool cplx, int npatch, int L, int rows, int np2, int dd, in
   BMI_CHECK_HIP(hipGetLastError());
 }
 
-void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, const int* rp, const int* src, const double* F,
-                 int64_t fstride, int64_t fcomp, const double* xs, int64_t ldxs, int64_t xseg, double* ys, int64_t ldys,
-                 int64_t yseg, int accumulate, hipStream_t st) {
-  const int64_t n = static_cast<int64_t>(ncl) * nrhs * dd;
+// near-field rows of every component: ys = A_near xs (blocks of the vd x vd component pairs dd x dd
+// entries apart)
+void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, int vd, const int* rp, const int* src,
+                 const double* F, const double* xs, int64_t ldxs, int64_t xseg, double* ys, int64_t ldys,
+                 int64_t yseg, hipStream_t st) {
+  if (ncl <= 0 || nrhs <= 0) return;
   TimedScope ts("matvec_nearfield", st);
-  if (nrhs >= MULTI_MIN_RHS) {
-    const MultiArgs ma{ncl, nrhs, nullptr, nullptr, rp, src, F, fstride, fcomp, dd, xs, xseg, dd, ldxs, 1, ys, yseg, dd,
-                       ldys, 1, accumulate};
-#define BMI_LEAF_M(CC, DDD)                                                                           \
-  if (cplx == CC && dd == DDD) {                                                                      \
-    constexpr int RPW = DDD;                                                                          \
-    const dim3 grid(static_cast<unsigned>(ncl), static_cast<unsigned>((nrhs + 63) / 64),              \
-                    static_cast<unsigned>((DDD + RPW - 1) / RPW));                                    \
-    hipLaunchKernelGGL((k_multi_rows<CC, double, DDD, RPW>), grid, dim3(64), 0, st, ma);              \
-    BMI_CHECK_HIP(hipGetLastError());                                                                 \
-    return;                                                                                           \
-  }
-    BMI_LEAF_M(false, 16)
-    BMI_LEAF_M(true, 16)
-    BMI_LEAF_M(false, 36)
-    BMI_LEAF_M(true, 36)
-#undef BMI_LEAF_M
-  }
-  const dim3 wgrid(static_cast<unsigned>((ncl + 3) / 4));
-  // wave-per-cluster kernels for the leaf sizes 4 (P+1)^2 of P = 1, 2
+  const int64_t dblk = static_cast<int64_t>(dd) * dd;
+  if (nrhs == 1 && vd == 1) {
+    // wave-per-cluster kernels for the leaf sizes 4 (P+1)^2 of P = 1, 2
+    const dim3 wgrid(static_cast<unsigned>((ncl + 3) / 4));
 #define BMI_LEAF_W(CC, DDD)                                                                                     \
   if (cplx == CC && dd == DDD) {                                                                                \
-    const LeafArgs la{ncl, nrhs, rp, src, F, fstride, fcomp, xs, ldxs, xseg, ys, ldys, yseg, accumulate};       \
-    if (nrhs == 1 && variant == 1)                                                                              \
+    const LeafArgs la{ncl, nrhs, rp, src, F, dblk, 0, xs, ldxs, 0, ys, ldys, 0, 0};  /* one component */        \
+    if (variant == 1)                                                                                           \
       hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1, 2>), wgrid, dim3(256), 0, st, la);                               \
-    else if (nrhs == 1)                                                                                         \
-      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1, 1>), wgrid, dim3(256), 0, st, la);                               \
     else                                                                                                        \
-      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 4, 1>), wgrid, dim3(256), 0, st, la);                               \
+      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1, 1>), wgrid, dim3(256), 0, st, la);                               \
     BMI_CHECK_HIP(hipGetLastError());                                                                           \
     return;                                                                                                     \
   }
-  BMI_LEAF_W(false, 16)
-  BMI_LEAF_W(true, 16)
-  BMI_LEAF_W(false, 36)
-  BMI_LEAF_W(true, 36)
+    BMI_LEAF_W(false, 16)
+    BMI_LEAF_W(true, 16)
+    BMI_LEAF_W(false, 36)
+    BMI_LEAF_W(true, 36)
 #undef BMI_LEAF_W
-  if (cplx)
-    hipLaunchKernelGGL(k_leaf<true>, dim3(nblk(n)), dim3(256), 0, st, ncl, nrhs, dd, rp, src, F, fstride, fcomp,
-                       xs, ldxs, xseg, nullptr, 0, nullptr, ys, ldys, yseg, accumulate);
-  else
-    hipLaunchKernelGGL(k_leaf<false>, dim3(nblk(n)), dim3(256), 0, st, ncl, nrhs, dd, rp, src, F, fstride, fcomp,
-                       xs, ldxs, xseg, nullptr, 0, nullptr, ys, ldys, yseg, accumulate);
-  BMI_CHECK_HIP(hipGetLastError());
+  }
+  launch_block_rows(cplx, false,
+                    RowsArgs{ncl, nrhs, dd, dd, vd, nullptr, nullptr, rp, src, F, dblk, xs, xseg, dd, ldxs, 1, ys,
+                             yseg, dd, ldys, 1, 0, 1, 1},
+                    st);
 }
 
 static bool launch_sweep_fused_sym(bool cplx, bool fp32, int leaf_variant, int cpl_variant, int ncl, int dd,

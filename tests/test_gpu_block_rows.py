@@ -1,0 +1,70 @@
+"""Block-row sweeps (bmi_rows.hip) at the edges of their tiles: products with several columns, and
+single columns of block sizes without a kernel of their own, against the oracle.
+
+Block sizes: coupling blocks of n_cheb^2 rows (1, 4, 9, ..., 81: one row, below, at and past whole
+16-row tiles and 4-column steps), near-field leaves of 4^min_cluster_level (P + 1)^2 rows.  Columns:
+one, and below, at and past the 8 (complex) and 16 (real) columns of a tile and the column groups.
+The products sum the same terms as the oracle in another order: 1e-12 relative, as the other
+parity tests.
+"""
+import numpy as np
+import pytest
+
+import bembel_amd as B
+import oracle_lib as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(op_name, M, P, n_cheb, mcl=1, precision=B.FP64):
+    op = B.LaplaceSingleLayerOperator() if op_name == "laplace" else B.HelmholtzSingleLayerOperator()
+    kappa = 0j if op_name == "laplace" else 2.5 - 0.3j
+    op.set_wavenumber(kappa)
+    ps = B.AnsatzSpace(B.Geometry(), M, P, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb, min_cluster_level=mcl, precision=precision)
+    kind = O.LAPLACE if op_name == "laplace" else O.HELMHOLTZ
+    oh = O.H2(O.Space(O.Geometry(), M, P), kind, kappa, n_cheb, mcl=mcl)
+    return H, oh, ps.number_of_dofs, op.scalar
+
+
+def _columns(n, cols, scalar, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.uniform(-1, 1, (n, cols))
+    return x if scalar == np.float64 else x + 1j * rng.uniform(-1, 1, (n, cols))
+
+
+def _check(H, oh, n, scalar, cols, tol=1e-12):
+    X = _columns(n, max(cols), scalar, 5)
+    ref = oh.matvec(X)
+    for c in cols:
+        Y = H @ X[:, :c]
+        e = np.linalg.norm(Y - ref[:, :c]) / np.linalg.norm(ref[:, :c])
+        assert e <= tol, (c, e)
+
+
+@pytest.mark.parametrize("op", ["laplace", "helmholtz"])
+@pytest.mark.parametrize("P,n_cheb", [(1, 1), (2, 2), (1, 3), (1, 4), (2, 5), (2, 6), (1, 7), (2, 9), (1, 11)])
+def test_gpu_block_rows_sizes(gpu, op, P, n_cheb):
+    H, oh, n, scalar = _pair(op, 3, P, n_cheb)
+    _check(H, oh, n, scalar, (1, 2, 5))
+
+
+@pytest.mark.parametrize("op", ["laplace", "helmholtz"])
+@pytest.mark.parametrize("P,mcl", [(1, 0), (2, 0), (1, 2), (2, 2)])
+def test_gpu_block_rows_leaf_sizes(gpu, op, P, mcl):
+    H, oh, n, scalar = _pair(op, 3, P, 4, mcl)
+    _check(H, oh, n, scalar, (1, 3))
+
+
+@pytest.mark.parametrize("op", ["laplace", "helmholtz"])
+@pytest.mark.parametrize("n_cheb", [4, 9])
+def test_gpu_block_rows_columns(gpu, op, n_cheb):
+    H, oh, n, scalar = _pair(op, 2, 2, n_cheb)
+    _check(H, oh, n, scalar, (1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 130))
+
+
+@pytest.mark.parametrize("op", ["laplace", "helmholtz"])
+def test_gpu_block_rows_fp32_blocks(gpu, op):
+    # FP32 copies of the coupling blocks, columns padded to whole vectors: 1e-8 from the FP64 operator
+    H, oh, n, scalar = _pair(op, 3, 1, 9, precision=B.MIXED)
+    _check(H, oh, n, scalar, (1, 3, 20), tol=1e-6)
