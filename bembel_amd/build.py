@@ -31,6 +31,7 @@ SOURCES = {
     "bmi_space_dev.cpp": ["-x", "hip"],
     "bmi_potential.hip": [],
     "bmi_rows.hip": [],
+    "bmi_tree.hip": [],
 }
 
 

@@ -173,6 +173,7 @@ struct bmi_h2 {
   int64_t lvl_total = 0;
   // FMM constants
   DevBuf<double> d_T, d_mom[2];
+  DevBuf<double> d_E, d_m1;  // the same matrices of one direction (TreeArgs)
   DevBuf<double> d_Tt, d_momt[2];  // transposed copies for the RHS-fastest backward steps
   // upper half of the coupling blocks (symmetric kernels) for single-RHS sweeps
   bool sym = false;
@@ -233,7 +234,7 @@ struct bmi_h2 {
   size_t bytes() const {
     return d_dense.bytes() + d_coup.bytes() + d_coup32.bytes() + d_coup16.bytes() + d_dense32.bytes() +
            d_fly_pts.bytes() + d_fly_org.bytes() + d_drp.bytes() + d_dsrc.bytes() + d_tgt.bytes() + d_tgt_all.bytes() + d_crp_all.bytes() +
-           d_crp.bytes() + d_csrc.bytes() + d_T.bytes() + d_mom[0].bytes() + d_mom[1].bytes() + d_Tt.bytes() + d_momt[0].bytes() + d_momt[1].bytes() + d_stgt.bytes() + d_sgtgt.bytes() + d_srp.bytes() +
+           d_crp.bytes() + d_csrc.bytes() + d_T.bytes() + d_E.bytes() + d_m1.bytes() + d_mom[0].bytes() + d_mom[1].bytes() + d_Tt.bytes() + d_momt[0].bytes() + d_momt[1].bytes() + d_stgt.bytes() + d_sgtgt.bytes() + d_srp.bytes() +
            d_ssrc.bytes() + d_sblk.bytes() + d_sgrp.bytes() + d_sgslot.bytes() + d_part.bytes() + d_xs.bytes() +
            d_ys.bytes() + d_fw[0].bytes() + d_fw[1].bytes() + d_bw.bytes() + d_yf.bytes() + d_mx_tan.bytes() +
            d_mxz.bytes() + d_mx_order.bytes() + d_ntgt.bytes() + d_ngtgt.bytes() + d_nrp.bytes() + d_nsrc.bytes() +
@@ -301,42 +302,52 @@ static Work handle_work(bmi_h2* h) {
               h->d_mxz.ptr};
 }
 
+// tree transformations of a column-major product: moments of xs up the tree into v0, v1 (upward), or
+// local expansions v0, v1 down to the leaf rows y
+// (xin: one column in the DOF space; xs_out = T xin is formed on the way and used in place of xs)
+static void apply_tree(const bmi_h2* h, bool upward, int nrhs, const double* xs, double* v0, double* v1, double* y,
+                       hipStream_t st, double* clear = nullptr, const double* xin = nullptr,
+                       double* xs_out = nullptr) {
+  const bmi_space* s = h->s;
+  TimedScope ts(upward ? "matvec_forward" : "matvec_backward", st);
+  TreeArgs ta{h->cplx, s->npatch, h->L, h->np, h->nc, h->vd, (1 << h->mcl) * (s->P + 1), h->mcl, s->P + 1, nrhs,
+                       h->d_E.ptr, h->d_m1.ptr, h->d_lvl_off.ptr, v0, v1, clear, xs, y, s->nsuper,
+                       static_cast<int64_t>(s->nel) * s->I2};
+  if (xin) ta.trp = s->d_rowptr.ptr, ta.tcol = s->d_col.ptr, ta.tval = s->d_val.ptr, ta.xin = xin, ta.xs = xs_out;
+  launch_tree(ta, upward, st);
+}
+
+// xs = T X (column-major)
+static void apply_t(const bmi_h2* h, int nrhs, const double* X, int64_t ldx, double* xs, hipStream_t st) {
+  const bmi_space* s = h->s;
+  launch_spmv(h->cplx, s->nsuper, nrhs, s->d_rowptr.ptr, s->d_col.ptr, s->d_val.ptr, X, ldx, xs, s->nsuper, nullptr,
+              nullptr, st);
+}
+
 // far-field chain: forward transformation, coupling, backward transformation, leaf rows -> yf
 static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, double* yf, bool reduced,
                       hipStream_t st) {
   const bmi_space* s = h->s;
   const bool C = h->cplx;
-  const int64_t N = s->nsuper;
   const int rows = h->cd;
-  const int64_t vcs = static_cast<int64_t>(s->nel) * s->I2;  // super DOFs per component
   const CouplingOperand co = coupling_operand(h, reduced);
-  for (int cc = 0; cc < h->vd; ++cc) {
-    TimedScope ts("matvec_forward", st);
-    launch_forward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[cc].ptr, h->d_T.ptr, xs, N, cc * vcs,
-                   w.fw[cc], h->d_lvl_off.ptr, st);
-  }
+  apply_tree(h, true, nrhs, xs, w.fw[0], w.fw[1], nullptr, st);
   if (h->mxf) {
     // four columns per cluster entry from both components' moments, one sweep over the kernel
     // values writing both components' local expansions (into the moment buffers, consumed), then
-    // the backward transformation per component
+    // the backward transformation of both components
     launch_mx_prep(h->lvl_total / rows, nrhs, h->np2, rows, w.fw[0], w.fw[1], h->d_mx_tan.ptr, w.z, st);
     launch_mx_coupling(co.fp32, h->ntgt_all, nrhs, h->np2, rows, h->d_mx_order.ptr, h->d_tgt_all.ptr,
                        h->d_crp_all.ptr, h->d_csrc.ptr,
                        co.F, h->d_lvl_off.ptr, h->d_mx_tan.ptr, w.z, w.fw[0], w.fw[1], h->mx_qre, h->mx_qim, st);
-    for (int rc = 0; rc < h->vd; ++rc) {
-      TimedScope ts("matvec_backward", st);
-      launch_backward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[rc].ptr, h->d_T.ptr, w.fw[rc],
-                      h->d_lvl_off.ptr, yf, N, rc * vcs, st);
-    }
+    apply_tree(h, false, nrhs, nullptr, w.fw[0], w.fw[1], yf, st);
     return;
   }
   // every cluster of every level is a target (zero where there are no blocks)
   launch_coupling_apply(C, co.fp32, std::max(h->cpl_variant, 0), h->ntgt_all, nrhs, rows, h->d_tgt_all.ptr,
                         h->d_crp_all.ptr, h->d_csrc.ptr, co.F, co.blk, 0, h->d_lvl_off.ptr, w.fw[0], w.bw, 0, st,
                         co.Fc, co.ncoarse, co.ld);
-  TimedScope ts("matvec_backward", st);
-  launch_backward(C, s->npatch, h->L, rows, h->np2, h->dd, nrhs, h->d_mom[0].ptr, h->d_T.ptr, w.bw,
-                  h->d_lvl_off.ptr, yf, N, 0, st);
+  apply_tree(h, false, nrhs, nullptr, w.bw, nullptr, yf, st);
 }
 
 // near-field sweep: ys = A_near xs
@@ -366,10 +377,8 @@ struct SweepScopeName {
 // sweeps write disjoint vectors (ys; bw, then yf), so both forms give the same bits.  false if the
 // sweep kernel is not instantiated for this operator.
 static bool fused_product(bmi_h2* h, const Work& w, const double* xs, double* ys, double* yf, bool reduced,
-                          hipStream_t st, bool overlap) {
-  const bmi_space* s = h->s;
+                          hipStream_t st, bool overlap, const double* xin = nullptr) {
   const CouplingOperand co = coupling_operand(h, reduced);
-  const int64_t N = s->nsuper;
   const bool use_sym = h->sym && h->sym_fused && !co.fp32;
   const SymList* sl = use_sym ? &h->sl : nullptr;
   const SymList* nsl = use_sym && h->sym_fused == 2 ? &h->nsl : nullptr;
@@ -379,11 +388,7 @@ static bool fused_product(bmi_h2* h, const Work& w, const double* xs, double* ys
                               h->d_crp.ptr, h->d_csrc.ptr, co.F, h->d_lvl_off.ptr, w.fw[0], w.bw, ss, co.Fc,
                               co.ncoarse, false, co.ld, csl, nl);
   };
-  {
-    TimedScope ts("matvec_forward", st);
-    launch_forward(h->cplx, s->npatch, h->L, h->cd, h->np2, h->dd, 1, h->d_mom[0].ptr, h->d_T.ptr, xs, N, 0,
-                   w.fw[0], h->d_lvl_off.ptr, st, w.bw);
-  }
+  apply_tree(h, true, 1, xs, w.fw[0], nullptr, nullptr, st, w.bw, xin, w.xs);
   hipStream_t fs = st;
   if (overlap) {
     if (!h->side_stream) BMI_CHECK_HIP(hipStreamCreateWithFlags(&h->side_stream, hipStreamNonBlocking));
@@ -409,11 +414,7 @@ static bool fused_product(bmi_h2* h, const Work& w, const double* xs, double* ys
     }
     ok = okc && okn;
   }
-  if (ok) {
-    TimedScope ts("matvec_backward", fs);
-    launch_backward(h->cplx, s->npatch, h->L, h->cd, h->np2, h->dd, 1, h->d_mom[0].ptr, h->d_T.ptr, w.bw,
-                    h->d_lvl_off.ptr, yf, N, 0, fs);
-  }
+  if (ok) apply_tree(h, false, 1, nullptr, w.bw, nullptr, yf, fs);
   if (overlap) {
     BMI_CHECK_HIP(hipEventRecord(h->ev_join, fs));
     BMI_CHECK_HIP(hipStreamWaitEvent(st, h->ev_join, 0));
@@ -539,19 +540,15 @@ static void autotune(bmi_h2* h, const double* xs, bool reduced, hipStream_t st) 
 }
 
 // super-space apply: ys = A_near xs on `st`, yf = A_far xs on the side stream (joined back into
-// `st` before returning); the caller adds the two
+// `st` before returning); the caller adds the two.  xin (one column, xs = w.xs): xs = T xin is formed
+// first, by the bottom launch of the forward transformation where that precedes every other use
 static void apply_super(bmi_h2* h, const Work& w, int nrhs, const double* xs, double* ys, double* yf,
-                        bool reduced, hipStream_t st) {
+                        bool reduced, hipStream_t st, const double* xin = nullptr) {
   const bool far = has_far(h);
   if (far && reduced && h->red1 && nrhs == 1) {
     // reduced operator, one RHS: FP32 near-field blocks and the coupling evaluated on the fly
-    const bmi_space* s = h->s;
-    const int64_t N = s->nsuper;
-    {
-      TimedScope ts("matvec_forward", st);
-      launch_forward(h->cplx, s->npatch, h->L, h->cd, h->np2, h->dd, 1, h->d_mom[0].ptr, h->d_T.ptr, xs, N, 0,
-                     w.fw[0], h->d_lvl_off.ptr, st, w.bw);
-    }
+    apply_tree(h, true, 1, xs, w.fw[0], nullptr, nullptr, st, w.bw, xin, w.xs);
+    xin = nullptr;
     // the variant the first product timed; before that (an allocation-free product on a handle
     // that has not run bmi_h2_matvec yet) the on-the-fly sweep for real kernels, else the FP32 copy
     const int v = h->fly_variant >= 0 ? h->fly_variant : (h->fly ? 0 : 2);
@@ -565,15 +562,15 @@ static void apply_super(bmi_h2* h, const Work& w, int nrhs, const double* xs, do
                                    h->d_crp.ptr, h->d_csrc.ptr, h->d_coup32.ptr, h->d_lvl_off.ptr, w.fw[0],
                                    w.bw, st, nullptr, 0, true, h->ld32, v >= 6 ? &h->sl : nullptr);
     if (ok) {
-      TimedScope ts("matvec_backward", st);
-      launch_backward(h->cplx, s->npatch, h->L, h->cd, h->np2, h->dd, 1, h->d_mom[0].ptr, h->d_T.ptr, w.bw,
-                      h->d_lvl_off.ptr, yf, N, 0, st);
+      apply_tree(h, false, 1, nullptr, w.bw, nullptr, yf, st);
       return;
     }
   }
-  if (far && nrhs == 1 && h->vd == 1 && h->fused_leaf_variant >= 0 && h->fused_cpl_variant >= 0 &&
-      fused_product(h, w, xs, ys, yf, reduced, st, w.own && h->overlap == 1))
-    return;
+  if (far && nrhs == 1 && h->vd == 1 && h->fused_leaf_variant >= 0 && h->fused_cpl_variant >= 0) {
+    if (fused_product(h, w, xs, ys, yf, reduced, st, w.own && h->overlap == 1, xin)) return;
+    xin = nullptr;
+  }
+  if (xin) apply_t(h, 1, xin, h->s->ndof, w.xs, st);
   if (far && !w.own) {
     // one stream: the two chains write disjoint vectors, so the order gives the same bits
     apply_far(h, w, nrhs, xs, yf, reduced, st);
@@ -659,13 +656,14 @@ static void apply_super_t(bmi_h2* h, const Work& w, int nrhs, bool reduced, hipS
 // timing needs host synchronisation per kernel and therefore runs eagerly.  A single-RHS product
 // (four launches, the longest a few hundred microseconds) also runs eagerly: measured, the next
 // kernel on the stream starts about 8 us after a graph ends, more than the launches save.
-static void apply_super_workspace(bmi_h2* h, int nrhs, bool reduced, bool tl, hipStream_t st) {
+// xin: one column in the DOF space whose T xin is not in the workspace yet.
+static void apply_super_workspace(bmi_h2* h, int nrhs, bool reduced, bool tl, hipStream_t st, const double* xin) {
   const Work w = handle_work(h);
   auto run = [&](hipStream_t rs) {
     if (tl)
       apply_super_t(h, w, nrhs, reduced, rs);
     else
-      apply_super(h, w, nrhs, w.xs, w.ys, w.yf, reduced, rs);
+      apply_super(h, w, nrhs, w.xs, w.ys, w.yf, reduced, rs, xin);
   };
   if (!tl) autotune(h, h->d_xs.ptr, reduced, st);
   if (!h->use_graphs || timing_enabled() || (nrhs == 1 && !tl)) {
@@ -701,17 +699,19 @@ static void apply_dof(bmi_h2* h, const Work& w, int nrhs, const double* X, int64
   const bmi_space* s = h->s;
   const int64_t N = s->nsuper;
   const bool tl = use_rhs_fastest(h, nrhs, reduced);
+  // one column: T x is formed inside the product (the choice between its forms, made by the first
+  // product, times them on a super vector that exists)
+  const double* xin = !tl && nrhs == 1 && (!w.own || h->leaf_variant >= 0) ? X : nullptr;
   if (tl)
     launch_spmv_tin(h->cplx, s->nsuper, nrhs, s->d_rowptr.ptr, s->d_col.ptr, s->d_val.ptr, X, ldx, w.xs, st);
-  else
-    launch_spmv(h->cplx, s->nsuper, nrhs, s->d_rowptr.ptr, s->d_col.ptr, s->d_val.ptr, X, ldx, w.xs, N, nullptr,
-                nullptr, st);
+  else if (!xin)
+    apply_t(h, nrhs, X, ldx, w.xs, st);
   if (w.own)
-    apply_super_workspace(h, nrhs, reduced, tl, st);
+    apply_super_workspace(h, nrhs, reduced, tl, st, xin);
   else if (tl)
     apply_super_t(h, w, nrhs, reduced, st);
   else
-    apply_super(h, w, nrhs, w.xs, w.ys, w.yf, reduced, st);
+    apply_super(h, w, nrhs, w.xs, w.ys, w.yf, reduced, st, xin);
   if (tl)
     launch_spmv_tout(h->cplx, s->ndof, nrhs, s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, w.ys,
                      has_far(h) ? w.yf : nullptr, Y, ldy, alpha, beta, st);
@@ -1039,6 +1039,17 @@ static void assemble_h2(bmi_h2* h, hipStream_t st) {
   std::vector<double> T, mom;
   transfer_matrix(h->np, T);
   h->d_T.upload(T, st);
+  {
+    std::vector<double> E, m1, dm;
+    transfer_1d(h->np, E);
+    h->d_E.upload(E, st);
+    moment1d(s->P, h->L, h->mcl, h->np, false, m1);
+    if (vd == 2) {
+      moment1d(s->P, h->L, h->mcl, h->np, true, dm);
+      m1.insert(m1.end(), dm.begin(), dm.end());
+    }
+    h->d_m1.upload(m1, st);
+  }
   {
     // T_q(i, j) = T[(q np2 + j) np2 + i]; Tt holds T_q^T in the same layout
     const int n2 = h->np2;

@@ -84,14 +84,29 @@ void launch_mx_coupling(bool fp32, int ntgt_all, int nrhs, int np2, int cd, cons
                         const int* rp_all, const int* src, const void* K, const int64_t* lvl_off, const double* tan, const double* Z,
                         double* bw0, double* bw1, double qre, double qim, hipStream_t st);
 void convert_to_bf16(const double* src, unsigned short* dst, int64_t n, hipStream_t st);
-// forward transformation of all levels (moments at level L, transfers up to level 0)
-void launch_forward(bool cplx, int npatch, int L, int rows, int np2, int dd, int nrhs, const double* mom,
-                    const double* T, const double* xs, int64_t ldxs, int64_t xseg, double* fw, const int64_t* lvl_off,
-                    hipStream_t st, double* bw_zero = nullptr);
-// backward transformation of all levels, ending in the leaf rows yf = Mom^T bw_L (written)
-void launch_backward(bool cplx, int npatch, int L, int rows, int np2, int dd, int nrhs, const double* mom,
-                     const double* T, double* bw, const int64_t* lvl_off, double* yf, int64_t ldy, int64_t yseg,
-                     hipStream_t st);
+// tree transformations of column-major products (bmi_tree.hip).  upward: moments of x at level L and
+// transfers up to level 0 into the multipole arrays v0, v1 (vd components of nc np^2 rows; clear: the
+// array of local expansions set to zero, or null); downward: local expansions v0, v1 down the tree
+// (read only) and the leaf rows y.
+struct TreeArgs {
+  bool cplx;
+  int npatch, L, np, nc, vd, c1, mcl, pp1, nrhs;
+  const double* E;  // np x 2 np: E[i * 2 np + h * np + j], polynomial j at node i of half h
+  const double* m;  // np x c1 moments of one direction, then (vd 2) their derivative counterparts
+  const int64_t* lvl_off;
+  double *v0, *v1, *clear;
+  const double* x;
+  double* y;
+  int64_t ldx, xseg;  // column and component strides of x or y
+  // upward, one column, one component: x = T xin formed by the bottom launch and written to xs (T in
+  // CSR; trp null: x is given)
+  const int* trp = nullptr;
+  const int* tcol = nullptr;
+  const double* tval = nullptr;
+  const double* xin = nullptr;
+  double* xs = nullptr;
+};
+void launch_tree(const TreeArgs& a, bool upward, hipStream_t st);
 void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, int vd, const int* rp, const int* src,
                  const double* F, const double* xs, int64_t ldxs, int64_t xseg, double* ys, int64_t ldys,
                  int64_t yseg, hipStream_t st);
@@ -134,7 +149,4 @@ bool launch_sweep_fly(bool cplx, int variant, int ncl, int dd, const int* drp, c
                       const double* xs, double* ys, int ntgt, int cd, const int2* tgt, const int* crp,
                       const int* csrc, const int64_t* lvl_off, const float4* pts, const double4* org,
                       double kre, double kim, const double* fw, double* bw, hipStream_t st);
-void launch_leaf_backward(bool cplx, int ncl, int nrhs, int dd, const double* mom, int rows, const double* bw,
-                          double* yf, int64_t ldy, int64_t yseg, hipStream_t st);
-
 }  // namespace bmi

@@ -271,249 +271,6 @@ __global__ void k_spmv_sub(int nrows, int nrhs, const int* __restrict__ rp, cons
   }
 }
 
-// ------------------------------------------------------------------ fused tree transformations
-// One workgroup owns one cluster at level `top` and walks its subtree down to level `bot`
-// (bot - top <= 3) in LDS; blockIdx.y is the right-hand side.  Each transformation is one launch
-// (instead of one per level, each a few microseconds of latency for very little work).
-// Level buffers in LDS: level top + d holds 4^d clusters x rows values.
-__device__ __forceinline__ int tree_lds_off(int d, int rows, int S) {
-  return S * rows * (((1 << (2 * d)) - 1) / 3);  // sum_{e<d} 4^e clusters before level top + d
-}
-
-// one subtree of the forward transformation (H2Multipole.hpp:380-422): level bot of cluster
-// ctop's subtree from the moments of the super vector (from_moment) or from fw, then parents by
-// the transfer matrices up to level top; every level is written to fw (and bw cleared there)
-template <bool C>
-__device__ __forceinline__ void forward_subtree(double* lds, int top, int bot, bool from_moment, int ctop, int k,
-                                                int rows, int np2, int dd, int nrhs, const double* mom,
-                                                const double* T, const double* __restrict__ xs, int64_t ldxs,
-                                                int64_t xseg, double* fw, const int64_t* __restrict__ lvl_off,
-                                                double* __restrict__ bwz) {
-  constexpr int S = C ? 2 : 1;
-  const int tid = threadIdx.x;
-  const int D = bot - top;
-  {
-    const int n = (1 << (2 * D)) * rows;
-    double* L = lds + tree_lds_off(D, rows, S);
-    const int64_t base = lvl_off[bot] * nrhs;
-    for (int idx = tid; idx < n; idx += blockDim.x) {
-      const int cl = idx / rows, row = idx - (idx / rows) * rows;
-      const int64_t c = (static_cast<int64_t>(ctop) << (2 * D)) + cl;
-      const int64_t g = S * (base + (c * nrhs + k) * rows + row);
-      if (from_moment) {
-        const double* x = xs + S * (static_cast<int64_t>(k) * ldxs + xseg + c * dd);
-        double ar = 0.0, ai = 0.0;
-#pragma unroll
-        for (int j = 0; j < dd; ++j) {
-          const double m = mom[static_cast<int64_t>(j) * rows + row];
-          ar += m * x[S * j];
-          if constexpr (C) ai += m * x[S * j + 1];
-        }
-        L[S * idx] = ar;
-        fw[g] = ar;
-        if constexpr (C) L[S * idx + 1] = ai, fw[g + 1] = ai;
-        if (bwz) {
-          bwz[g] = 0.0;
-          if constexpr (C) bwz[g + 1] = 0.0;
-        }
-      } else {
-        L[S * idx] = fw[g];
-        if constexpr (C) L[S * idx + 1] = fw[g + 1];
-      }
-    }
-  }
-  __syncthreads();
-  for (int d = D - 1; d >= 0; --d) {
-    const int n = (1 << (2 * d)) * rows;
-    const double* Ch = lds + tree_lds_off(d + 1, rows, S);
-    double* Pa = lds + tree_lds_off(d, rows, S);
-    const int64_t base = lvl_off[top + d] * nrhs;
-    for (int idx = tid; idx < n; idx += blockDim.x) {
-      const int cl = idx / rows, row = idx - (idx / rows) * rows;
-      const int comp = row / np2, i = row - comp * np2;
-      double ar = 0.0, ai = 0.0;
-#pragma unroll 1
-      for (int q = 0; q < 4; ++q) {
-        const double* ch = Ch + S * ((4 * cl + q) * rows + comp * np2);
-#pragma unroll
-        for (int j = 0; j < np2; ++j) {
-          const double t = T[static_cast<int64_t>(q * np2 + j) * np2 + i];
-          ar += t * ch[S * j];
-          if constexpr (C) ai += t * ch[S * j + 1];
-        }
-      }
-      Pa[S * idx] = ar;
-      const int64_t c = (static_cast<int64_t>(ctop) << (2 * d)) + cl;
-      const int64_t g = S * (base + (c * nrhs + k) * rows + row);
-      fw[g] = ar;
-      if constexpr (C) Pa[S * idx + 1] = ai, fw[g + 1] = ai;
-      if (bwz) {
-        bwz[g] = 0.0;
-        if constexpr (C) bwz[g + 1] = 0.0;
-      }
-    }
-    __syncthreads();
-  }
-}
-
-// forward transformation (H2Multipole.hpp:380-422), one segment of levels per launch: workgroup
-// (ctop, rhs) computes the subtree of levels bot (from the moments of the super vector, or from
-// fw) .. top below cluster ctop.  The segments are separate launches: handing a finished level to
-// another workgroup inside one launch needs device-scope fences, which write back and invalidate
-// the L2 of every XCD and measured slower than the launch they save.
-// NPC / DDC != 0 fix np2 (= rows, one FMM component) and dd at compile time: the dot products
-// then unroll and their loads are issued together instead of one latency per term.
-template <bool C, int NPC = 0, int DDC = 0>
-__global__ __launch_bounds__(256) void k_forward_tree(int top, int bot, int from_moment, int rows_, int np2_, int dd_,
-                                                      int nrhs, const double* __restrict__ mom,
-                                                      const double* __restrict__ T, const double* __restrict__ xs,
-                                                      int64_t ldxs, int64_t xseg, double* __restrict__ fw,
-                                                      const int64_t* __restrict__ lvl_off, double* __restrict__ bwz,
-                                                      int lvl_doubles, int stage) {
-  extern __shared__ double lds[];
-  const int rows = NPC ? NPC : rows_, np2 = NPC ? NPC : np2_, dd = DDC ? DDC : dd_;
-  const int k = blockIdx.y, tid = threadIdx.x;
-  // the transfer matrix (and the moment matrix for the bottom level) are read many times per
-  // workgroup: stage them in LDS after the level buffers when they fit (stage != 0)
-  if (stage) {
-    double* Ts = lds + lvl_doubles;
-    for (int q = tid; q < 4 * np2 * np2; q += blockDim.x) Ts[q] = T[q];
-    T = Ts;
-    if (from_moment) {
-      double* Ms = Ts + 4 * np2 * np2;
-      for (int q = tid; q < dd * rows; q += blockDim.x) Ms[q] = mom[q];
-      mom = Ms;
-      __syncthreads();  // the moments use Ms; otherwise the barrier after the bottom level covers T
-    }
-  }
-  forward_subtree<C>(lds, top, bot, from_moment != 0, blockIdx.x, k, rows, np2, dd, nrhs, mom, T, xs, ldxs, xseg,
-                     fw, lvl_off, bwz);
-}
-
-// backward transformation (H2Multipole.hpp:428-469) in one launch: workgroup (ctop, rhs) owns
-// cluster ctop at level top.  It first forms the local expansion of its ancestors from level 0
-// down to ctop (one cluster per level: coupling sum in bw plus T^T of the parent; every
-// workgroup repeats this short chain instead of waiting for a launch above it); then children get
-// their coupling sums plus T^T of their parent, down to level bot; level bot is written back,
-// or, with to_leaf, turned into the leaf rows yf = Mom^T bw_bot.
-template <bool C, int NPC = 0, int DDC = 0, bool ST = false>
-__global__ __launch_bounds__(256) void k_backward_tree(int top, int bot, int to_leaf, int rows_, int np2_, int dd_,
-                                                       int nrhs, const double* __restrict__ mom,
-                                                       const double* __restrict__ T, double* __restrict__ bw,
-                                                       const int64_t* __restrict__ lvl_off, double* __restrict__ yf,
-                                                       int64_t ldy, int64_t yseg, int lvl_doubles) {
-  extern __shared__ double lds[];
-  constexpr int S = C ? 2 : 1;
-  const int rows = NPC ? NPC : rows_, np2 = NPC ? NPC : np2_, dd = DDC ? DDC : dd_;  // as in k_forward_tree
-  const int ctop = blockIdx.x, k = blockIdx.y, tid = threadIdx.x;
-  const int D = bot - top;
-  double* A = lds + lvl_doubles;  // ancestors' expansions: (top + 1) x rows, after the staged matrices
-  // ST: T and Mom staged in LDS transposed, so that lanes (consecutive child rows, leaf entries)
-  // read consecutive words; in the global layout their reads are np2 or rows words apart, which
-  // puts a wave's lanes on a few LDS banks
-  if constexpr (ST) {
-    double* Ts = lds + lvl_doubles;
-    const int nt = np2 * np2;
-    for (int e = tid; e < 4 * nt; e += blockDim.x) {
-      const int q = e / nt, r = e - q * nt, i = r / np2, j = r - i * np2;
-      Ts[e] = T[static_cast<int64_t>(q * np2 + j) * np2 + i];
-    }
-    T = Ts;
-    A = Ts + 4 * nt;
-    if (to_leaf) {
-      double* Ms = A;
-      for (int e = tid; e < dd * rows; e += blockDim.x) {
-        const int q = e / dd, i = e - q * dd;
-        Ms[e] = mom[static_cast<int64_t>(i) * rows + q];
-      }
-      mom = Ms;
-      A = Ms + dd * rows;
-    }
-  }
-  // entry (j, i) of transfer block q (child row j, parent row i) and moment entry (i, q)
-  auto tval = [&](int q, int j, int i) {
-    return ST ? T[(q * np2 + i) * np2 + j] : T[static_cast<int64_t>(q * np2 + j) * np2 + i];
-  };
-  auto mval = [&](int i, int q) { return ST ? mom[q * dd + i] : mom[static_cast<int64_t>(i) * rows + q]; };
-  for (int idx = tid; idx < (top + 1) * rows; idx += blockDim.x) {
-    const int l = idx / rows, row = idx - l * rows;
-    const int64_t a = static_cast<int64_t>(ctop) >> (2 * (top - l));
-    const int64_t g = S * (lvl_off[l] * nrhs + (a * nrhs + k) * rows + row);
-    A[S * idx] = bw[g];
-    if constexpr (C) A[S * idx + 1] = bw[g + 1];
-  }
-  __syncthreads();
-  for (int l = 1; l <= top; ++l) {
-    const int q = (ctop >> (2 * (top - l))) & 3;
-    for (int row = tid; row < rows; row += blockDim.x) {
-      const int comp = row / np2, j = row - comp * np2;
-      const double* pa = A + S * ((l - 1) * rows + comp * np2);
-      double ar = A[S * (l * rows + row)], ai = C ? A[S * (l * rows + row) + 1] : 0.0;
-#pragma unroll
-      for (int i = 0; i < np2; ++i) {
-        const double t = tval(q, j, i);
-        ar += t * pa[S * i];
-        if constexpr (C) ai += t * pa[S * i + 1];
-      }
-      A[S * (l * rows + row)] = ar;
-      if constexpr (C) A[S * (l * rows + row) + 1] = ai;
-    }
-    __syncthreads();
-  }
-  for (int idx = tid; idx < rows; idx += blockDim.x) {
-    lds[S * idx] = A[S * (top * rows + idx)];
-    if constexpr (C) lds[S * idx + 1] = A[S * (top * rows + idx) + 1];
-  }
-  __syncthreads();
-  for (int d = 1; d <= D; ++d) {
-    const int n = (1 << (2 * d)) * rows;
-    const double* Pa = lds + tree_lds_off(d - 1, rows, S);
-    double* Ch = lds + tree_lds_off(d, rows, S);
-    const int64_t base = lvl_off[top + d] * nrhs;
-    for (int idx = tid; idx < n; idx += blockDim.x) {
-      const int ch = idx / rows, row = idx - (idx / rows) * rows;
-      const int comp = row / np2, j = row - comp * np2;
-      const int pc = ch >> 2, q = ch & 3;
-      const int64_t c = (static_cast<int64_t>(ctop) << (2 * d)) + ch;
-      const int64_t g = S * (base + (c * nrhs + k) * rows + row);
-      double ar = bw[g], ai = C ? bw[g + 1] : 0.0;
-      const double* pa = Pa + S * (pc * rows + comp * np2);
-#pragma unroll
-      for (int i = 0; i < np2; ++i) {
-        const double t = tval(q, j, i);
-        ar += t * pa[S * i];
-        if constexpr (C) ai += t * pa[S * i + 1];
-      }
-      Ch[S * idx] = ar;
-      if constexpr (C) Ch[S * idx + 1] = ai;
-      if (d == D && !to_leaf) {
-        bw[g] = ar;
-        if constexpr (C) bw[g + 1] = ai;
-      }
-    }
-    __syncthreads();
-  }
-  if (to_leaf) {
-    const double* Lv = lds + tree_lds_off(D, rows, S);
-    const int n = (1 << (2 * D)) * dd;
-    for (int idx = tid; idx < n; idx += blockDim.x) {
-      const int cl = idx / dd, i = idx - (idx / dd) * dd;
-      const double* b = Lv + S * cl * rows;
-      double ar = 0.0, ai = 0.0;
-#pragma unroll
-      for (int q = 0; q < rows; ++q) {
-        const double m = mval(i, q);
-        ar += m * b[S * q];
-        if constexpr (C) ai += m * b[S * q + 1];
-      }
-      const int64_t c = (static_cast<int64_t>(ctop) << (2 * D)) + cl;
-      double* y = yf + S * (static_cast<int64_t>(k) * ldy + yseg + c * dd + i);
-      y[0] = ar;
-      if constexpr (C) y[1] = ai;
-    }
-  }
-}
-
 // ------------------------------------------------------------------ Maxwell far field
 // The Maxwell coupling leaf (level, t, s) is K_ts (np2 x np2 kernel values at the Chebyshev nodes
 // of clusters t and s), and its component block (r, c) in the reference is
@@ -758,28 +515,6 @@ __global__ __launch_bounds__(256) void k_leaf_w(LeafArgs a) {
   const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6));
   if (c >= a.ncl) return;
   leaf_wave<C, DD, RT, UB>(c, a);
-}
-
-// leaf rows of the backward transformation: yf[seg + c*dd + i, k] = sum_q Mom(q, i) bw_L[c][k][q]
-template <bool C>
-__global__ void k_leaf_backward(int ncl, int nrhs, int dd, const double* __restrict__ mom, int rows,
-                                const double* __restrict__ bw, double* __restrict__ yf, int64_t ldy, int64_t yseg) {
-  constexpr int S = C ? 2 : 1;
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= static_cast<int64_t>(ncl) * nrhs * dd) return;
-  const int i = static_cast<int>(gid % dd);
-  const int64_t ck = gid / dd;
-  const int c = static_cast<int>(ck % ncl), k = static_cast<int>(ck / ncl);
-  const double* b = bw + S * ((static_cast<int64_t>(c) * nrhs + k) * rows);
-  const double* m = mom + static_cast<int64_t>(i) * rows;
-  double ar = 0.0, ai = 0.0;
-  for (int q = 0; q < rows; ++q) {
-    ar += m[q] * b[S * q];
-    if constexpr (C) ai += m[q] * b[S * q + 1];
-  }
-  double* y = yf + S * (static_cast<int64_t>(k) * ldy + yseg + static_cast<int64_t>(c) * dd + i);
-  y[0] = ar;
-  if constexpr (C) y[1] = ai;
 }
 
 // coupling: bw[t][k][i] (+)= sum over blocks (t, s) of F (CD x CD) fw[s][k][:], all levels in one
@@ -2663,99 +2398,6 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   rows();
 }
 
-// deepest subtree (at most three levels below its root) whose level buffers fit in 64 KB of LDS
-static int tree_max_depth(int doubles_per_cluster) {
-  int d = 3;
-  while (d > 0 && sizeof(double) * doubles_per_cluster * (((1 << (2 * (d + 1))) - 1) / 3) > 64 * 1024) --d;
-  return d;
-}
-
-// whole forward transformation: leaf moments at level L, then every level up to 0, in subtree
-// launches of at most three levels
-void launch_forward(bool cplx, int npatch, int L, int rows, int np2, int dd, int nrhs, const double* mom,
-                    const double* T, const double* xs, int64_t ldxs, int64_t xseg, double* fw, const int64_t* lvl_off,
-                    hipStream_t st, double* bw_zero) {
-  const int S = cplx ? 2 : 1;
-  // the bottom segment spans up to two levels (many workgroups for the moments), the others up
-  // to three, as far as the level buffers fit in 64 KB of LDS
-  const int maxd = tree_max_depth(rows * S);
-  BMI_REQUIRE(maxd >= 1, BMI_UNSUPPORTED, "cluster rows too large for the tree kernels");
-  int bot = L;
-  bool first = true;
-  while (true) {
-    const int depth = first ? std::min(2, maxd) : maxd;
-    const int top = bot - depth > 0 ? bot - depth : 0;
-    const int D = bot - top;
-    const size_t lvl_doubles = static_cast<size_t>(S) * rows * (((1 << (2 * (D + 1))) - 1) / 3);
-    size_t lds = sizeof(double) * lvl_doubles;
-    BMI_REQUIRE(lds <= 64 * 1024, BMI_UNSUPPORTED, "cluster rows too large for the tree kernels");
-    // staging pays off when a workgroup's tree is the whole work (one RHS); with many RHS the
-    // matrices stay in the caches across the workgroups of the same subtree
-    const size_t staged = lds + sizeof(double) * (4 * np2 * np2 + (first ? dd * rows : 0));
-    const int stage = (nrhs == 1 && staged <= 64 * 1024) ? 1 : 0;
-    if (stage) lds = staged;
-    const dim3 grid(static_cast<unsigned>(npatch << (2 * top)), static_cast<unsigned>(nrhs));
-    const int fm = first ? 1 : 0, ld = static_cast<int>(lvl_doubles);
-    bool launched = false;
-#define BMI_FWD(CC, NPC, DDC)                                                                                     \
-  if (!launched && cplx == CC && (NPC == 0 || (rows == NPC && np2 == NPC && dd == DDC))) {                          \
-    hipLaunchKernelGGL((k_forward_tree<CC, NPC, DDC>), grid, dim3(256), lds, st, top, bot, fm, rows, np2, dd, nrhs,  \
-                       mom, T, xs, ldxs, xseg, fw, lvl_off, bw_zero, ld, stage);                                   \
-    launched = true;                                                                                               \
-  }
-    BMI_FWD(false, 16, 36) BMI_FWD(false, 16, 16) BMI_FWD(true, 25, 36) BMI_FWD(true, 25, 16)
-    BMI_FWD(true, 16, 36) BMI_FWD(false, 25, 36) BMI_FWD(false, 0, 0) BMI_FWD(true, 0, 0)
-#undef BMI_FWD
-    BMI_CHECK_HIP(hipGetLastError());
-    first = false;
-    if (top == 0) break;
-    bot = top;
-  }
-}
-
-// whole backward transformation from level 0 to the leaf rows yf: one launch over the clusters at
-// the top of the deepest segment (at most two levels above L), each workgroup recomputing its
-// ancestors' expansions from level 0
-void launch_backward(bool cplx, int npatch, int L, int rows, int np2, int dd, int nrhs, const double* mom,
-                     const double* T, double* bw, const int64_t* lvl_off, double* yf, int64_t ldy, int64_t yseg,
-                     hipStream_t st) {
-  const int S = cplx ? 2 : 1;
-  const int maxd = tree_max_depth(rows * S);
-  BMI_REQUIRE(maxd >= 1, BMI_UNSUPPORTED, "cluster rows too large for the tree kernels");
-  // subtree depth: two levels, fewer when the level buffers and the ancestors' expansions (one
-  // per level above) do not fit in 64 KB of LDS
-  const int bot = L;
-  int top = 0;
-  size_t lvl_doubles = 0, lds = 0;
-  for (int depth = std::min(2, maxd); depth >= 0; --depth) {
-    top = L - depth > 0 ? L - depth : 0;
-    lvl_doubles = static_cast<size_t>(S) * rows * (((1 << (2 * (bot - top + 1))) - 1) / 3);
-    lds = sizeof(double) * (lvl_doubles + static_cast<size_t>(S) * rows * (top + 1));
-    if (lds <= 64 * 1024) break;
-  }
-  BMI_REQUIRE(lds <= 64 * 1024, BMI_UNSUPPORTED, "cluster rows too large for the tree kernels");
-  const size_t staged = lds + sizeof(double) * (4 * np2 * np2 + dd * rows);
-  const int stage = (nrhs == 1 && staged <= 64 * 1024) ? 1 : 0;
-  if (stage) lds = staged;
-  const dim3 grid(static_cast<unsigned>(npatch << (2 * top)), static_cast<unsigned>(nrhs));
-  const int ld = static_cast<int>(lvl_doubles);
-  bool launched = false;
-#define BMI_BWD(CC, NPC, DDC)                                                                                       \
-  if (!launched && cplx == CC && (NPC == 0 || (rows == NPC && np2 == NPC && dd == DDC))) {                            \
-    if (stage)                                                                                                       \
-      hipLaunchKernelGGL((k_backward_tree<CC, NPC, DDC, true>), grid, dim3(256), lds, st, top, bot, 1, rows, np2, dd,  \
-                         nrhs, mom, T, bw, lvl_off, yf, ldy, yseg, ld);                                             \
-    else                                                                                                             \
-      hipLaunchKernelGGL((k_backward_tree<CC, NPC, DDC, false>), grid, dim3(256), lds, st, top, bot, 1, rows, np2, dd, \
-                         nrhs, mom, T, bw, lvl_off, yf, ldy, yseg, ld);                                             \
-    launched = true;                                                                                                 \
-  }
-  BMI_BWD(false, 16, 36) BMI_BWD(false, 16, 16) BMI_BWD(true, 25, 36) BMI_BWD(true, 25, 16)
-  BMI_BWD(true, 16, 36) BMI_BWD(false, 25, 36) BMI_BWD(false, 0, 0) BMI_BWD(true, 0, 0)
-#undef BMI_BWD
-  BMI_CHECK_HIP(hipGetLastError());
-}
-
 // near-field rows of every component: ys = A_near xs (blocks of the vd x vd component pairs dd x dd
 // entries apart)
 void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, int vd, const int* rp, const int* src,
@@ -3275,19 +2917,6 @@ void convert_blocks_to_fp32(const double* src, float* dst, int64_t nb, int cd, i
 void convert_to_bf16(const double* src, unsigned short* dst, int64_t n, hipStream_t st) {
   if (n <= 0) return;
   hipLaunchKernelGGL(k_to_bf16, dim3(nblk(n)), dim3(256), 0, st, src, dst, n);
-  BMI_CHECK_HIP(hipGetLastError());
-}
-
-void launch_leaf_backward(bool cplx, int ncl, int nrhs, int dd, const double* mom, int rows, const double* bw,
-                          double* yf, int64_t ldy, int64_t yseg, hipStream_t st) {
-  const int64_t n = static_cast<int64_t>(ncl) * nrhs * dd;
-  if (n == 0) return;
-  if (cplx)
-    hipLaunchKernelGGL(k_leaf_backward<true>, dim3(nblk(n)), dim3(256), 0, st, ncl, nrhs, dd, mom, rows, bw, yf, ldy,
-                       yseg);
-  else
-    hipLaunchKernelGGL(k_leaf_backward<false>, dim3(nblk(n)), dim3(256), 0, st, ncl, nrhs, dd, mom, rows, bw, yf, ldy,
-                       yseg);
   BMI_CHECK_HIP(hipGetLastError());
 }
 

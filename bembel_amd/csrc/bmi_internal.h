@@ -164,7 +164,10 @@ void build_block_tree(const bmi_space* s, double eta, int mcl, std::vector<Leaf>
 
 // FMM constant matrices (H2Matrix/H2Multipole.hpp), all column-major
 void cheb_points(int n, double* x);
+void transfer_1d(int n, std::vector<double>& E);      // n x 2n, row-major
 void transfer_matrix(int n, std::vector<double>& T);  // n^2 x 4n^2
+// moments of one direction (deriv: of the derivatives), np x 2^cr (P + 1), row-major
+void moment1d(int P, int cl, int cr, int np, bool deriv, std::vector<double>& out);
 void moment_matrix(int P, int cl, int cr, int np, int comp, std::vector<double>& out,
                    int* rows, int* cols);
 

@@ -394,19 +394,25 @@ static double newton_eval(int n, const double* x, const std::vector<double>& L, 
   for (int k = n - 2; k >= 0; --k) r = r * (t - x[k]) + L[k * n + i];
   return r;
 }
-// computeTransferMatrices (H2Multipole.hpp:76-115): column-major n^2 x 4n^2, child blocks in
-// son order (0,0),(1/2,0),(1/2,1/2),(0,1/2)
-void transfer_matrix(int n, std::vector<double>& T) {
-  const int n2 = n * n;
+// one direction of the transfer: polynomial j of the parent interval at node i of its half h,
+// E[i * 2 n + h n + j]
+void transfer_1d(int n, std::vector<double>& E) {
   std::vector<double> x(n);
   cheb_points(n, x.data());
   const auto L = lagrange_newton(n, x.data());
-  std::vector<double> E(n * 2 * n);
+  E.assign(n * 2 * n, 0.0);
   for (int j = 0; j < n; ++j)
     for (int i = 0; i < n; ++i) {
       E[i * 2 * n + j] = newton_eval(n, x.data(), L, j, 0.5 * x[i]);
       E[i * 2 * n + j + n] = newton_eval(n, x.data(), L, j, 0.5 * x[i] + 0.5);
     }
+}
+// computeTransferMatrices (H2Multipole.hpp:76-115): column-major n^2 x 4n^2, child blocks in
+// son order (0,0),(1/2,0),(1/2,1/2),(0,1/2)
+void transfer_matrix(int n, std::vector<double>& T) {
+  const int n2 = n * n;
+  std::vector<double> E;
+  transfer_1d(n, E);
   static const int son_of_quadrant[4] = {0, 3, 1, 2};
   T.assign(static_cast<size_t>(n2) * 4 * n2, 0.0);
   for (int k = 0; k < 4; ++k)
@@ -419,7 +425,7 @@ void transfer_matrix(int n, std::vector<double>& T) {
 }
 
 // Moment1D / Moment1DDerivative (H2Multipole.hpp:120-218), row-major np x 2^cr (P+1)
-static void moment1d(int P, int cl, int cr, int np, bool deriv, std::vector<double>& out);
+void moment1d(int P, int cl, int cr, int np, bool deriv, std::vector<double>& out);
 
 }  // namespace bmi
 
@@ -447,7 +453,7 @@ void linear_form_points(const bmi_space* s, double* out) {
   }
 }
 
-static void moment1d(int P, int cl, int cr, int np, bool deriv, std::vector<double>& out) {
+void moment1d(int P, int cl, int cr, int np, bool deriv, std::vector<double>& out) {
   const int n = 1 << cr, N = 1 << cl, pp1 = P + 1;
   const double h = 1. / n, H = 1. / N;
   const int nq = static_cast<int>(std::ceil(0.5 * (np + P - 2))) + 1;
