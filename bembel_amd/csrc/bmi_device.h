@@ -101,4 +101,49 @@ __device__ __forceinline__ void surface_point(const double* __restrict__ cp, dou
   }
 }
 
+// sine and cosine beyond the reach of the reduction below, kept out of line: inlined, its registers (a
+// reduction by a long expansion of 2 / pi) would be those of every kernel
+static __device__ __noinline__ double2 sincos_far(double x) {
+  double s, c;
+  sincos(x, &s, &c);
+  return make_double2(s, c);
+}
+
+// sine and cosine of the phases kappa r: reduction to [-pi/4, pi/4] by subtracting n pi/2 in two parts
+// (Cody and Waite, with fused multiply-adds) and the Taylor sums of both, whose first neglected terms
+// are below 1e-18 there.  Absolute error within 3e-16 for |x| < 2^20 (checked against extended
+// precision), a third of the library function's instructions.
+__device__ __forceinline__ void sincos_phase(double x, double* s, double* c) {
+  if (!(fabs(x) < 1048576.0)) {
+    const double2 v = sincos_far(x);
+    *s = v.x, *c = v.y;
+    return;
+  }
+  const double n = rint(x * 0.63661977236758134308);  // 2 / pi
+  double y = fma(-n, 1.57079632679489655800, x);      // pi / 2 rounded, and the rest
+  y = fma(-n, 6.12323399573676603587e-17, y);
+  const double z = y * y;
+  double p = 1.0 / 355687428096000.0;  // 1 / 17!
+  p = fma(p, z, -1.0 / 1307674368000.0);
+  p = fma(p, z, 1.0 / 6227020800.0);
+  p = fma(p, z, -1.0 / 39916800.0);
+  p = fma(p, z, 1.0 / 362880.0);
+  p = fma(p, z, -1.0 / 5040.0);
+  p = fma(p, z, 1.0 / 120.0);
+  p = fma(p, z, -1.0 / 6.0);
+  const double sn = fma(y * z, p, y);
+  double q = 1.0 / 20922789888000.0;  // 1 / 16!
+  q = fma(q, z, -1.0 / 87178291200.0);
+  q = fma(q, z, 1.0 / 479001600.0);
+  q = fma(q, z, -1.0 / 3628800.0);
+  q = fma(q, z, 1.0 / 40320.0);
+  q = fma(q, z, -1.0 / 720.0);
+  q = fma(q, z, 1.0 / 24.0);
+  const double cs = fma(z * z, q, fma(-0.5, z, 1.0));
+  const int k = static_cast<int>(n) & 3;  // quadrant
+  const double a = (k & 1) ? cs : sn, b = (k & 1) ? sn : cs;
+  *s = (k & 2) ? -a : a;
+  *c = (k == 1 || k == 2) ? -b : b;
+}
+
 }  // namespace bmi

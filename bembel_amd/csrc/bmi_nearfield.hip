@@ -7,15 +7,19 @@
 // Maxwell/SingleLayerOperator.hpp:44-88) and the test operator
 // (LinearOperator/Dummy/DummyOperator.hpp:53-59).
 //
-// Design: all lanes of a workgroup work on the same element pair, so the patch control
-// points are wave-uniform and are read through the scalar cache.  Each lane evaluates a
-// strided share of the quadrature index space (i, j), computes its surface points in
-// registers and accumulates the (P+1)^2 x (P+1)^2 block in registers; the block is reduced
-// across the workgroup at the end.  The work is FP64-VALU bound (rational Bezier surface
-// points dominate), which is why FP64 MFMA (same peak as FP64 VALU on this chip, 9x9 blocks
-// padded to 16x16) is not used for the block accumulation.  Maxwell blocks have four
-// (P+1)^2 x (P+1)^2 complex component blocks; one workgroup computes one component block
-// (blockIdx.y = 2*row component + column component) so the accumulators stay in registers.
+// Design: all lanes of a workgroup work on the same element pair, so the elements' polynomials
+// (k_element_poly) are wave-uniform and are read through the scalar cache.  The scalar operators run
+// factorised rules: a lane fixes an outer point, sums kernel x basis over inner points, and the outer
+// products of the sums go to the block -- on the matrix cores where a block per lane would cost the
+// second wave per SIMD (identical and edge rules), in registers else.  Maxwell blocks (four
+// (P+1)^2 x (P+1)^2 complex component blocks; blockIdx.y = 2*row component + column component) are
+// accumulated per evaluation.  Bound: FP64 VALU.
+//
+// Measured, 24,576 elements of the sphere, P 2, 13 points per direction for touching pairs, against
+// points in Bernstein form, blocks in registers and the library's sine and cosine: Laplace identical 58.0
+// -> 22.7 ms, edge 97.0 -> 40.7, vertex 18.6 -> 17.6, regular 16.6 -> 15.9; Helmholtz identical 82.5 ->
+// 30.8, edge 149.5 -> 69.8, vertex 54.7 -> 47.7, regular 35.7 -> 31.7 (VALU busy: identical 0.76, edge
+// 0.71, vertex 0.65, regular 0.60).
 #include <hip/hip_runtime.h>
 
 #include "bmi_internal.h"
@@ -24,11 +28,10 @@
 namespace bmi {
 
 struct NFParams {
-  const double* cp;  // control points of all patches
-  int cp_stride;     // doubles per patch
-  const int* elem_patch;
-  const double* elem_llc;
+  const double* poly;  // element polynomials, 4 PD^2 doubles per element (k_element_poly)
+  int poly_stride;
   double h;        // element width in the parameter domain
+  double rh, rh2;  // 1 / h, 1 / h^2 (powers of two)
   double kre, kim;  // wavenumber
   int dummy_fn;
   const double* ffield;  // far-field table, FF_STRIDE doubles per point
@@ -81,11 +84,83 @@ struct Pt<BMI_MAXWELL_SL> {
   double t[6];  // d/ds x, d/dt x
 };
 
+// Surface points.  A patch is a rational polynomial of degree PD - 1 in either parameter; on one element
+// its four homogeneous coordinates are kept in powers of the centred local coordinates u - 1/2,
+// v - 1/2 (G[(a * PD + b) * 4 + k], k_element_poly): values and derivatives take half the operations
+// of the Bernstein form (no basis to evaluate), and |u - 1/2| <= 1/2 keeps the sums as well
+// conditioned.  With x = p / w the tangents are (p_u - x w_u) / w, (p_v - x w_v) / w; derivatives
+// in the patch parameters are 1 / h times those in u, v.
+// element polynomials, written by an earlier kernel only: in the constant address space, so that
+// wave-uniform loads go through the scalar cache wherever they stand (as plain global memory the
+// compiler gave that up in the longer rules)
+typedef const __attribute__((address_space(4))) double* PolyPtr;
+
+// Sums over wave-uniform coefficients (scalar registers) take powers of the coordinate: of the operands
+// of a multiply-add one may be scalar, and a Horner chain starts with two (moves into vector registers
+// were half the instructions of a contraction).
+template <int PD>
+struct Powers {
+  double f[PD], d[PD];  // t^a, a t^(a - 1)
+  __device__ explicit Powers(double t) {
+    f[0] = 1.0, d[0] = 0.0;
+#pragma unroll
+    for (int a = 1; a < PD; ++a) f[a] = f[a - 1] * t, d[a] = a * f[a - 1];
+  }
+  // r = sum g(a) t^a, rd its derivative
+  template <class Coef>
+  __device__ void sum(Coef g, double& r, double& rd) const {
+    r = g(PD - 1) * f[PD - 1], rd = g(PD - 1) * d[PD - 1];
+#pragma unroll
+    for (int a = PD - 2; a >= 1; --a) r = fma(g(a), f[a], r);
+#pragma unroll
+    for (int a = PD - 2; a >= 2; --a) rd = fma(g(a), d[a], rd);
+    r += g(0);
+    if constexpr (PD > 2) rd += g(1);
+  }
+};
+
+template <int PD>
+__device__ __forceinline__ void poly_point(PolyPtr G, double u, double v, double X[3], double Eu[3],
+                                           double Ev[3], double& bot) {
+  // G is uniform: the coefficients are loaded at every point (kept across a loop they would fill the
+  // vector registers)
+  asm volatile("" : "+s"(G));
+  v -= 0.5;
+  Powers<PD> q(u - 0.5);
+  double p[4] = {0, 0, 0, 0}, pu[4] = {0, 0, 0, 0}, pv[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int b = PD - 1; b >= 0; --b) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double r, ru;
+      q.sum([&](int a) { return G[(a * PD + b) * 4 + k]; }, r, ru);
+      pv[k] = fma(pv[k], v, p[k]);
+      p[k] = fma(p[k], v, r);
+      pu[k] = fma(pu[k], v, ru);
+    }
+  }
+  bot = rcp_newton(p[3]);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    X[k] = p[k] * bot;
+    Eu[k] = fma(-X[k], pu[3], pu[k]);
+    Ev[k] = fma(-X[k], pv[3], pv[k]);
+  }
+}
+
+// |a x b|^2
+__device__ __forceinline__ double cross_square(const double a[3], const double b[3]) {
+  const double c0 = a[1] * b[2] - a[2] * b[1];
+  const double c1 = a[2] * b[0] - a[0] * b[2];
+  const double c2 = a[0] * b[1] - a[1] * b[0];
+  return c0 * c0 + c1 * c1 + c2 * c2;
+}
+
 template <int PD, int KIND>
-__device__ __forceinline__ Pt<KIND> make_point(const double* __restrict__ cp, double lx, double ly,
-                                               double h, double u, double v, double w) {
-  double X[3], Ds[3], Dt[3];
-  surface_point<PD>(cp, lx + h * u, ly + h * v, X, Ds, Dt);
+__device__ __forceinline__ Pt<KIND> make_point(PolyPtr G, const NFParams& prm, double u, double v,
+                                               double w) {
+  double X[3], Eu[3], Ev[3], bot;
+  poly_point<PD>(G, u, v, X, Eu, Ev, bot);
   Pt<KIND> p;
   p.x0 = X[0], p.x1 = X[1], p.x2 = X[2];
   p.s0 = u, p.s1 = v;
@@ -93,22 +168,20 @@ __device__ __forceinline__ Pt<KIND> make_point(const double* __restrict__ cp, do
     // the vector basis carries no surface measure: the Piola factor cancels
     // (Maxwell/SingleLayerOperator.hpp:71-85)
     p.W = w;
+    const double f = bot * prm.rh;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) p.t[k] = Ds[k], p.t[3 + k] = Dt[k];
+    for (int k = 0; k < 3; ++k) p.t[k] = Eu[k] * f, p.t[3 + k] = Ev[k] * f;
   } else if (KIND == BMI_DUMMY) {
     p.W = w;
   } else {
-    const double c0 = Ds[1] * Dt[2] - Ds[2] * Dt[1];
-    const double c1 = Ds[2] * Dt[0] - Ds[0] * Dt[2];
-    const double c2 = Ds[0] * Dt[1] - Ds[1] * Dt[0];
-    p.W = sqrt(c0 * c0 + c1 * c1 + c2 * c2) * w;
+    p.W = sqrt(cross_square(Eu, Ev)) * (bot * bot) * (prm.rh2 * w);
   }
   return p;
 }
 
 // test functions of the reference Duffy unit tests (tests/DuffyTrick/test_testFunctions.hpp)
-template <class PT>
-__device__ __forceinline__ double dummy_value(int fn, const PT& a, const PT& b) {
+template <class PA, class PB>
+__device__ __forceinline__ double dummy_value(int fn, const PA& a, const PB& b) {
   if (fn == 0)
     return sin(M_PI * a.x0) * sin(2 * M_PI * b.x0) * exp(-a.x1) * exp(b.x1);
   if (fn == 1) {
@@ -169,7 +242,7 @@ struct BlockAcc {
     } else if constexpr (CPLX) {
       // exp(-i kappa r) / (4 pi r), kappa = kre + i kim (Helmholtz/SingleLayerOperator.hpp:115-120)
       double sn, cs;
-      sincos(prm.kre * r, &sn, &cs);
+      sincos_phase(prm.kre * r, &sn, &cs);
       const double damp = prm.kim != 0.0 ? exp(prm.kim * r) : 1.0;
       const double mag = damp * (a.W * b.W) * (0.25 * M_1_PI) * ri;
       const double kr = mag * cs, ki = -mag * sn;
@@ -323,70 +396,102 @@ __host__ __device__ constexpr int vertex_chunk(int n, int nt) {
   return pick_chunk(n * n * n, nt, mx > 0 ? mx : 1);
 }
 
-// Edge rule, scalar operators: the computed points of sub-regions g = 1, 2 are tau(t4 or 1 - t4,
-// e1; r) with t4 fixed by (i, j0), so for one outer point they lie on a coordinate line of the
-// patch.  The patch is contracted once per line in the fixed direction (a degree-(PD-1) curve of
-// homogeneous points and cross derivatives, 2 PD x 4 values held in registers) and each point on
-// the line costs a one-dimensional evaluation.
+// Coordinate lines of an element (edge and identical rules, scalar operators): with one coordinate
+// fixed the four homogeneous coordinates and their derivatives across the line are polynomials of
+// degree PD - 1 in the other: L[4 a + k] and L[4 PD + 4 a + k], a the power of the moving coordinate.
 template <int PD>
-__device__ __forceinline__ void line_contract(const double* __restrict__ cp, bool fix_s, double f, double* L) {
-  double B[PD], E[PD];
-  bernstein_basis_der<PD - 1>(f, B, E);
-#pragma unroll
-  for (int a = 0; a < PD; ++a) {
-    double r[4] = {0, 0, 0, 0}, rs[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < PD; ++b) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const double c = fix_s ? cp[4 * (b * PD + a) + k] : cp[4 * (a * PD + b) + k];
-        r[k] += B[b] * c;
-        rs[k] += E[b] * c;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) L[4 * a + k] = r[k], L[4 * PD + 4 * a + k] = rs[k];
-  }
-}
-
-// a point of a contracted line at local coordinates (u, v) with weight w, as make_point
-template <int PD, int KIND>
-__device__ __forceinline__ Pt<KIND> line_point(const double* L, bool fix_s, double lx, double ly, double h, double u,
-                                               double v, double w) {
-  double B[PD], E[PD];
-  bernstein_basis_der<PD - 1>(fix_s ? ly + h * v : lx + h * u, B, E);
-  double p[4] = {0, 0, 0, 0}, d1[4] = {0, 0, 0, 0}, d2[4] = {0, 0, 0, 0};
+__device__ __forceinline__ void line_contract(PolyPtr G, bool fix_u, double f, double* L) {
+  const Powers<PD> q(f - 0.5);
 #pragma unroll
   for (int a = 0; a < PD; ++a)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      p[k] += B[a] * L[4 * a + k];
-      d1[k] += B[a] * L[4 * PD + 4 * a + k];  // across the line (the fixed direction)
-      d2[k] += E[a] * L[4 * a + k];           // along the line
+    for (int k = 0; k < 4; ++k)
+      q.sum([&](int b) { return fix_u ? G[(b * PD + a) * 4 + k] : G[(a * PD + b) * 4 + k]; }, L[4 * a + k],
+            L[4 * PD + 4 * a + k]);
+}
+
+// A point of a contracted line.  The surface measure stays split as sqrt(cc) m, m with the weight: the
+// kernel takes sqrt(cc / |x - y|^2) by one reciprocal square root of the product.
+struct LinePt {
+  double x0, x1, x2, cc, m, s0, s1;
+};
+
+// the smallest cc used: a vanishing measure (a collapsed edge) then gives zero, not 0 / 0
+constexpr double MIN_CC = 1e-200;
+
+template <int PD, int KIND>
+__device__ __forceinline__ LinePt line_point(const double* L, const NFParams& prm, bool fix_u, double u, double v,
+                                             double w) {
+  const double t = (fix_u ? v : u) - 0.5;
+  double p[4], d1[4], d2[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    p[k] = L[4 * (PD - 1) + k], d1[k] = L[4 * PD + 4 * (PD - 1) + k], d2[k] = p[k];
+#pragma unroll
+    for (int a = PD - 2; a >= 0; --a) {
+      if (a < PD - 2) d2[k] = fma(d2[k], t, p[k]);     // along the line
+      p[k] = fma(p[k], t, L[4 * a + k]);
+      d1[k] = fma(d1[k], t, L[4 * PD + 4 * a + k]);  // across the line (the fixed direction)
     }
+  }
   const double bot = rcp_newton(p[3]);
-  const double b2 = bot * bot;
-  double X[3], Ds[3], Dt[3];
+  double X[3], E1[3], E2[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     X[k] = p[k] * bot;
-    const double ds = fix_s ? d1[k] : d2[k], dt = fix_s ? d2[k] : d1[k];
-    const double dsw = fix_s ? d1[3] : d2[3], dtw = fix_s ? d2[3] : d1[3];
-    Ds[k] = (ds * p[3] - p[k] * dsw) * b2;
-    Dt[k] = (dt * p[3] - p[k] * dtw) * b2;
+    E1[k] = fma(-X[k], d1[3], d1[k]);
+    E2[k] = fma(-X[k], d2[3], d2[k]);
   }
-  Pt<KIND> q;
+  LinePt q;
   q.x0 = X[0], q.x1 = X[1], q.x2 = X[2];
   q.s0 = u, q.s1 = v;
   if constexpr (KIND == BMI_DUMMY) {
-    q.W = w;
+    q.cc = 1.0, q.m = w;
   } else {
-    const double c0 = Ds[1] * Dt[2] - Ds[2] * Dt[1];
-    const double c1 = Ds[2] * Dt[0] - Ds[0] * Dt[2];
-    const double c2 = Ds[0] * Dt[1] - Ds[1] * Dt[0];
-    q.W = sqrt(c0 * c0 + c1 * c1 + c2 * c2) * w;
+    q.cc = fmax(cross_square(E1, E2), MIN_CC), q.m = (bot * bot) * (prm.rh2 * w);
   }
   return q;
+}
+
+// N points of one line in LDS at moving coordinates t (weights one, local coordinates unset), each
+// coefficient read once
+template <int PD, int KIND, int N>
+__device__ __forceinline__ void line_points(const double* L, const NFParams& prm, const double* t, LinePt* q) {
+  double p[N][4], d1[N][4], d2[N][4];
+#pragma unroll
+  for (int k = 3; k >= 0; --k) {
+    const double c = L[4 * (PD - 1) + k], d = L[4 * PD + 4 * (PD - 1) + k];
+#pragma unroll
+    for (int m = 0; m < N; ++m) p[m][k] = c, d1[m][k] = d, d2[m][k] = c;
+#pragma unroll
+    for (int a = PD - 2; a >= 0; --a) {
+      const double ca = L[4 * a + k], da = L[4 * PD + 4 * a + k];
+#pragma unroll
+      for (int m = 0; m < N; ++m) {
+        if (a < PD - 2) d2[m][k] = fma(d2[m][k], t[m] - 0.5, p[m][k]);
+        p[m][k] = fma(p[m][k], t[m] - 0.5, ca);
+        d1[m][k] = fma(d1[m][k], t[m] - 0.5, da);
+      }
+    }
+    // keeps the coefficients of at most two coordinates in registers
+    if (k == 2) __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int m = 0; m < N; ++m) {
+    const double bot = rcp_newton(p[m][3]);
+    double X[3], E1[3], E2[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      X[k] = p[m][k] * bot;
+      E1[k] = fma(-X[k], d1[m][3], d1[m][k]);
+      E2[k] = fma(-X[k], d2[m][3], d2[m][k]);
+    }
+    q[m].x0 = X[0], q[m].x1 = X[1], q[m].x2 = X[2];
+    q[m].cc = fmax(cross_square(E1, E2), MIN_CC), q[m].m = (bot * bot) * prm.rh2;
+    // computed here: moved behind the branches of the phases, the points would keep both lines'
+    // coefficients in registers
+    asm volatile("" : "+v"(q[m].x0), "+v"(q[m].x1), "+v"(q[m].x2), "+v"(q[m].cc), "+v"(q[m].m));
+  }
 }
 
 // Factorised vertex rule (scalar operators): a lane fixes one outer point and sums
@@ -418,11 +523,25 @@ __host__ __device__ constexpr FactorShape vertex_shape(int n, int nt, int ptsize
   const int cap = DUFFY_TABLE_BYTES / (2 * n * n * ptsize);
   return factor_shape(n, cap < n ? (cap > 0 ? cap : 1) : n, nt, g, 90);
 }
-// edge rule, factorised: chunks of outer indices i (n outer points (i, j0) each), inner range n
-__host__ __device__ constexpr FactorShape edge_shape(int n, int nt, int ptsize, int g) {
-  const int cap = DUFFY_TABLE_BYTES / (8 * n * ptsize);
-  const int mx = cap < n * n ? cap : n * n;
-  return factor_shape(n, mx > 0 ? mx : 1, nt, g, 48);
+// doubles between lines in LDS (16 bytes beyond a whole number of 64-byte rows: lanes on neighbouring
+// lines read different banks)
+__host__ __device__ constexpr int line_stride(int pd) { return 8 * pd + 2; }
+// edge rule, factorised: chunks of outer indices i (n units (i, j0) each, S lanes per unit sharing the n
+// inner indices).  A lane's work per chunk, in instructions counted from the compiled code: 3,260 per unit
+// (contracted lines, fixed points, vectors, tables) and 630 per inner index
+__host__ __device__ constexpr FactorShape edge_shape(int n, int nt, int ptsize) {
+  const int cap = DUFFY_TABLE_BYTES / (2 * n * ptsize);
+  FactorShape best{1, 1};
+  long best_cost = -1;
+  for (int S = 1; S <= n; ++S) {
+    int c = nt / (S * n);
+    if (c > cap) c = cap;
+    if (c > n * n) c = n * n;
+    if (c < 1) break;
+    const long cost = static_cast<long>((n * n + c - 1) / c) * (3260 + static_cast<long>((n + S - 1) / S) * 630);
+    if (best_cost < 0 || cost < best_cost) best_cost = cost, best = FactorShape{c, S};
+  }
+  return best;
 }
 
 // kernel times both point weights, (kr, ki): the scalar integrands of eval() without the basis
@@ -437,13 +556,62 @@ __device__ __forceinline__ void kernel_ww(const Pt<KIND>& a, const Pt<KIND>& b, 
   } else if constexpr (KIND == BMI_HELMHOLTZ_SL) {
     const double r = s * ri;
     double sn, cs;
-    sincos(prm.kre * r, &sn, &cs);
+    sincos_phase(prm.kre * r, &sn, &cs);
     const double damp = prm.kim != 0.0 ? exp(prm.kim * r) : 1.0;
     const double mag = damp * (a.W * b.W) * (0.25 * M_1_PI) * ri;
     kr = mag * cs, ki = -mag * sn;
   } else {
     kr = dummy_value(prm.dummy_fn, a, b) * a.W * b.W, ki = 0.0;
   }
+}
+
+// the same with the second point (or both) on a contracted line
+template <int KIND>
+__device__ __forceinline__ void kernel_scaled(double d0, double d1, double d2, double cc, double f, const NFParams& prm,
+                                              double& kr, double& ki) {
+  // f sqrt(cc) exp(-i kappa r) / (4 pi r)
+  const double s = d0 * d0 + d1 * d1 + d2 * d2;
+  const double mag = (f * (0.25 * M_1_PI)) * (cc * rsqrt_newton(cc * s));
+  if constexpr (KIND == BMI_LAPLACE_SL) {
+    kr = mag, ki = 0.0;
+  } else {
+    const double r = s * rsqrt_newton(s);
+    double sn, cs;
+    sincos_phase(prm.kre * r, &sn, &cs);
+    const double a = prm.kim != 0.0 ? mag * exp(prm.kim * r) : mag;
+    kr = a * cs, ki = -a * sn;
+  }
+}
+template <int KIND>
+__device__ __forceinline__ void kernel_ww(const Pt<KIND>& a, const LinePt& b, const NFParams& prm, double& kr,
+                                          double& ki) {
+  if constexpr (KIND == BMI_DUMMY)
+    kr = dummy_value(prm.dummy_fn, a, b) * a.W * b.m, ki = 0.0;
+  else
+    kernel_scaled<KIND>(a.x0 - b.x0, a.x1 - b.x1, a.x2 - b.x2, b.cc, a.W * b.m, prm, kr, ki);
+}
+template <int KIND>
+__device__ __forceinline__ void kernel_ww(const LinePt& a, const Pt<KIND>& b, const NFParams& prm, double& kr,
+                                          double& ki) {
+  if constexpr (KIND == BMI_DUMMY)
+    kr = dummy_value(prm.dummy_fn, a, b) * a.m * b.W, ki = 0.0;
+  else
+    kernel_scaled<KIND>(a.x0 - b.x0, a.x1 - b.x1, a.x2 - b.x2, a.cc, a.m * b.W, prm, kr, ki);
+}
+template <int KIND>
+__device__ __forceinline__ void kernel_ww(const LinePt& a, const LinePt& b, const NFParams& prm, double& kr,
+                                          double& ki) {
+  if constexpr (KIND == BMI_DUMMY)
+    kr = dummy_value(prm.dummy_fn, a, b) * a.m * b.m, ki = 0.0;
+  else
+    kernel_scaled<KIND>(a.x0 - b.x0, a.x1 - b.x1, a.x2 - b.x2, a.cc * b.cc, a.m * b.m, prm, kr, ki);
+}
+
+// the value of the lane's neighbour (lane ^ 1)
+__device__ __forceinline__ double neighbour(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0xB1, 0xF, 0xF, true);  // quad permute 1, 0, 3, 2
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0xB1, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
 }
 
 // lane-private sum of (kernel x basis vector) over inner points
@@ -472,23 +640,110 @@ struct VecSum {
         if constexpr (CPLX) i[iy * I + ix] += ki * b;
       }
   }
-  // the vector summed over the G lanes of this lane's group (each holds a share of the inner
-  // range): real parts, or for complex vectors the part of this lane's role (role & 1: 0 real,
-  // 1 imaginary); all lanes must call this together
-  template <int G>
+  // the vector summed over the two lanes of this lane's group (each holds a share of the inner
+  // range): real parts, or for complex vectors the part of this lane's role (0 real, 1 imaginary);
+  // all lanes must call this together
   __device__ __forceinline__ void total(int role, double* w) const {
 #pragma unroll
     for (int k = 0; k < I2; ++k) {
-      double sr = r[k], si = CPLX ? i[k] : 0.0;
-#pragma unroll
-      for (int m = 1; m < G; m <<= 1) {
-        sr += __shfl_xor(sr, m, 64);
-        if constexpr (CPLX) si += __shfl_xor(si, m, 64);
+      if constexpr (CPLX) {
+        // hand the neighbour the part it keeps
+        const double give = (role & 1) ? r[k] : i[k], keep = (role & 1) ? i[k] : r[k];
+        w[k] = keep + neighbour(give);
+      } else {
+        w[k] = r[k] + neighbour(r[k]);
       }
-      w[k] = (CPLX && (role & 1)) ? si : sr;
     }
   }
 };
+
+// D(i, j) of v_mfma_f64_16x16x4f64 on lane j + 16 (i mod 4), element i / 4
+typedef double nf_d4 __attribute__((ext_vector_type(4)));
+
+// Sums of outer products on the matrix cores: every lane pair of a wave contributes row vector x column
+// vector, (P+1)^2 entries each; the pairs put them in the wave's own part of LDS (three arrays of 32
+// vectors: fixed, real, imaginary) and eight 16x16x4 steps add the 32 products to the wave's block.  The
+// block takes 8 registers (16 complex) instead of a share of it per lane (90 and 162 for P = 2), which
+// kept the rules at one wave per SIMD.
+template <int I2>
+__host__ __device__ constexpr int stage_doubles(bool cplx) {
+  return 32 * (cplx ? 3 : 2) * I2;
+}
+// LDS operations of a wave are in order; the fences keep the compiler's order as well
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+template <int I2, bool CPLX, bool COLS>
+__device__ __forceinline__ void add_products(const double* stage, int lane, nf_d4& dr, nf_d4& di) {
+  const int li = lane & 15, lk = lane >> 4, row = li < I2 ? li : I2 - 1;  // entries past the block are not read back
+#pragma unroll
+  for (int st = 0; st < 8; ++st) {
+    const int m = (4 * st + lk) * I2 + row;
+    const double f = stage[m], r = stage[32 * I2 + m];
+    dr = __builtin_amdgcn_mfma_f64_16x16x4f64(COLS ? f : r, COLS ? r : f, dr, 0, 0, 0);
+    if constexpr (CPLX) {
+      const double i = stage[64 * I2 + m];
+      di = __builtin_amdgcn_mfma_f64_16x16x4f64(COLS ? f : i, COLS ? i : f, di, 0, 0, 0);
+    }
+  }
+}
+
+// One sub-region of the edge rule: the fixed point F against the inner points inner(j) for j = sub,
+// sub + S, ... < count, which differ in one local coordinate only (FIX0: s0 is the same for all), so
+// the sum over them needs the P + 1 basis values of the moving coordinate and the other direction's
+// values multiply the sum.  COLS: F supplies the rows (element 1) and the inner points the columns;
+// otherwise the inner points supply the rows.  Adds the outer product of F's basis with the summed
+// vector to the wave's block.  All lanes of the wave must call this together.
+template <int P, int KIND, bool COLS, bool FIX0, class PtF, class Inner>
+__device__ __forceinline__ void line_pass(nf_d4& dr, nf_d4& di, double* stage, const PtF& F, int lane, bool act,
+                                          int sub, int S, int count, const NFParams& prm, double fixed, Inner inner) {
+  constexpr int I = P + 1, I2 = I * I;
+  constexpr bool CPLX = KIND == BMI_HELMHOLTZ_SL;
+  double ur[I], ui[I];
+#pragma unroll
+  for (int k = 0; k < I; ++k) ur[k] = 0.0, ui[k] = 0.0;
+  if (act) {
+#pragma unroll 1
+    for (int j = sub; j < count; j += S) {
+      const auto b = inner(j);
+      double kr, ki, B[I];
+      if constexpr (COLS)
+        kernel_ww<KIND>(F, b, prm, kr, ki);
+      else
+        kernel_ww<KIND>(b, F, prm, kr, ki);
+      bernstein_basis<P>(FIX0 ? b.s1 : b.s0, B);
+#pragma unroll
+      for (int k = 0; k < I; ++k) {
+        ur[k] += kr * B[k];
+        if constexpr (CPLX) ui[k] += ki * B[k];
+      }
+    }
+  }
+  double Bf[I], X[I], Y[I];
+  bernstein_basis<P>(fixed, Bf);
+  bernstein_basis<P>(F.s0, X);
+  bernstein_basis<P>(F.s1, Y);
+  // 32 lanes' vectors at a time (inactive lanes contribute zero)
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    if ((lane >> 5) == half) {
+      const int m = (lane & 31) * I2;
+#pragma unroll
+      for (int k = 0; k < I2; ++k) {
+        const double g = Bf[FIX0 ? k % I : k / I];
+        const int o = FIX0 ? k / I : k % I;
+        stage[m + k] = act ? X[k % I] * Y[k / I] : 0.0;
+        stage[32 * I2 + m + k] = act ? g * ur[o] : 0.0;
+        if constexpr (CPLX) stage[64 * I2 + m + k] = act ? g * ui[o] : 0.0;
+      }
+    }
+    wave_fence();
+    add_products<I2, CPLX, COLS>(stage, lane, dr, di);
+    wave_fence();
+  }
+}
 
 // One factorised sub-region: the fixed point F against the inner points inner(j) for j = sub,
 // sub + S, ... < count.  COLS: F supplies the rows (element 1) and the inner points the columns;
@@ -514,7 +769,7 @@ __device__ __forceinline__ void factor_pass(Acc& acc, const PtK& F, int role, bo
     }
   }
   double w[I2];
-  u.template total<Acc::G>(role, w);
+  u.total(role, w);
   if (!act) return;
   double X[I], Y[I];
   bernstein_basis<P>(F.s0, X);
@@ -592,18 +847,51 @@ __device__ __forceinline__ void reduce_block(Acc& acc, double* lds, int tid, dou
   __syncthreads();
 }
 
+// the waves' blocks in LDS: entry (row, column) of part p (0 real, 1 imaginary) of wave w at
+// lds[(w * parts + p) * I2^2 + row * I2 + column]; the caller has passed a barrier since lds was last used
+template <int I2, bool CPLX>
+__device__ __forceinline__ void spread_blocks(double* lds, int wave, int lane, const nf_d4& dr, const nf_d4& di) {
+  const int li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int row = 4 * v + lk;
+    if (row < I2 && li < I2) {
+      lds[(wave * (CPLX ? 2 : 1)) * I2 * I2 + row * I2 + li] = dr[v];
+      if constexpr (CPLX) lds[(wave * 2 + 1) * I2 * I2 + row * I2 + li] = di[v];
+    }
+  }
+  __syncthreads();
+}
+
+// identical rule: outer coordinates xi0 whose lines are staged together: the chunk with the fewest
+// rounds of 128 units, within LDS for two workgroups per CU
+__host__ __device__ constexpr int identical_chunk(int n, int pd) {
+  const int cap = 52 * 1024 / (4 * n * line_stride(pd) * 8);
+  int best = 1, best_rounds = 1 << 30;
+  for (int c = 1; c <= (cap < n ? cap : n); ++c) {
+    const int rounds = n / c * ((c * n * n + 127) / 128) + (n % c * n * n + 127) / 128;
+    if (rounds < best_rounds) best = c, best_rounds = rounds;
+  }
+  return best;
+}
+
+// waves per SIMD asked of the compiler: two for the scalar rules whose points lie on contracted lines
+// (the latencies of one wave covered by the other; the Helmholtz vertex rule, whose lanes hold half a
+// block each, spills at two waves: 48 -> 55 ms)
+__host__ __device__ constexpr int nf_waves(int kind, int cls) {
+  return (kind == BMI_LAPLACE_SL || kind == BMI_HELMHOLTZ_SL) && (cls == 2 || cls == 3) ? 2 : 1;
+}
+
 template <int P, int KIND, int PD, int CLS, int NT>
-__global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pairs, NFParams prm) {
+__global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFPair* __restrict__ pairs, NFParams prm) {
   extern __shared__ double lds[];
   using Acc = BlockAcc<P, KIND>;
   constexpr int I2 = Acc::I2;
   const NFPair pr = pairs[blockIdx.x];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const double* cp1 = prm.cp + static_cast<int64_t>(prm.elem_patch[pr.e1]) * prm.cp_stride;
-  const double* cp2 = prm.cp + static_cast<int64_t>(prm.elem_patch[pr.e2]) * prm.cp_stride;
-  const double l1x = prm.elem_llc[2 * pr.e1], l1y = prm.elem_llc[2 * pr.e1 + 1];
-  const double l2x = prm.elem_llc[2 * pr.e2], l2y = prm.elem_llc[2 * pr.e2 + 1];
+  const PolyPtr g1 = (PolyPtr)(prm.poly + static_cast<int64_t>(pr.e1) * prm.poly_stride);
+  const PolyPtr g2 = (PolyPtr)(prm.poly + static_cast<int64_t>(pr.e2) * prm.poly_stride);
   const double h = prm.h;
   const int n = pr.deg + 1;
   const int nq = n * n;
@@ -615,7 +903,9 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
   const int cc = KIND == BMI_MAXWELL_SL ? static_cast<int>(blockIdx.y) & 1 : 0;
   Acc acc;
   acc.zero();
-  double aval = 0.0;  // the block entry a thread owns (factorised identical rule)
+  double aval = 0.0;  // the block entry a thread owns (factorised identical and regular rules)
+  constexpr bool IDENT = KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL;  // factorised identical rule
+  nf_d4 dr{0.0, 0.0, 0.0, 0.0}, di{0.0, 0.0, 0.0, 0.0};  // sums over units on the matrix cores
   // every lane runs the same number of iterations (lane groups swap values); lanes past the end
   // evaluate a valid point with zero weight
 
@@ -658,8 +948,8 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
     double* bas = rec + NT * VR;                       // basis products of the round's outer points
     for (int k = tid; k < nq; k += NT) {
       const double u = gx[k / n], v = gx[k % n], w = h * (gw[k / n] * gw[k % n]);
-      q1[k] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
-      q2[k] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q1[k] = make_point<PD, KIND>(g1, prm, u, v, w);
+      q2[k] = make_point<PD, KIND>(g2, prm, u, v, w);
     }
     __syncthreads();
     const int S = NT / nq > 1 ? NT / nq : 1;
@@ -715,8 +1005,8 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
     PtK* q2 = q1 + nq;
     for (int k = tid; k < nq; k += NT) {
       const double u = gx[k / n], v = gx[k % n], w = h * (gw[k / n] * gw[k % n]);
-      q1[k] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
-      q2[k] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q1[k] = make_point<PD, KIND>(g1, prm, u, v, w);
+      q2[k] = make_point<PD, KIND>(g2, prm, u, v, w);
     }
     __syncthreads();
     const int total = nq * nq;
@@ -727,144 +1017,137 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
       acc.add(q1[i], q2[j], prm, rc, cc, valid, lane);
     }
     __syncthreads();
-  } else if constexpr (CLS == 2 && (KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL)) {
+  } else if constexpr (CLS == 2 && IDENT) {
     // integrate2, factorised (symmetric kernels).  The sub-simplex pairs of the unfactorised form
     // below are, with t1 = xj0 (1 - xi0), t3 = t1 + xi0 (outer unit (i, j0)) and t2 = xj1 (1 - xi0 xi1),
     // t4 = t2 + xi0 xi1 (inner index j1): (t1,t2)-(t3,t4), (t1,t4)-(t3,t2), (t2,t1)-(t4,t3),
     // (t2,t3)-(t4,t1).  For one unit the eight points lie on four coordinate lines of the patch
-    // (s = t1, s = t3, t = t1, t = t3), contracted once per round into LDS (one line per thread),
-    // and each point is a one-dimensional evaluation.  The tensor basis splits the block: with
-    // B(x) the Bernstein values, A((ix,iy),(jx,jy)) += B_ix(t1) B_jx(t3) U01(iy,jy) + B_iy(t1)
-    // B_jy(t3) U23(ix,jx), U01 = sum over j1 of K0 B(t2) B(t4)^T + K1 B(t4) B(t2)^T and U23 likewise
-    // with K2, K3 (the fourth pair taken in the other order, which the symmetric kernel allows).
-    // The rule adds every pair in both orders, so the block is A + A^T, formed when it is written.
-    // S = 4 lanes share a unit (a lane pair of an even wave for the s-lines, one of an odd wave for
-    // the t-lines, each pair taking every second j1) and add their sums; the unit's sums, basis
-    // values and outer weight go to LDS, and after each round every thread adds the units'
-    // contributions to the one entry of A it owns (no per-lane block in registers).
+    // (s = t1, s = t3, t = t1, t = t3), which depend on xi0 and j0 only: the lines of a chunk of xi0
+    // values are contracted into LDS (one line per thread) and serve every xi1.  The tensor basis
+    // splits the block: with B(x) the Bernstein values, A((ix,iy),(jx,jy)) += B_ix(t1) B_jx(t3)
+    // U01(iy,jy) + B_iy(t1) B_jy(t3) U23(ix,jx), U01 = sum over j1 of K0 B(t2) B(t4)^T + K1 B(t4) B(t2)^T
+    // and U23 likewise with K2, K3 (the fourth pair taken in the other order, which the symmetric
+    // kernel allows).  The rule adds every pair in both orders, so the block is A + A^T, formed when
+    // it is written.
+    // A lane holds a unit; even waves sum U01 over the s-lines, odd waves U23 over the t-lines.  Two j1 are
+    // evaluated together, so each line coefficient read from LDS serves four points (with two the
+    // LDS reads bound the rule: 55 ms for 24,576 elements).  The sums over the units are outer products
+    // of two (P+1)^2 vectors with the units as the inner index: each wave puts 32 units' vectors at a
+    // time in its own part of LDS and multiplies them on the matrix cores (eight 16x16x4 steps), so a
+    // round of units needs no barrier and no block in registers.  Bound: FP64 VALU.
     constexpr bool CPLX = Acc::CPLX;
     constexpr int I = P + 1;
-    constexpr int S = 4;
-    constexpr int UPR = NT / S;                // units per round
-    constexpr int LS = 8 * PD;                 // doubles of one contracted line
-    constexpr int US = 4 * LS + 2;             // doubles per unit: the 16-byte pad puts the 16 units
-                                               // a wave reads at once on different LDS banks
-    constexpr int UR = 7 + (CPLX ? 4 : 2) * I2;  // record of a unit: sc, B(t1), B(t3), U01, U23
-    constexpr int NE = Acc::TOT;               // entries of A (real parts, then imaginary parts)
-    static_assert(UPR * 4 == NT && NE <= NT, "one line and at most one block entry per thread");
-    static_assert(NT == 256, "four waves: two lane-pair halves of 32 units each");
-    double* ua = lds + UPR * US;
-    const int units = nq * n;
-    // evaluation lanes: even waves sum U01 over the s-lines, odd waves U23 over the t-lines (the
-    // line direction is uniform in a wave and fixed at compile time below); a lane pair holds a
-    // unit and takes every second j1
+    constexpr int LST = line_stride(PD);
+    constexpr int UPR = NT / 2;  // units per round
+    static_assert(NT == 256, "four waves: two of 64 units each per direction");
+    const int C = identical_chunk(n, PD);
     const int wv = tid >> 6, ln = tid & 63;
     const bool tl = (wv & 1) != 0;
-    const int myu = (wv >> 1) * 32 + (ln >> 1), par = ln & 1;
-    // the block entry this thread owns
-    const int epart = tid / (I2 * I2), erem = tid - epart * (I2 * I2);
-    const int erow = erem / I2, ecol = erem - erow * I2;
-    const int eiy = erow / I, eix = erow - eiy * I, ejy = ecol / I, ejx = ecol - ejy * I;
-    for (int u0 = 0; u0 < units; u0 += UPR) {
-      __syncthreads();
-      {
-        const int uu = u0 + (tid >> 2), q = tid & 3;
-        if (uu < units) {
-          const int i = uu / n, j0 = uu - (uu / n) * n;
-          const double xi0 = gx[i / n];
-          const double t1 = gx[j0] * (1 - xi0), tf = (q & 1) ? t1 + xi0 : t1;
-          const bool fs = q < 2;
-          line_contract<PD>(cp1, fs, fs ? l1x + h * tf : l1y + h * tf, lds + (tid >> 2) * US + q * LS);
-        }
+    const int myu = (wv >> 1) * 64 + ln;
+    double* stage = lds + C * 4 * n * LST + wv * stage_doubles<I2>(CPLX);
+    for (int c0 = 0; c0 < n; c0 += C) {
+      const int cn = n - c0 < C ? n - c0 : C;
+      __syncthreads();  // the previous chunk's lines are no longer read
+      for (int l = tid; l < cn * n * 4; l += NT) {
+        // line q of (ci, j0) at (q * cn + ci) * n + j0: lanes on consecutive j0 read neighbouring lines
+        const int q = l / (cn * n), r = l - q * (cn * n), ci = r / n, j0 = r - ci * n;
+        const double xi0 = gx[c0 + ci];
+        const double t1 = gx[j0] * (1 - xi0);
+        double L[8 * PD];
+        line_contract<PD>(g1, q < 2, (q & 1) ? t1 + xi0 : t1, L);
+#pragma unroll
+        for (int k = 0; k < 8 * PD; ++k) lds[l * LST + k] = L[k];
       }
       __syncthreads();
-      const int uu = u0 + myu;
-      const bool act = uu < units;
-      const int uc = act ? uu : 0;
-      const int i = uc / n, j0 = uc - (uc / n) * n;
-      const double xi0 = gx[i / n], xi1 = gx[i % n], wi = gw[i / n] * gw[i % n];
-      const double t1 = gx[j0] * (1 - xi0), t3 = t1 + xi0;
-      double ur[I2], ui[CPLX ? I2 : 1];
-#pragma unroll
-      for (int k = 0; k < I2; ++k) {
-        ur[k] = 0.0;
-        if constexpr (CPLX) ui[k] = 0.0;
-      }
-      auto sums = [&](auto TLC) {
-        constexpr bool TL = decltype(TLC)::value;
-#pragma unroll 1
-        for (int j1 = par; j1 < n; j1 += 2) {
-          const double t2 = gx[j1] * (1 - xi0 * xi1), t4 = t2 + xi0 * xi1;
-          const double wj = gw[j1];
-          // the lines are read again in every iteration, one at a time (an opaque offset keeps
-          // the compiler from holding them in registers across the loop)
-          int off = myu * US + (TL ? 2 * LS : 0);
-          asm volatile("" : "+v"(off));
-          const double* Lq = lds + off;
-          // s-lines: (t1,t2)-(t3,t4) and (t1,t4)-(t3,t2); t-lines: (t2,t1)-(t4,t3) and
-          // (t4,t1)-(t2,t3) (the second pair in the other order); either way the first line
-          // holds the points at (t2, t4) of the first member, the second line those of the second
-          const PtK a0 = line_point<PD, KIND>(Lq, !TL, l1x, l1y, h, TL ? t2 : t1, TL ? t1 : t2, 1.0);
-          const PtK a1 = line_point<PD, KIND>(Lq, !TL, l1x, l1y, h, TL ? t4 : t1, TL ? t1 : t4, TL ? wj : 1.0);
-          __builtin_amdgcn_sched_barrier(0);
-          const PtK b0 = line_point<PD, KIND>(Lq + LS, !TL, l1x, l1y, h, TL ? t4 : t3, TL ? t3 : t4, wj);
-          const PtK b1 = line_point<PD, KIND>(Lq + LS, !TL, l1x, l1y, h, TL ? t2 : t3, TL ? t3 : t2, TL ? 1.0 : wj);
-          double kar, kai, kbr, kbi;
-          kernel_ww<KIND>(a0, b0, prm, kar, kai);
-          kernel_ww<KIND>(a1, b1, prm, kbr, kbi);
-          double B2[I], B4[I];
-          bernstein_basis<P>(t2, B2);
-          bernstein_basis<P>(t4, B4);
-#pragma unroll
-          for (int p = 0; p < I; ++p)
-#pragma unroll
-            for (int q = 0; q < I; ++q) {
-              const double f = B2[p] * B4[q], g = B4[p] * B2[q];
-              ur[p * I + q] += kar * f + kbr * g;
-              if constexpr (CPLX) ui[p * I + q] += kai * f + kbi * g;
-            }
-        }
-      };
-      if (act) {
-        if (tl)
-          sums(std::integral_constant<bool, true>());
-        else
-          sums(std::integral_constant<bool, false>());
-      }
-      // the two lanes of a unit add their sums; the first lane of the s-line pair writes the
-      // unit's record with U01, the first lane of the t-line pair adds U23
-#pragma unroll
-      for (int k = 0; k < I2; ++k) {
-        ur[k] += __shfl_xor(ur[k], 1, 64);
-        if constexpr (CPLX) ui[k] += __shfl_xor(ui[k], 1, 64);
-      }
-      if (par == 0) {
-        double* r = ua + myu * UR;
-        if (!tl) {
-          double B1[I], B3[I];
-          bernstein_basis<P>(t1, B1);
-          bernstein_basis<P>(t3, B3);
-          r[0] = act ? h * h * wi * xi0 * (1 - xi0) * (1 - xi0 * xi1) * gw[j0] : 0.0;
-#pragma unroll
-          for (int k = 0; k < I; ++k) r[1 + k] = B1[k], r[1 + I + k] = B3[k];
-        }
-        const int o = tl ? I2 : 0;
+      const int units = cn * nq;
+      for (int u0 = 0; u0 < units; u0 += UPR) {
+        if (u0 + (wv >> 1) * 64 >= units) continue;  // no unit for this wave
+        const bool act = u0 + myu < units;
+        const int uc = act ? u0 + myu : 0;
+        const int ci = uc / nq, rem = uc - ci * nq, i1 = rem / n, j0 = rem - i1 * n;
+        const double xi0 = gx[c0 + ci], xi1 = gx[i1], x01 = xi0 * xi1;
+        const double t1 = gx[j0] * (1 - xi0), t3 = t1 + xi0;
+        double ur[I2], ui[CPLX ? I2 : 1];
 #pragma unroll
         for (int k = 0; k < I2; ++k) {
-          r[7 + o + k] = ur[k];
-          if constexpr (CPLX) r[7 + 2 * I2 + o + k] = ui[k];
+          ur[k] = 0.0;
+          if constexpr (CPLX) ui[k] = 0.0;
+        }
+        // s-lines: (t1,t2)-(t3,t4) and (t1,t4)-(t3,t2); t-lines: (t2,t1)-(t4,t3) and (t4,t1)-(t2,t3)
+        // (the second pair in the other order); either way the first line holds the points at
+        // (t2, t4) of the first member, the second line those of the second at (t4, t2)
+        const double* L0 = lds + ((tl ? 2 * cn * n : 0) + ci * n + j0) * LST;
+        const int L1 = cn * n * LST;
+#pragma unroll 1
+        for (int j1 = 0; j1 < n; j1 += 2) {
+          const bool two = j1 + 1 < n;  // an odd rule ends with a repeated point of weight zero
+          const double g0 = gx[j1], g1_ = gx[two ? j1 + 1 : j1], w0 = gw[j1], w1 = two ? gw[j1 + 1] : 0.0;
+          const double t[4] = {g0 * (1 - x01), g0 * (1 - x01) + x01, g1_ * (1 - x01), g1_ * (1 - x01) + x01};
+          // the lines are read again in every iteration, one at a time (an opaque offset keeps
+          // the compiler from holding them in registers across the loop)
+          int off = 0;
+          asm volatile("" : "+v"(off));
+          const double* Lq = L0 + off;
+          LinePt a[4], b[4];
+          line_points<PD, KIND, 4>(Lq, prm, t, a);
+          __builtin_amdgcn_sched_barrier(0);
+          line_points<PD, KIND, 4>(Lq + L1, prm, t, b);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            double B2[I], B4[I];
+            bernstein_basis<P>(t[2 * h], B2);
+            bernstein_basis<P>(t[2 * h + 1], B4);
+            const double wj = h ? w1 : w0;
+            // K0 B(t2) B(t4)^T, then K1 B(t4) B(t2)^T (one kernel evaluation's registers at a time)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+              double kr, ki;
+              kernel_ww<KIND>(a[2 * h + m], b[2 * h + 1 - m], prm, kr, ki);
+              kr *= wj, ki *= wj;
+#pragma unroll
+              for (int p = 0; p < I; ++p) {
+                const double f = kr * (m ? B4[p] : B2[p]), fi = CPLX ? ki * (m ? B4[p] : B2[p]) : 0.0;
+#pragma unroll
+                for (int q = 0; q < I; ++q) {
+                  ur[p * I + q] += f * (m ? B2[q] : B4[q]);
+                  if constexpr (CPLX) ui[p * I + q] += fi * (m ? B2[q] : B4[q]);
+                }
+              }
+              if constexpr (CPLX) __builtin_amdgcn_sched_barrier(0);
+            }
+          }
+        }
+        double B1[I], B3[I];
+        bernstein_basis<P>(t1, B1);
+        bernstein_basis<P>(t3, B3);
+        const double sc = act ? h * h * (gw[c0 + ci] * gw[i1]) * xi0 * (1 - xi0) * (1 - x01) * gw[j0] : 0.0;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+          if ((ln >> 5) == half) {
+            const int m = (ln & 31) * I2;
+#pragma unroll
+            for (int k = 0; k < I2; ++k) {
+              stage[m + k] = sc * B1[k / I] * B3[k % I];
+              stage[32 * I2 + m + k] = ur[k];
+              if constexpr (CPLX) stage[64 * I2 + m + k] = ui[k];
+            }
+          }
+          wave_fence();
+          add_products<I2, CPLX, true>(stage, ln, dr, di);
+          wave_fence();
         }
       }
-      __syncthreads();
-      if (tid < NE) {
-        const int o01 = 7 + (epart ? 2 * I2 : 0), o23 = o01 + I2;
-#pragma unroll 4
-        for (int m = 0; m < UPR; ++m) {
-          const double* r = ua + m * UR;
-          aval += r[0] * (r[1 + eix] * r[1 + I + ejx] * r[o01 + eiy * I + ejy] +
-                          r[1 + eiy] * r[1 + I + ejy] * r[o23 + eix * I + ejx]);
-        }
-      }
+    }
+    __syncthreads();
+    spread_blocks<I2, CPLX>(lds, wv, ln, dr, di);
+    if (tid < Acc::TOT) {
+      const int part = tid / (I2 * I2), rem = tid - part * (I2 * I2);
+      const int ei = rem / I2, ej = rem - ei * I2;
+      const int iy = ei / I, ix = ei - iy * I, jy = ej / I, jx = ej - jy * I;
+      const int o01 = (ix * I + jx) * I2 + iy * I + jy, o23 = (iy * I + jy) * I2 + ix * I + jx;
+      auto at = [&](int w, int o) { return lds[(w * (CPLX ? 2 : 1) + part) * I2 * I2 + o]; };
+      aval = (at(0, o01) + at(2, o01)) + (at(1, o23) + at(3, o23));
     }
     __syncthreads();
   } else if constexpr (CLS == 2) {
@@ -889,107 +1172,114 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
         const bool sw = k >= 2, odd = k & 1;
         const double pu = sw ? t2 : t1, qu = sw ? t4 : t3;
         const double r = sw ? t1 : t2, sv = sw ? t3 : t4;
-        const PtK a = make_point<PD, KIND>(cp1, l1x, l1y, h, pu, odd ? sv : r, w);
-        const PtK b = make_point<PD, KIND>(cp1, l1x, l1y, h, qu, odd ? r : sv, wj);
+        const PtK a = make_point<PD, KIND>(g1, prm, pu, odd ? sv : r, w);
+        const PtK b = make_point<PD, KIND>(g1, prm, qu, odd ? r : sv, wj);
         acc.add(a, b, prm, rc, cc, valid, lane);
         acc.add(b, a, prm, rc, cc, valid, lane);
       }
     }
   } else if constexpr (CLS == 3 && !Acc::MAXW) {
-    // integrate3, factorised: the sub-regions and points of the unfactorised form below.  Outer
-    // point (i, j0), inner index j1.  g = 0: rows (t1, e0) and columns (t2, e1) from the tables;
-    // g = 1: rows (t3, xi1) from the tables, columns on element 2 at tau(t4 or 1 - t4, e1; r2);
-    // g = 2: rows on element 1 at tau(t4 or 1 - t4, e1; r1), columns (t3, xi1) from the tables.
-    // The computed points come from the contracted line of their (i, j0).  The weight products
-    // are split into the outer factor (w and the j0 part of the inner weights) and gw[j1].
+    // integrate3, factorised: the sub-regions and points of the unfactorised form below.  Unit (i, j0), inner
+    // index j1.  g = 0: rows (t1, e0), columns (t2, e1); g = 1: rows (t3, xi1), columns on element 2 at
+    // tau(t4 or 1 - t4, e1; r2); g = 2: rows on element 1 at tau(t4 or 1 - t4, e1; r1), columns (t3, xi1).
+    // The weight products are split into the unit's factor (w and the j0 part of the inner weights)
+    // and gw[j1].  What a unit needs of each point:
+    // * (t4, e1) runs along a coordinate line over j1: one contraction per unit, held in registers, and
+    //   a one-dimensional evaluation per j1;
+    // * (t3, xi1) lies on the line of xi1: 2 n lines per element pair, contracted into LDS once;
+    // * (t1, e0) once per unit, and (t2, e1) from a table per chunk of i, shared by the j0.
+    // In every sub-region the inner points have one coordinate in common, so their sum is over P + 1
+    // basis values (line_pass).  Bound: FP64 VALU, two waves per SIMD.
     const int r1 = pr.rot1, r2 = pr.rot2;
     constexpr bool CPLX = Acc::CPLX;
-    const FactorShape shp = edge_shape(n, NT, static_cast<int>(sizeof(PtK)), Acc::G);
+    constexpr int LST = line_stride(PD);
+    const FactorShape shp = edge_shape(n, NT, static_cast<int>(sizeof(PtK)));
     const int CI = shp.chunk, S = shp.lanes;
-    const int role = lane & (Acc::G - 1);
-    // tau(x, y; r) fixes u for r = 0, 2: the line of a computed point runs along v there
-    PtK* tab = reinterpret_cast<PtK*>(lds);
+    PtK* tab = reinterpret_cast<PtK*>(lds);  // (odd, ci, j1)
+    double* lines = lds + (2 * CI * n * static_cast<int>(sizeof(PtK)) >> 3);  // (element, i1)
+    double* stage = lines + 2 * n * LST + (tid >> 6) * stage_doubles<I2>(CPLX);
+    // tau(x, y; r) with y fixed: the fixed and the moving local coordinate
+    auto held = [](int r, double y) { return (r == 0 || r == 3) ? y : 1 - y; };
+    auto moved = [](int r, double x) { return r < 2 ? x : 1 - x; };
+    for (int l = tid; l < 2 * n; l += NT) {
+      const int el = l / n, r = el ? r2 : r1;
+      double L[8 * PD];
+      line_contract<PD>(el ? g2 : g1, r & 1, held(r, gx[l - el * n]), L);
+#pragma unroll
+      for (int k = 0; k < 8 * PD; ++k) lines[l * LST + k] = L[k];
+    }
     for (int i0 = 0; i0 < nq; i0 += CI) {
       const int cn = nq - i0 < CI ? nq - i0 : CI;
       const int per = cn * n;
       __syncthreads();
-      for (int e = tid; e < 8 * per; e += NT) {
-        const int kind = e / per, rem = e - kind * per;
-        const int ci = rem / n, jx = rem - ci * n;
-        const int i = i0 + ci;
-        const double xi0 = gx[i / n], xi1 = gx[i % n], xj = gx[jx];
-        const bool odd = kind & 1;
+      for (int e = tid; e < 2 * per; e += NT) {
+        const bool odd = e >= per;
+        const int rem = odd ? e - per : e, ci = rem / n, jx = rem - ci * n, i = i0 + ci;
+        const double xi0 = gx[i / n], xi1 = gx[i % n];
+        const double t2 = (1 - xi0) * (1 - xi1);
         double u, v;
-        if (kind < 2) {
-          const double t1 = xi0 * (1 - xi1);
-          tau(odd ? 1 - t1 : t1, xi1 * xj, r1, u, v);
-          tab[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
-        } else if (kind < 4) {
-          const double t3 = xi0 * (1 - xi1 * xj);
-          tau(odd ? 1 - t3 : t3, xi1, r1, u, v);
-          tab[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
-        } else if (kind < 6) {
-          const double t3 = xi0 * (1 - xi1 * xj);
-          tau(odd ? 1 - t3 : t3, xi1, r2, u, v);
-          tab[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
-        } else {
-          const double t2 = (1 - xi0) * (1 - xi1);
-          tau(odd ? 1 - t2 : t2, xi1 * xj, r2, u, v);
-          tab[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
-        }
+        tau(odd ? 1 - t2 : t2, xi1 * gx[jx], r2, u, v);
+        tab[e] = make_point<PD, KIND>(g2, prm, u, v, gw[jx]);
       }
       __syncthreads();
-      const int units = cn * n;
       const int unit = tid / S, sub = tid - (tid / S) * S;
-      const bool act = unit < units;
+      const bool act = unit < per;
       const int uu = act ? unit : 0;
       const int ci = uu / n, j0 = uu - (uu / n) * n;
-      const int i = i0 + ci;
-      const double xi0 = gx[i / n], xi1 = gx[i % n], wi = gw[i / n] * gw[i % n];
+      const int i = i0 + ci, i1 = i % n;
+      const double xi0 = gx[i / n], xi1 = gx[i1], wi = gw[i / n] * gw[i1];
       const double w = h * h * wi * xi1 * xi1;
       const double e0 = xi1 * gx[j0];
-      const double t4 = (1 - xi0) * (1 - e0);
+      const double t1 = xi0 * (1 - xi1), t2 = (1 - xi0) * (1 - xi1), t3 = xi0 * (1 - e0), t4 = (1 - xi0) * (1 - e0);
       const double fa = w * (gw[j0] * (1 - xi1)), fb = w * (gw[j0] * (1 - e0));
-      const int ta = ci * n + j0;
       const PtK* colt = tab + ci * n;
+      // the point (t3 or 1 - t3, xi1) of element 1 or 2
+      auto on_line = [&](int el, double x) {
+        const int r = el ? r2 : r1;
+        const bool fu = r & 1;
+        const double f = held(r, xi1), m = moved(r, x);
+        return line_point<PD, KIND>(lines + (el * n + i1) * LST, prm, fu, fu ? f : m, fu ? m : f, fb);
+      };
 #pragma unroll 1
       for (int odd = 0; odd < 2; ++odd) {
+        {
+          double u, v;
+          tau(odd ? 1 - t1 : t1, e0, r1, u, v);
+          const PtK F = make_point<PD, KIND>(g1, prm, u, v, fa);
+          const double xc = moved(r2, odd ? 1 - t2 : t2);
+          auto col = [&](int j1) { return colt[odd * per + j1]; };
+          if (r2 & 1)
+            line_pass<P, KIND, true, false>(dr, di, stage, F, lane, act, sub, S, n, prm, xc, col);
+          else
+            line_pass<P, KIND, true, true>(dr, di, stage, F, lane, act, sub, S, n, prm, xc, col);
+        }
         const double x = odd ? 1 - t4 : t4;
-        // g = 0: table rows and columns
-        PtK F = tab[odd * per + ta];
-        F.W *= fa;
-        factor_pass<P, KIND, true>(acc, F, role, act, sub, S, n, prm, [&](int j1) {
-          PtK b = colt[(6 + odd) * per + j1];
-          b.W *= gw[j1];
-          return b;
-        });
-        // g = 1: table rows, columns on the line of element 2 (the rotation, uniform in the
-        // workgroup, fixed at compile time: tau and the line evaluation without selects)
-        F = tab[(2 + odd) * per + ta];
-        F.W *= fb;
+        // g = 1, 2: the rotation, uniform in the workgroup, fixed at compile time (tau and the line
+        // evaluation without selects)
+        const LinePt F1 = on_line(0, odd ? 1 - t3 : t3);
         with_rotation(r2, [&](auto R) {
           constexpr int RC = decltype(R)::value;
           constexpr bool FS = (RC & 1) == 0;
           double L[8 * PD];
-          line_contract<PD>(cp2, FS, FS ? l2x + h * (RC < 2 ? x : 1 - x) : l2y + h * (RC < 2 ? x : 1 - x), L);
-          factor_pass<P, KIND, true>(acc, F, role, act, sub, S, n, prm, [&](int j1) {
+          const double xf = RC < 2 ? x : 1 - x;
+          line_contract<PD>(g2, FS, xf, L);
+          line_pass<P, KIND, true, FS>(dr, di, stage, F1, lane, act, sub, S, n, prm, xf, [&](int j1) {
             double u, v;
             tau(x, xi1 * gx[j1], RC, u, v);
-            return line_point<PD, KIND>(L, FS, l2x, l2y, h, u, v, gw[j1]);
+            return line_point<PD, KIND>(L, prm, FS, u, v, gw[j1]);
           });
         });
-        // g = 2: rows on the line of element 1, table columns
-        F = tab[(4 + odd) * per + ta];
-        F.W *= fb;
+        const LinePt F2 = on_line(1, odd ? 1 - t3 : t3);
         with_rotation(r1, [&](auto R) {
           constexpr int RC = decltype(R)::value;
           constexpr bool FS = (RC & 1) == 0;
           double L[8 * PD];
-          line_contract<PD>(cp1, FS, FS ? l1x + h * (RC < 2 ? x : 1 - x) : l1y + h * (RC < 2 ? x : 1 - x), L);
-          factor_pass<P, KIND, false>(acc, F, role, act, sub, S, n, prm, [&](int j1) {
+          const double xf = RC < 2 ? x : 1 - x;
+          line_contract<PD>(g1, FS, xf, L);
+          line_pass<P, KIND, false, FS>(dr, di, stage, F2, lane, act, sub, S, n, prm, xf, [&](int j1) {
             double u, v;
             tau(x, xi1 * gx[j1], RC, u, v);
-            return line_point<PD, KIND>(L, FS, l1x, l1y, h, u, v, gw[j1]);
+            return line_point<PD, KIND>(L, prm, FS, u, v, gw[j1]);
           });
         });
       }
@@ -1010,13 +1300,13 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
       const double w = h * h * wi * (xi0 * xi0 * xi0);
       double u, v;
       tau(xi0, xi1, r1, u, v);
-      q[4 * i + 0] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
+      q[4 * i + 0] = make_point<PD, KIND>(g1, prm, u, v, w);
       tau(xi1, xi0, r1, u, v);
-      q[4 * i + 1] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
+      q[4 * i + 1] = make_point<PD, KIND>(g1, prm, u, v, w);
       tau(xi0, xi1, r2, u, v);
-      q[4 * i + 2] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q[4 * i + 2] = make_point<PD, KIND>(g2, prm, u, v, w);
       tau(xi1, xi0, r2, u, v);
-      q[4 * i + 3] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q[4 * i + 3] = make_point<PD, KIND>(g2, prm, u, v, w);
     }
     const FactorShape shp = vertex_shape(n, NT, static_cast<int>(sizeof(PtK)), Acc::G);
     const int C0 = shp.chunk, S = shp.lanes;
@@ -1033,10 +1323,10 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
         double u, v;
         if (which == 0) {
           tau(e0, e1, r2, u, v);
-          tin[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, wj);
+          tin[e] = make_point<PD, KIND>(g2, prm, u, v, wj);
         } else {
           tau(e0, e1, r1, u, v);
-          tin[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, wj);
+          tin[e] = make_point<PD, KIND>(g1, prm, u, v, wj);
         }
       }
       __syncthreads();
@@ -1081,19 +1371,19 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
         if (kind < 2) {  // g = 0, a: (t1, e0) on element 1
           const double t1 = xi0 * (1 - xi1);
           tau(odd ? 1 - t1 : t1, xi1 * xj, r1, u, v);
-          tab[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
+          tab[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
         } else if (kind < 4) {  // g = 1, a: (t3, xi1) on element 1
           const double t3 = xi0 * (1 - xi1 * xj);
           tau(odd ? 1 - t3 : t3, xi1, r1, u, v);
-          tab[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
+          tab[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
         } else if (kind < 6) {  // g = 2, b: (t3, xi1) on element 2
           const double t3 = xi0 * (1 - xi1 * xj);
           tau(odd ? 1 - t3 : t3, xi1, r2, u, v);
-          tab[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
+          tab[e] = make_point<PD, KIND>(g2, prm, u, v, 1.0);
         } else {  // g = 0, b: (t2, e1) on element 2 (xj = xj1)
           const double t2 = (1 - xi0) * (1 - xi1);
           tau(odd ? 1 - t2 : t2, xi1 * xj, r2, u, v);
-          tab[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
+          tab[e] = make_point<PD, KIND>(g2, prm, u, v, 1.0);
         }
       }
       __syncthreads();
@@ -1123,11 +1413,11 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
             double u, v;
             a = tab[(2 + odd) * per + ta];
             tau(odd ? 1 - t4 : t4, e1, r2, u, v);
-            b = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
+            b = make_point<PD, KIND>(g2, prm, u, v, 1.0);
           } else {
             double u, v;
             tau(odd ? 1 - t4 : t4, e1, r1, u, v);
-            a = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
+            a = make_point<PD, KIND>(g1, prm, u, v, 1.0);
             b = tab[(4 + odd) * per + ta];
           }
           a.W *= w;
@@ -1150,13 +1440,13 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
       const double w = h * h * wi * (xi0 * xi0 * xi0);
       double u, v;
       tau(xi0, xi1, r1, u, v);
-      q[4 * i + 0] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
+      q[4 * i + 0] = make_point<PD, KIND>(g1, prm, u, v, w);
       tau(xi1, xi0, r1, u, v);
-      q[4 * i + 1] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, w);
+      q[4 * i + 1] = make_point<PD, KIND>(g1, prm, u, v, w);
       tau(xi0, xi1, r2, u, v);
-      q[4 * i + 2] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q[4 * i + 2] = make_point<PD, KIND>(g2, prm, u, v, w);
       tau(xi1, xi0, r2, u, v);
-      q[4 * i + 3] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, w);
+      q[4 * i + 3] = make_point<PD, KIND>(g2, prm, u, v, w);
     }
     const int C0 = vertex_chunk<PtK>(n, NT);
     for (int a0 = 0; a0 < n; a0 += C0) {
@@ -1170,10 +1460,10 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
         double u, v;
         if (which == 0) {
           tau(e0, e1, r2, u, v);
-          tin[e] = make_point<PD, KIND>(cp2, l2x, l2y, h, u, v, 1.0);
+          tin[e] = make_point<PD, KIND>(g2, prm, u, v, 1.0);
         } else {
           tau(e0, e1, r1, u, v);
-          tin[e] = make_point<PD, KIND>(cp1, l1x, l1y, h, u, v, 1.0);
+          tin[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
         }
       }
       __syncthreads();
@@ -1200,8 +1490,18 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
   // reduce the per-lane partial blocks and write the result
   double* red = lds;
   double* sum = lds + (NT / 64) * Acc::TOT;
-  if constexpr ((CLS == 2 && (KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL)) || (CLS == 1 && !Acc::MAXW)) {
+  if constexpr ((CLS == 2 && IDENT) || (CLS == 1 && !Acc::MAXW)) {
     if (tid < Acc::TOT) sum[tid] = aval;  // each entry summed by its owner
+    __syncthreads();
+  } else if constexpr (CLS == 3 && !Acc::MAXW) {
+    // the four waves' blocks (the rules above end with a barrier)
+    spread_blocks<I2, Acc::CPLX>(lds, tid >> 6, lane, dr, di);
+    for (int k = tid; k < Acc::TOT; k += NT) {
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < NT / 64; ++w) v += lds[w * Acc::TOT + k];
+      sum[k] = v;
+    }
     __syncthreads();
   } else {
     reduce_block<NT>(acc, red, tid, sum);
@@ -1210,7 +1510,7 @@ __global__ __launch_bounds__(NT) void k_nearfield(const NFPair* __restrict__ pai
   constexpr bool CPLX = Acc::CPLX;
   const int64_t base = pr.off + rc * prm.comp_rs + cc * prm.comp_cs;
   // the factorised identical rule accumulated A; its block is A + A^T
-  constexpr bool SYMW = CLS == 2 && (KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL);
+  constexpr bool SYMW = CLS == 2 && IDENT;
   for (int k = tid; k < I2 * I2; k += NT) {
     const int i = k / I2, j = k - (k / I2) * I2;
     const int64_t idx = base + i * prm.rs + j * prm.cs;
@@ -1268,6 +1568,64 @@ void launch_ffield_table(const bmi_space* s, int n, int fs, double* out, hipStre
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+// the homogeneous coordinates of every element in powers of u - 1/2, v - 1/2 (poly_point): coefficient
+// (a, b) is h^(a + b) / (a! b!) times the derivative at the element's centre, from differences of the
+// control points in Bernstein form; one thread per (element, a, b)
+template <int PD>
+__global__ void k_element_poly(const double* __restrict__ cp, int cp_stride, const int* __restrict__ elem_patch,
+                               const double* __restrict__ elem_llc, int nel, double h, double* __restrict__ out) {
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (gid >= static_cast<int64_t>(nel) * PD * PD) return;
+  const int e = static_cast<int>(gid / (PD * PD)), q = static_cast<int>(gid % (PD * PD));
+  const double* c = cp + static_cast<int64_t>(elem_patch[e]) * cp_stride;
+  // weights of the control points in the a-th power coefficient of one direction about x:
+  // h^a binom(p, a) sum over r of (-1)^(a - r) binom(a, r) B_(i - r) of degree p - a
+  auto weights = [&](int a, double x, double* w) {
+    constexpr int p = PD - 1;
+    double B[PD];
+    for (int i = 0; i < PD; ++i) w[i] = 0.0, B[i] = 0.0;
+    B[0] = 1.0;
+    for (int d = 1; d <= p - a; ++d)  // Bernstein recurrence up to degree p - a
+      for (int i = d; i >= 0; --i) B[i] = (i > 0 ? x * B[i - 1] : 0.0) + (i < d ? (1 - x) * B[i] : 0.0);
+    double f = 1.0;
+    for (int k = 0; k < a; ++k) f = f * (p - k) / (k + 1) * h;
+    double bin = 1.0;
+    for (int r = 0; r <= a; ++r) {
+      const double g = ((a - r) & 1) ? -f * bin : f * bin;
+      for (int i = 0; i + a <= p; ++i) w[i + r] += g * B[i];
+      bin = bin * (a - r) / (r + 1);
+    }
+  };
+  double ws[PD], wt[PD];
+  weights(q / PD, elem_llc[2 * e] + 0.5 * h, ws);
+  weights(q % PD, elem_llc[2 * e + 1] + 0.5 * h, wt);
+  double v[4] = {0, 0, 0, 0};
+  for (int j = 0; j < PD; ++j) {
+    double r[4] = {0, 0, 0, 0};
+    for (int i = 0; i < PD; ++i)
+      for (int k = 0; k < 4; ++k) r[k] += ws[i] * c[4 * (i * PD + j) + k];
+    for (int k = 0; k < 4; ++k) v[k] += wt[j] * r[k];
+  }
+  for (int k = 0; k < 4; ++k) out[gid * 4 + k] = v[k];
+}
+
+static const double* element_polynomials(const bmi_space* s, DevBuf<double>& buf, hipStream_t st) {
+  const int64_t n = static_cast<int64_t>(s->nel) * s->pd * s->pd;
+  buf.alloc(static_cast<size_t>(4 * n));
+  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+  const int stride = 4 * s->pd * s->pd;
+  if (s->pd == 2)
+    hipLaunchKernelGGL(k_element_poly<2>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
+                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, buf.ptr);
+  else if (s->pd == 5)
+    hipLaunchKernelGGL(k_element_poly<5>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
+                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, buf.ptr);
+  else
+    throw Error(BMI_UNSUPPORTED, "patch degree not supported on the device");
+  BMI_CHECK_HIP(hipGetLastError());
+  return buf.ptr;
+}
+
 // dynamic LDS of one workgroup of class CLS at quadrature degree deg (each workgroup sizes its
 // point tables from its own pair's degree)
 template <int P, int KIND, int PD, int CLS, int NT>
@@ -1282,11 +1640,16 @@ static size_t class_lds_bytes(int deg) {
   constexpr bool FACT = KIND != BMI_MAXWELL_SL;  // factorised vertex rule
   constexpr int PS = static_cast<int>(sizeof(Pt<KIND>));
   const int cv = FACT ? vertex_shape(n, NT, PS, BlockAcc<P, KIND>::G).chunk : vertex_chunk<Pt<KIND>>(n, NT);
-  const int ce = FACT ? edge_shape(n, NT, PS, BlockAcc<P, KIND>::G).chunk : edge_chunk<Pt<KIND>>(n, NT);
-  if (CLS == 3) lds = std::max(lds, static_cast<size_t>(8 * n * ce) * sizeof(Pt<KIND>));
-  if (CLS == 2 && (KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL))
-    lds = std::max(lds, static_cast<size_t>(NT / 4) * (32 * PD + 2 + 7 + (BlockAcc<P, KIND>::CPLX ? 4 : 2) *
-                                                     (P + 1) * (P + 1)) * sizeof(double));  // lines, unit records
+  // the waves' vectors behind the tables (factorised edge rule)
+  const size_t stg = FACT ? (NT / 64) * stage_doubles<(P + 1) * (P + 1)>(BlockAcc<P, KIND>::CPLX) * sizeof(double) : 0;
+  if (CLS == 3)
+    lds = std::max(lds, FACT ? static_cast<size_t>(2 * n * edge_shape(n, NT, PS).chunk) * sizeof(Pt<KIND>) +
+                                   static_cast<size_t>(2 * n * line_stride(PD)) * sizeof(double) + stg
+                             : static_cast<size_t>(8 * n * edge_chunk<Pt<KIND>>(n, NT)) * sizeof(Pt<KIND>));
+  if (CLS == 2 && (KIND == BMI_LAPLACE_SL || KIND == BMI_HELMHOLTZ_SL))  // lines, the waves' unit vectors
+    lds = std::max(lds, (static_cast<size_t>(identical_chunk(n, PD)) * 4 * n * line_stride(PD) +
+                         static_cast<size_t>(NT / 2) * (BlockAcc<P, KIND>::CPLX ? 3 : 2) * (P + 1) * (P + 1)) *
+                            sizeof(double));
   if (CLS == 4) lds = std::max(lds, static_cast<size_t>(4 * nq + 2 * nq * cv) * sizeof(Pt<KIND>));
   return lds;
 }
@@ -1382,12 +1745,13 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
     pairs.swap(sorted);
     d_pairs.upload(pairs, st);
   }
+  DevBuf<double> d_poly;
   NFParams prm;
-  prm.cp = s->d_cp.ptr;
-  prm.cp_stride = 4 * s->pd * s->pd;
-  prm.elem_patch = s->d_elem_patch.ptr;
-  prm.elem_llc = s->d_elem_llc.ptr;
+  prm.poly = element_polynomials(s, d_poly, st);
+  prm.poly_stride = 4 * s->pd * s->pd;
   prm.h = 1.0 / s->n;
+  prm.rh = s->n;
+  prm.rh2 = static_cast<double>(s->n) * s->n;
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;
   prm.dummy_fn = op.dummy_fn;
@@ -1432,12 +1796,13 @@ void launch_integrate_jobs(const bmi_space* s, const bmi_op_desc& op, const std:
   }
   DevBuf<NFPair> d_pairs;
   d_pairs.upload(pairs, st);
+  DevBuf<double> d_poly;
   NFParams prm;
-  prm.cp = s->d_cp.ptr;
-  prm.cp_stride = 4 * s->pd * s->pd;
-  prm.elem_patch = s->d_elem_patch.ptr;
-  prm.elem_llc = s->d_elem_llc.ptr;
+  prm.poly = element_polynomials(s, d_poly, st);
+  prm.poly_stride = 4 * s->pd * s->pd;
   prm.h = 1.0 / s->n;
+  prm.rh = s->n;
+  prm.rh2 = static_cast<double>(s->n) * s->n;
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;
   prm.dummy_fn = op.dummy_fn;
