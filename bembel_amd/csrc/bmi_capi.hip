@@ -359,8 +359,6 @@ static void apply_near(bmi_h2* h, int nrhs, const double* xs, double* ys, hipStr
               h->d_dense.ptr, xs, N, vcs, ys, N, vcs, st);
 }
 
-// time both variants of the two sweeps once (1 RHS) and keep the faster; the variants give
-// identical bits, so the choice affects speed only
 // names the timing scope of the sweep launches made while it lives
 struct SweepScopeName {
   explicit SweepScopeName(const char* n) { tl_sweep_scope = n; }
@@ -422,118 +420,118 @@ static bool fused_product(bmi_h2* h, const Work& w, const double* xs, double* ys
   return ok;
 }
 
+// The first single-column product of a handle picks its sweep kernels by timing: one untimed and two
+// timed launches of each candidate.  Variants of a form (blocks loaded per iteration) give the same
+// bits, forms agree to rounding.  The forms (every block, upper blocks, upper leaves too; for reduced
+// operators also blocks recomputed on the fly) are timed on one variant each and the variants of the
+// fastest form after that: 9 candidates instead of 18 (Laplace, 24,576 elements: first product
+// 16.9 -> 6.6 ms; Helmholtz mixed 34.3 -> 17.7 ms).  The kernels of the separate sweeps are timed only where no fused one exists.
 static void autotune(bmi_h2* h, const double* xs, bool reduced, hipStream_t st) {
   if (h->leaf_variant >= 0 && h->cpl_variant >= 0) return;
   hipEvent_t a, b;
   BMI_CHECK_HIP(hipEventCreate(&a));
   BMI_CHECK_HIP(hipEventCreate(&b));
+  // milliseconds of two runs of fn, or a negative number if it cannot run (fn returns false)
   auto time_it = [&](auto&& fn) {
-    fn();  // warm-up
+    if (!fn()) return -1.f;  // warm-up
     BMI_CHECK_HIP(hipEventRecord(a, st));
-    for (int r = 0; r < 3; ++r) fn();
+    for (int r = 0; r < 2; ++r) fn();
     BMI_CHECK_HIP(hipEventRecord(b, st));
     BMI_CHECK_HIP(hipEventSynchronize(b));
     float ms = 0.f;
     BMI_CHECK_HIP(hipEventElapsedTime(&ms, a, b));
     return ms;
   };
-  float best = 0.f;
-  int pick = 0;
-  for (int v = 0; v < 2; ++v) {
-    h->leaf_variant = v;
-    const float t = time_it([&] { apply_near(h, 1, xs, h->d_ys.ptr, st); });
-    if (v == 0 || t < best) best = t, pick = v;
-  }
-  h->leaf_variant = pick;
-  if (has_far(h) && !h->mxf) {
-    const int S = h->cplx ? 2 : 1;
-    const CouplingOperand co = coupling_operand(h, reduced);
-    const bool fp32 = co.fp32;
-    const void* coupF = co.F;
-    const int64_t cblk = co.blk;
-    device_fill(h->d_fw[0].ptr, S * h->lvl_total, 0.0, st);
-    pick = 0;
-    for (int v = 0; v < 2; ++v) {
-      const float t = time_it([&] {
-        launch_coupling_apply(h->cplx, fp32, v, h->ntgt, 1, h->cd, h->d_tgt.ptr, h->d_crp.ptr, h->d_csrc.ptr, coupF,
-                              h->vd * h->vd * cblk, 0, h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, 0, st, co.Fc,
-                              co.ncoarse, co.ld);
-      });
-      if (v == 0 || t < best) best = t, pick = v;
+  // the fastest of the candidates that run: forms on variant v0, then the other variants of the winner;
+  // (-1, -1) if none runs
+  auto pick = [&](const std::vector<int>& forms, int nv, int v0, auto&& fn) {
+    int form = -1, var = v0;
+    float best = 0.f;
+    for (int f : forms) {
+      const float t = time_it([&] { return fn(f, v0); });
+      if (t >= 0.f && (form < 0 || t < best)) best = t, form = f;
     }
-    h->cpl_variant = pick;
-    // the fused sweep: all four combinations (register use, and so occupancy, differs)
-    if (h->vd == 1) {
-      // full block lists, and (symmetric kernels, FP64 blocks) the upper blocks with transposed
-      // partials: the upper form reads half the coupling bytes but adds the column sums
-      int pl = -1, pc = -1, ps = 0;
-      // forms: 0 every block, 1 upper coupling blocks, 2 upper coupling blocks and upper near-field leaves
-      const int nsym = (h->sym && !fp32) ? (h->nsym ? 3 : 2) : 1;
-      const int s0 = h->sweep_mode >= 0 ? std::min(h->sweep_mode, nsym - 1) : 0;
-      const int s1 = h->sweep_mode >= 0 ? s0 : nsym - 1;
-      for (int sy = s0; sy <= s1; ++sy)
-        for (int vl = 0; vl < 2; ++vl)
-          for (int vc = 0; vc < 2; ++vc) {
-            bool ok = true;
-            const float t = time_it([&] {
-              ok = launch_sweep_fused(h->cplx, fp32, vl, vc, h->ncl_leaf, h->dd, h->d_drp.ptr, h->d_dsrc.ptr,
-                                      h->d_dense.ptr, xs, h->d_ys.ptr, h->ntgt, h->cd, h->d_tgt.ptr, h->d_crp.ptr,
-                                      h->d_csrc.ptr, coupF, h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, st, co.Fc,
-                                      co.ncoarse, false, co.ld, sy ? &h->sl : nullptr,
-                                      sy == 2 ? &h->nsl : nullptr);
-            });
-            if (ok && (pl < 0 || t < best)) best = t, pl = vl, pc = vc, ps = sy;
-          }
-      h->fused_leaf_variant = pl;
-      h->fused_cpl_variant = pc;
-      h->sym_fused = ps;
-      // whole products: both sweeps in one launch, or the near-field leaves beside the far chain
-      h->overlap = 0;
-      if (pl >= 0 && h->overlap_mode != 0) {
-        const Work w = handle_work(h);
-        if (h->overlap_mode > 0) {
-          h->overlap = 1;
-        } else {
-          float tb = 0.f;
-          for (int o = 0; o < 2; ++o) {
-            bool ok = true;
-            const float t = time_it([&] { ok = fused_product(h, w, xs, w.ys, w.yf, reduced, st, o == 1); });
-            if (ok && (o == 0 || t < tb)) tb = t, h->overlap = o;
-          }
-        }
-      }
+    for (int v = 0; form >= 0 && v < nv; ++v) {
+      if (v == v0) continue;
+      const float t = time_it([&] { return fn(form, v); });
+      if (t >= 0.f && t < best) best = t, var = v;
+    }
+    return std::make_pair(form, form < 0 ? -1 : var);
+  };
+  const bool far = has_far(h) && !h->mxf;
+  const CouplingOperand co = coupling_operand(h, reduced);
+  if (far) device_fill(h->d_fw[0].ptr, (h->cplx ? 2 : 1) * h->lvl_total, 0.0, st);
+  if (far && h->vd == 1) {
+    // forms: 0 every block, 1 upper coupling blocks, 2 upper coupling blocks and upper near-field leaves
+    // (FP64 blocks of symmetric kernels; the upper forms read half the bytes but add column sums)
+    const int nform = (h->sym && !co.fp32) ? (h->nsym ? 3 : 2) : 1;
+    std::vector<int> forms;
+    for (int f = 0; f < nform; ++f)
+      if (h->sweep_mode < 0 || f == std::min(h->sweep_mode, nform - 1)) forms.push_back(f);
+    const auto p = pick(forms, 4, 2, [&](int sy, int v) {
+      return launch_sweep_fused(h->cplx, co.fp32, v >> 1, v & 1, h->ncl_leaf, h->dd, h->d_drp.ptr, h->d_dsrc.ptr,
+                                h->d_dense.ptr, xs, h->d_ys.ptr, h->ntgt, h->cd, h->d_tgt.ptr, h->d_crp.ptr,
+                                h->d_csrc.ptr, co.F, h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, st, co.Fc,
+                                co.ncoarse, false, co.ld, sy ? &h->sl : nullptr, sy == 2 ? &h->nsl : nullptr);
+    });
+    h->fused_leaf_variant = p.first < 0 ? -1 : p.second >> 1;
+    h->fused_cpl_variant = p.first < 0 ? -1 : p.second & 1;
+    h->sym_fused = std::max(p.first, 0);
+    // whole products: both sweeps in one launch, or the near-field leaves beside the far chain
+    h->overlap = 0;
+    if (p.first >= 0 && h->overlap_mode != 0) {
+      const Work w = handle_work(h);
+      if (h->overlap_mode > 0)
+        h->overlap = 1;
+      else
+        h->overlap = std::max(0, pick({0, 1}, 1, 0, [&](int o, int) {
+                                   return fused_product(h, w, xs, w.ys, w.yf, reduced, st, o == 1);
+                                 }).first);
     }
     if (h->red1) {
-      // reduced single-RHS sweep: coupling recomputed on the fly (variants 0, 1; real kernels:
-      // an oscillatory kernel's FP32 phase is less accurate than the FP32-rounded FP64 entries and
-      // costs Krylov steps) or read from the FP32 copy (variants 2 + 2 * near blocks per
-      // iteration + coupling blocks per iteration), both with the FP32 near-field blocks;
-      // whichever is faster (arithmetic vs bytes)
-      // (variants 6-9: the FP32 copy's upper blocks with transposed partials)
-      int pv = -1;
-      const int v0 = (h->sym && h->sweep_mode >= 1) ? 6 : (h->fly ? 0 : 2);
-      const int v1 = (h->sym && h->sweep_mode != 0) ? 10 : 6;
-      for (int v = v0; v < v1; ++v) {
-        bool ok = true;
-        const float t = time_it([&] {
-          if (v < 2)
-            ok = launch_sweep_fly(h->cplx, v, h->ncl_leaf, h->dd, h->d_drp.ptr, h->d_dsrc.ptr, h->d_dense32.ptr, xs,
-                                  h->d_ys.ptr, h->ntgt, h->cd, h->d_tgt.ptr, h->d_crp.ptr, h->d_csrc.ptr,
-                                  h->d_lvl_off.ptr, h->d_fly_pts.ptr, h->d_fly_org.ptr, h->op.kappa_re,
-                                  h->op.kappa_im, h->d_fw[0].ptr, h->d_bw.ptr, st);
-          else
-            ok = launch_sweep_fused(h->cplx, true, ((v - 2) & 3) >> 1, (v - 2) & 1, h->ncl_leaf, h->dd,
-                                    h->d_drp.ptr, h->d_dsrc.ptr, h->d_dense32.ptr, xs, h->d_ys.ptr, h->ntgt, h->cd,
-                                    h->d_tgt.ptr, h->d_crp.ptr, h->d_csrc.ptr, h->d_coup32.ptr, h->d_lvl_off.ptr,
-                                    h->d_fw[0].ptr, h->d_bw.ptr, st, nullptr, 0, true, h->ld32,
-                                    v >= 6 ? &h->sl : nullptr);
-        });
-        if (ok && (pv < 0 || t < best)) best = t, pv = v;
+      // reduced single-RHS sweep, all with the FP32 near-field blocks: coupling recomputed on the fly
+      // (variants 0, 1; real kernels: an oscillatory kernel's FP32 phase is less accurate than the
+      // FP32-rounded FP64 entries and costs Krylov steps), read from the FP32 copy (2 + 2 * near
+      // blocks per iteration + coupling blocks per iteration), or its upper blocks (6 + ...)
+      auto run = [&](int base, int v) {
+        if (base == 0)
+          return v < 2 && launch_sweep_fly(h->cplx, v, h->ncl_leaf, h->dd, h->d_drp.ptr, h->d_dsrc.ptr,
+                                           h->d_dense32.ptr, xs, h->d_ys.ptr, h->ntgt, h->cd, h->d_tgt.ptr,
+                                           h->d_crp.ptr, h->d_csrc.ptr, h->d_lvl_off.ptr, h->d_fly_pts.ptr,
+                                           h->d_fly_org.ptr, h->op.kappa_re, h->op.kappa_im, h->d_fw[0].ptr,
+                                           h->d_bw.ptr, st);
+        return launch_sweep_fused(h->cplx, true, v >> 1, v & 1, h->ncl_leaf, h->dd, h->d_drp.ptr, h->d_dsrc.ptr,
+                                  h->d_dense32.ptr, xs, h->d_ys.ptr, h->ntgt, h->cd, h->d_tgt.ptr, h->d_crp.ptr,
+                                  h->d_csrc.ptr, h->d_coup32.ptr, h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, st,
+                                  nullptr, 0, true, h->ld32, base == 6 ? &h->sl : nullptr);
+      };
+      std::vector<int> bases;
+      if (!(h->sym && h->sweep_mode >= 1)) {
+        if (h->fly) bases.push_back(0);
+        bases.push_back(2);
       }
-      h->fly_variant = pv;
+      if (h->sym && h->sweep_mode != 0) bases.push_back(6);
+      const auto q = pick(bases, 4, 1, run);
+      h->fly_variant = q.first < 0 ? -1 : q.first + q.second;
     }
-  } else {
-    h->cpl_variant = 0;
+  }
+  h->leaf_variant = h->cpl_variant = 0;
+  if (h->fused_leaf_variant < 0) {
+    // no fused sweep for these sizes
+    if (h->vd == 1 && wave_leaf_supported(h->dd))
+      h->leaf_variant = std::max(0, pick({0, 1}, 1, 0, [&](int v, int) {
+                                      h->leaf_variant = v;
+                                      apply_near(h, 1, xs, h->d_ys.ptr, st);
+                                      return true;
+                                    }).first);
+    if (far && wave_coupling_supported(h->cplx, h->cd))
+      h->cpl_variant = std::max(0, pick({0, 1}, 1, 0, [&](int v, int) {
+                                     launch_coupling_apply(h->cplx, co.fp32, v, h->ntgt, 1, h->cd, h->d_tgt.ptr,
+                                                           h->d_crp.ptr, h->d_csrc.ptr, co.F, co.blk, 0,
+                                                           h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, 0, st,
+                                                           co.Fc, co.ncoarse, co.ld);
+                                     return true;
+                                   }).first);
   }
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);

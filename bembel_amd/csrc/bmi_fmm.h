@@ -43,6 +43,9 @@ void launch_coupling_assemble(int kind, const int4* d_leaves, int nleaves, int n
 void launch_spmv(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, const double* v, const double* x,
                  int64_t ldx, double* y, int64_t ldy, const double* alpha, const double* beta, hipStream_t st,
                  const double* x2 = nullptr, bool long_rows = false);
+// block sizes whose single columns run one wave per cluster, in two variants
+bool wave_leaf_supported(int dd);
+bool wave_coupling_supported(bool cplx, int cd);
 // variant: 0 = one block per lane group per iteration, 1 = two (chosen by the autotuner)
 // Fc/ncoarse: BF16 copies of the first ncoarse blocks (fp32 only); ld: column stride of F (0: cd)
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,

@@ -2352,6 +2352,9 @@ void launch_spmv(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, c
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+bool wave_leaf_supported(int dd) { return dd == 16 || dd == 36; }
+bool wave_coupling_supported(bool cplx, int cd) { return cd == 16 || cd == 25 || (cplx && cd == 32); }
+
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,
                            const int* rp, const int* src, const void* F, int64_t fstride, int64_t fcomp,
                            const int64_t* lvl_off, const double* fw, double* bw, int accumulate, hipStream_t st,
