@@ -109,6 +109,61 @@ void launch_mirror_blocks(int64_t nm, const int64_t* map, int I2, int dd, int64_
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+// the part of a symmetric matrix (N x N, column-major, S doubles per entry) whose row element is behind
+// its column element, from the other part: entry (i, j) with element(i) > element(j) = entry (j, i);
+// super rows are component-major, I2 per element within a component of vcs rows.  32 x 32 tiles through
+// LDS, so that both sides are read and written along columns.
+template <int S>
+__global__ __launch_bounds__(256) void k_mirror_dense(int64_t N, int64_t vcs, int I2, double* A) {
+  __shared__ double tile[S * 32 * 33];
+  const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 32, j0 = static_cast<int64_t>(blockIdx.y) * 32;
+  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  // source entries (j, i) at A[i * N + j]: consecutive threads walk j
+  for (int r = ty; r < 32; r += 8) {
+    const int64_t i = i0 + r, j = j0 + tx;
+    if (i < N && j < N)
+      for (int t = 0; t < S; ++t) tile[S * (r * 33 + tx) + t] = A[S * (i * N + j) + t];
+  }
+  __syncthreads();
+  for (int r = ty; r < 32; r += 8) {
+    const int64_t i = i0 + tx, j = j0 + r;
+    if (i < N && j < N && (i % vcs) / I2 > (j % vcs) / I2)
+      for (int t = 0; t < S; ++t) A[S * (j * N + i) + t] = tile[S * (tx * 33 + r) + t];
+  }
+}
+void launch_mirror_dense(bool cplx, int64_t N, int64_t vcs, int I2, double* A, hipStream_t st) {
+  const unsigned n = static_cast<unsigned>((N + 31) / 32);
+  if (cplx)
+    hipLaunchKernelGGL(k_mirror_dense<2>, dim3(n, n), dim3(256), 0, st, N, vcs, I2, A);
+  else
+    hipLaunchKernelGGL(k_mirror_dense<1>, dim3(n, n), dim3(256), 0, st, N, vcs, I2, A);
+  BMI_CHECK_HIP(hipGetLastError());
+}
+
+// C = A T for a dense column-major A (N rows, S doubles per entry): column j of C is the sum of the
+// columns of A that T^T's row j lists; consecutive threads on consecutive rows.  Bound: HBM, A once
+// per reading column (neighbouring columns of C share them through the caches).
+template <int S>
+__global__ __launch_bounds__(256) void k_times_t(int64_t N, const int* __restrict__ trp, const int* __restrict__ tcol,
+                                                 const double* __restrict__ tval, const double* __restrict__ A,
+                                                 double* __restrict__ C) {
+  const int64_t i = static_cast<int64_t>(blockIdx.y) * blockDim.x + threadIdx.x, j = blockIdx.x;
+  if (i >= S * N) return;  // double i of the column
+  double v = 0.0;
+  for (int p = trp[j]; p < trp[j + 1]; ++p) v += tval[p] * A[S * tcol[p] * N + i];
+  C[S * j * N + i] = v;
+}
+void launch_times_t(bool cplx, int64_t N, int64_t D, const int* trp, const int* tcol, const double* tval, const double* A,
+                    double* C, hipStream_t st) {
+  const int S = cplx ? 2 : 1;
+  const dim3 grid(static_cast<unsigned>(D), static_cast<unsigned>((S * N + 255) / 256));
+  if (cplx)
+    hipLaunchKernelGGL(k_times_t<2>, grid, dim3(256), 0, st, N, trp, tcol, tval, A, C);
+  else
+    hipLaunchKernelGGL(k_times_t<1>, grid, dim3(256), 0, st, N, trp, tcol, tval, A, C);
+  BMI_CHECK_HIP(hipGetLastError());
+}
+
 __global__ void k_fill(double* p, int64_t n, double v) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -788,6 +843,48 @@ bool h2_is_symmetric_real(const bmi_h2* h) { return h->op.kind == BMI_LAPLACE_SL
 bool h2_is_mixed(const bmi_h2* h) { return h->op.precision != BMI_PRECISION_FP64; }
 
 // ------------------------------------------------------------------ assembly
+// fn(thread, begin, end) over [0, n) in contiguous ranges, on up to 16 threads with at least `grain`
+// items each; an exception of any of them is rethrown here.
+template <class F>
+static void parallel_ranges(int64_t n, int64_t grain, F&& fn) {
+  const int nth = static_cast<int>(std::max<int64_t>(
+      1, std::min<int64_t>(std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency())), n / grain)));
+  std::vector<std::string> errors(nth);
+  auto work = [&](int t) {
+    try {
+      fn(t, n * t / nth, n * (t + 1) / nth);
+    } catch (const std::exception& e) {
+      errors[t] = e.what();
+      if (errors[t].empty()) errors[t] = "host phase failed";
+    }
+  };
+  std::vector<std::thread> pool;
+  for (int t = 1; t < nth; ++t) pool.emplace_back(work, t);
+  work(0);
+  for (auto& th : pool) th.join();
+  for (const std::string& e : errors) BMI_REQUIRE(e.empty(), BMI_UNSUPPORTED, e);
+}
+
+// class, Duffy rotations and quadrature degree of the element pair (e1, e2) (a pure function of the
+// space); ff: the far-field degree of the operator
+static NFPair classify_pair(const bmi_space* s, int kind, int ff, int e1, int e2, int64_t off) {
+  NFPair p;
+  p.e1 = e1;
+  p.e2 = e2;
+  int cp[3];
+  double dist;
+  compare_elements(s, e1, e2, cp, &dist);
+  int nf = nearfield_degree(kind, s->P, dist, s->M);
+  nf = nf >= ff ? nf : ff;
+  BMI_REQUIRE(nf < 50, BMI_UNSUPPORTED, "near-field quadrature degree too large");
+  p.cls = (cp[2] == 0) ? (nf == ff ? 0 : 1) : cp[2];
+  p.rot1 = cp[0];
+  p.rot2 = cp[1];
+  p.deg = nf;
+  p.off = off;
+  return p;
+}
+
 // Coupling blocks of a symmetric kernel pair up: (level, c2, c1) is the transpose of (level, c1,
 // c2) (same kernel values; the two weights multiply in the other order). For single-RHS sweeps
 // list one block per pair under its smaller cluster c1 (the upper block (c1, c2) for real
@@ -968,51 +1065,24 @@ static void assemble_h2(bmi_h2* h, hipStream_t st) {
   const int ff = farfield_degree(op.kind, s->P);
   {
     HostTimedScope hs("assembly_host_pairs");
-    const int64_t nd = static_cast<int64_t>(quad.size());
-    const int nth = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(
-        std::min<unsigned>(16u, std::max(1u, std::thread::hardware_concurrency())), nd / 256)));
-    std::vector<std::array<int, 5>> counts(nth, std::array<int, 5>{0, 0, 0, 0, 0});
-    std::vector<std::string> errors(nth);
-    auto work = [&](int t) {
-      try {
-        for (int64_t kq = nd * t / nth; kq < nd * (t + 1) / nth; ++kq) {
-          const int64_t k = quad[kq];
-          const Leaf& lf = h->dense[k];
-          BMI_REQUIRE(lf.level == h->L, BMI_UNSUPPORTED, "dense leaf above the leaf level");
-          const bool dg = diag(static_cast<int>(k));
-          int64_t slot = pstart[kq];
-          for (int b = 0; b < ne; ++b)
-            for (int a = 0; a < ne; ++a) {
-              if (dg && a > b) continue;
-              NFPair& p = pairs[slot++];
-              p.e1 = lf.c1 * ne + a;
-              p.e2 = lf.c2 * ne + b;
-              int cp[3];
-              double dist;
-              compare_elements(s, p.e1, p.e2, cp, &dist);
-              int nf = nearfield_degree(op.kind, s->P, dist, s->M);
-              nf = nf >= ff ? nf : ff;
-              BMI_REQUIRE(nf < 50, BMI_UNSUPPORTED, "near-field quadrature degree too large");
-              p.cls = (cp[2] == 0) ? (nf == ff ? 0 : 1) : cp[2];
-              p.rot1 = cp[0];
-              p.rot2 = cp[1];
-              p.deg = nf;
-              p.off = sub_off(k, a, b);
-              counts[t][p.cls]++;
-            }
-        }
-      } catch (const std::exception& e) {
-        errors[t] = e.what();
+    std::array<std::array<int, 5>, 16> counts{};
+    parallel_ranges(static_cast<int64_t>(quad.size()), 256, [&](int t, int64_t q0, int64_t q1) {
+      for (int64_t kq = q0; kq < q1; ++kq) {
+        const int64_t k = quad[kq];
+        const Leaf& lf = h->dense[k];
+        BMI_REQUIRE(lf.level == h->L, BMI_UNSUPPORTED, "dense leaf above the leaf level");
+        const bool dg = diag(static_cast<int>(k));
+        int64_t slot = pstart[kq];
+        for (int b = 0; b < ne; ++b)
+          for (int a = 0; a < ne; ++a) {
+            if (dg && a > b) continue;
+            pairs[slot] = classify_pair(s, op.kind, ff, lf.c1 * ne + a, lf.c2 * ne + b, sub_off(k, a, b));
+            counts[t][pairs[slot++].cls]++;
+          }
       }
-    };
-    std::vector<std::thread> pool;
-    for (int t = 1; t < nth; ++t) pool.emplace_back(work, t);
-    work(0);
-    for (auto& th : pool) th.join();
-    for (int t = 0; t < nth; ++t) {
-      BMI_REQUIRE(errors[t].empty(), BMI_UNSUPPORTED, errors[t]);
-      for (int c = 0; c < 5; ++c) h->pair_class_count[c] += counts[t][c];
-    }
+    });
+    for (const auto& ct : counts)
+      for (int c = 0; c < 5; ++c) h->pair_class_count[c] += ct[c];
   }
   h->npairs = static_cast<int64_t>(pairs.size());
   // component block (rc, cc) of leaf k starts at (k*vd*vd + rc*vd + cc) * dblk
@@ -1456,21 +1526,9 @@ bmi_status bmi_pair_blocks(const bmi_space* s, const bmi_op_desc* op, int npairs
   const int ff = farfield_degree(op->kind, s->P);
   std::vector<NFPair> v(npairs);
   for (int k = 0; k < npairs; ++k) {
-    NFPair& p = v[k];
-    p.e1 = pairs[2 * k];
-    p.e2 = pairs[2 * k + 1];
-    BMI_REQUIRE(p.e1 >= 0 && p.e1 < s->nel && p.e2 >= 0 && p.e2 < s->nel, BMI_INVALID_ARG, "element out of range");
-    int cp[3];
-    double dist;
-    compare_elements(s, p.e1, p.e2, cp, &dist);
-    int nf = nearfield_degree(op->kind, s->P, dist, s->M);
-    nf = nf >= ff ? nf : ff;
-    BMI_REQUIRE(nf < 50, BMI_UNSUPPORTED, "near-field quadrature degree too large");
-    p.cls = (cp[2] == 0) ? (nf == ff ? 0 : 1) : cp[2];
-    p.rot1 = cp[0];
-    p.rot2 = cp[1];
-    p.deg = nf;
-    p.off = static_cast<int64_t>(k) * n * n;
+    const int e1 = pairs[2 * k], e2 = pairs[2 * k + 1];
+    BMI_REQUIRE(e1 >= 0 && e1 < s->nel && e2 >= 0 && e2 < s->nel, BMI_INVALID_ARG, "element out of range");
+    v[k] = classify_pair(s, op->kind, ff, e1, e2, static_cast<int64_t>(k) * n * n);
   }
   DevBuf<double> d_out;
   d_out.alloc(static_cast<size_t>(npairs) * n * n * (cplx ? 2 : 1));
@@ -1515,63 +1573,44 @@ bmi_status bmi_dense_assemble(const bmi_space* s, const bmi_op_desc* op, int sup
   const int S = cplx ? 2 : 1;
   const int64_t N = s->nsuper, D = s->ndof;
   const int ff = farfield_degree(op->kind, s->P);
-  std::vector<NFPair> v;
-  v.reserve(static_cast<size_t>(s->nel) * s->nel);
-  for (int e2 = 0; e2 < s->nel; ++e2)
-    for (int e1 = 0; e1 < s->nel; ++e1) {
-      NFPair p;
-      p.e1 = e1;
-      p.e2 = e2;
-      int cp[3];
-      double dist;
-      compare_elements(s, e1, e2, cp, &dist);
-      int nf = nearfield_degree(op->kind, s->P, dist, s->M);
-      nf = nf >= ff ? nf : ff;
-      BMI_REQUIRE(nf < 50, BMI_UNSUPPORTED, "near-field quadrature degree too large");
-      p.cls = (cp[2] == 0) ? (nf == ff ? 0 : 1) : cp[2];
-      p.rot1 = cp[0];
-      p.rot2 = cp[1];
-      p.deg = nf;
-      p.off = static_cast<int64_t>(e2 * s->I2) * N + e1 * s->I2;
-      v.push_back(p);
+  // The super matrix of a single layer is symmetric (as for the H2 leaves): the pairs e1 <= e2 are
+  // integrated and the other half is copied; the test operator's is not.  384 elements, P = 1: 6.2 ms with
+  // every pair and T^T A T on the host, 1.7 ms so.
+  const bool sym = op->kind != BMI_DUMMY;
+  const int64_t ne = s->nel, np = sym ? ne * (ne + 1) / 2 : ne * ne;
+  std::vector<NFPair> v(np);
+  // element e2's pairs e1 = 0 .. (e2 or the last); item a stands for e2 = a and, from the other end,
+  // e2 = ne - 1 - a, so that the ranges of the triangle weigh the same
+  parallel_ranges((ne + 1) / 2, 1 + 4096 / ne, [&](int, int64_t a, int64_t b) {
+    for (int64_t k = 2 * a; k < 2 * b; ++k) {
+      const int64_t e2 = k & 1 ? ne - 1 - k / 2 : k / 2;
+      if ((k & 1) && e2 == k / 2) continue;
+      int64_t slot = sym ? e2 * (e2 + 1) / 2 : e2 * ne;
+      for (int64_t e1 = 0; e1 < (sym ? e2 + 1 : ne); ++e1)
+        v[slot++] = classify_pair(s, op->kind, ff, static_cast<int>(e1), static_cast<int>(e2), e2 * s->I2 * N + e1 * s->I2);
     }
+  });
   DevBuf<double> A;
   A.alloc(static_cast<size_t>(S) * N * N);
   // super-space rows and columns are component-major: component c starts at c * nel * I2
   const int64_t vcs = static_cast<int64_t>(s->nel) * s->I2;
   launch_nearfield(s, *op, v, A.ptr, 1, N, vcs, vcs * N, st);
+  if (sym) launch_mirror_dense(cplx, N, vcs, s->I2, A.ptr, st);
+  const hipMemcpyKind to = mem == BMI_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
   if (super_only) {
-    BMI_CHECK_HIP(hipMemcpyAsync(out, A.ptr, A.bytes(), mem == BMI_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st));
-    BMI_CHECK_HIP(hipStreamSynchronize(st));
+    BMI_CHECK_HIP(hipMemcpyAsync(out, A.ptr, A.bytes(), to, st));
   } else {
-    // A T (N x D) then T^T (A T) (D x D), both with the sparse kernels
-    DevBuf<double> AT, ATt, R;
-    ensure_device_space(s, st);
-    // (A T)^T = T^T A^T: compute column j of A T as A * T(:, j) via spmv on A^T rows is awkward;
-    // use the identity T^T A T = (T^T (T^T A^T)^T) with explicit transposes on the host side.
-    std::vector<double> hA(static_cast<size_t>(S) * N * N);
-    BMI_CHECK_HIP(hipMemcpyAsync(hA.data(), A.ptr, A.bytes(), hipMemcpyDeviceToHost, st));
-    BMI_CHECK_HIP(hipStreamSynchronize(st));
-    std::vector<double> hAT(static_cast<size_t>(S) * N * D, 0.0);
-    for (int64_t r = 0; r < N; ++r)
-      for (int k = s->rowptr[r]; k < s->rowptr[r + 1]; ++k) {
-        const int64_t c = s->col[k];
-        const double v0 = s->val[k];
-        const double* src = &hA[S * r * N];
-        double* dst = &hAT[S * c * N];
-        for (int64_t i = 0; i < S * N; ++i) dst[i] += v0 * src[i];
-      }
-    std::vector<double> hR(static_cast<size_t>(S) * D * D, 0.0);
-    for (int64_t j = 0; j < D; ++j)
-      for (int64_t r = 0; r < N; ++r)
-        for (int k = s->rowptr[r]; k < s->rowptr[r + 1]; ++k) {
-          const int64_t row = s->col[k];
-          for (int q = 0; q < S; ++q) hR[S * (j * D + row) + q] += s->val[k] * hAT[S * (j * N + r) + q];
-        }
-    BMI_CHECK_HIP(hipMemcpyAsync(out, hR.data(), hR.size() * sizeof(double),
-                                 mem == BMI_MEM_DEVICE ? hipMemcpyHostToDevice : hipMemcpyHostToHost, st));
+    // C = A T (N x D), then T^T C (D x D)
+    DevBuf<double> C, R;
+    C.alloc(static_cast<size_t>(S) * N * D);
+    R.alloc(static_cast<size_t>(S) * D * D);
+    launch_times_t(cplx, N, D, s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, A.ptr, C.ptr, st);
+    launch_spmv(cplx, static_cast<int>(D), static_cast<int>(D), s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, C.ptr, N,
+                R.ptr, D, nullptr, nullptr, st);
+    BMI_CHECK_HIP(hipMemcpyAsync(out, R.ptr, R.bytes(), to, st));
     BMI_CHECK_HIP(hipStreamSynchronize(st));
   }
+  BMI_CHECK_HIP(hipStreamSynchronize(st));
   BMI_API_END
 }
 

@@ -1,0 +1,48 @@
+"""Dense assembly from half of the element pairs: the copied half and T^T A T, at sizes around the
+32-entry tiles of the copy.
+
+The super matrix of a single layer is symmetric by construction, bit by bit; its blocks are those of the
+pairs (e1 <= e2) integrated alone; and the small matrix is T^T A T, whose entries sum at most m products
+of T's entries: roundoff within m 2^-52 of the sum of magnitudes.
+"""
+import numpy as np
+import pytest
+import scipy.sparse
+
+import bembel_amd as B
+
+pytestmark = pytest.mark.gpu
+
+
+def _operator(kind):
+    op = B.LaplaceSingleLayerOperator() if kind == "laplace" else (
+        B.HelmholtzSingleLayerOperator() if kind == "helmholtz" else B.MaxwellSingleLayerOperator())
+    if kind != "laplace":
+        op.set_wavenumber(2.0 - 0.1j)
+    return op
+
+
+# 6 elements of 4 and 9 functions: 24 and 54 rows; 24 of 4: 96, three whole tiles
+@pytest.mark.parametrize("M,P", [(0, 1), (0, 2), (1, 1)])
+@pytest.mark.parametrize("kind", ["laplace", "helmholtz", "maxwell"])
+def test_gpu_dense_halves_and_projection(gpu, kind, M, P):
+    op = _operator(kind)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), M, P, op)
+    A = np.asarray(B.DenseMatrix(ps, op, super_only=True).matrix)
+    assert np.isfinite(A).all()
+    nel, i2 = 6 * 4 ** M, (P + 1) ** 2
+    vcs = nel * i2
+    e = (np.arange(len(A)) % vcs) // i2
+    off = e[:, None] != e[None, :]
+    assert np.array_equal(A[off], A.T[off])
+    if kind != "maxwell":
+        pairs = [(i, j) for j in range(nel) for i in range(j + 1)]
+        for (i, j), b in zip(pairs, ps.pair_blocks(op, pairs)):
+            got = A[i * i2:(i + 1) * i2, j * i2:(j + 1) * i2]
+            assert np.abs(got - b).max() <= 1e-14 * np.abs(b).max(), (i, j)
+    rp, col, val = ps.get_transformation_matrix()
+    T = scipy.sparse.csr_matrix((val, col, rp), shape=(len(A), ps.number_of_dofs)).toarray()
+    G = np.asarray(B.DenseMatrix(ps, op).matrix)
+    want, mag = T.T @ A @ T, np.abs(T).T @ np.abs(A) @ np.abs(T)
+    m = int((T != 0).sum(0).max())
+    assert (np.abs(G - want) <= 4 * m * 2.0 ** -52 * mag).all()
