@@ -101,49 +101,85 @@ __device__ __forceinline__ void surface_point(const double* __restrict__ cp, dou
   }
 }
 
-// sine and cosine beyond the reach of the reduction below, kept out of line: inlined, its registers (a
-// reduction by a long expansion of 2 / pi) would be those of every kernel
+// 1 / sqrt(s), s > 0: the hardware estimate (v_rsq_f64) refined by two steps of Newton's
+// iteration for 1/sqrt, y <- y + y (1 - s y^2) / 2, each of which squares the relative error
+// (the residual 1 - s y^2 formed with one rounding by an FMA); within a few ulps of the rounded
+// quotient 1 / sqrt(s), for a third of the instructions of a square root and a division
+__device__ __forceinline__ double rsqrt_newton(double s) {
+  double y = __builtin_amdgcn_rsq(s);
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const double e = fma(-(s * y), y, 1.0);
+    y = fma(0.5 * y, e, y);
+  }
+  return y;
+}
+
+// the same for every s >= 0: where the estimate is 0 or infinite (s infinite or 0) it is the result, of
+// which the iteration would make a NaN
+__device__ __forceinline__ double rsqrt_newton_any(double s) {
+  const double y0 = __builtin_amdgcn_rsq(s);
+  return __builtin_amdgcn_class(y0, 0x240) ? y0 : rsqrt_newton(s);  // +infinity, +0
+}
+
+// a b + c with the constant c in scalar registers: from vector registers the compiler copies it first,
+// into the accumulator of the two-operand form
+__device__ __forceinline__ double fma_const(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+
+// sine and cosine of the phases kappa r, |x| < SINCOS_NEAR: reduction to [-pi/4, pi/4] by subtracting
+// n pi/2 in two parts (Cody and Waite, with fused multiply-adds) and the Taylor sums of both, whose first
+// neglected terms are below 1e-18 there.  Absolute error within 3e-16 (checked against extended
+// precision), a third of the library function's instructions.
+constexpr double SINCOS_NEAR = 1048576.0;
+__device__ __forceinline__ void sincos_near(double x, double* s, double* c) {
+  // n = 2 x / pi rounded: adding 3 2^51 leaves the integer in the low bits
+  const double t = fma(x, 0.63661977236758134308, 6755399441055744.0);
+  const double n = t - 6755399441055744.0;
+  double y = fma(-n, 1.57079632679489655800, x);  // pi / 2 rounded, and the rest
+  y = fma(-n, 6.12323399573676603587e-17, y);
+  const double z = y * y;
+  double p = 1.0 / 355687428096000.0;  // 1 / 17!
+  p = fma_const(p, z, -1.0 / 1307674368000.0);
+  p = fma_const(p, z, 1.0 / 6227020800.0);
+  p = fma_const(p, z, -1.0 / 39916800.0);
+  p = fma_const(p, z, 1.0 / 362880.0);
+  p = fma_const(p, z, -1.0 / 5040.0);
+  p = fma_const(p, z, 1.0 / 120.0);
+  p = fma_const(p, z, -1.0 / 6.0);
+  const double sn = fma(y * z, p, y);
+  double q = 1.0 / 20922789888000.0;  // 1 / 16!
+  q = fma_const(q, z, -1.0 / 87178291200.0);
+  q = fma_const(q, z, 1.0 / 479001600.0);
+  q = fma_const(q, z, -1.0 / 3628800.0);
+  q = fma_const(q, z, 1.0 / 40320.0);
+  q = fma_const(q, z, -1.0 / 720.0);
+  q = fma_const(q, z, 1.0 / 24.0);
+  const double cs = fma(z * z, q, fma(-0.5, z, 1.0));
+  const unsigned k = static_cast<unsigned>(__double2loint(t));  // quadrant k mod 4
+  const double a = (k & 1) ? cs : sn, b = (k & 1) ? sn : cs;
+  const unsigned sa = (k << 30) & 0x80000000u, sb = ((k + 1) << 30) & 0x80000000u;  // their signs
+  *s = __hiloint2double(__double2hiint(a) ^ sa, __double2loint(a));
+  *c = __hiloint2double(__double2hiint(b) ^ sb, __double2loint(b));
+}
+
+// the same for any x.  Beyond the reach of the reduction the library's function is kept out of line:
+// inlined, its registers (a reduction by a long expansion of 2 / pi) would be those of every kernel
 static __device__ __noinline__ double2 sincos_far(double x) {
   double s, c;
   sincos(x, &s, &c);
   return make_double2(s, c);
 }
-
-// sine and cosine of the phases kappa r: reduction to [-pi/4, pi/4] by subtracting n pi/2 in two parts
-// (Cody and Waite, with fused multiply-adds) and the Taylor sums of both, whose first neglected terms
-// are below 1e-18 there.  Absolute error within 3e-16 for |x| < 2^20 (checked against extended
-// precision), a third of the library function's instructions.
 __device__ __forceinline__ void sincos_phase(double x, double* s, double* c) {
-  if (!(fabs(x) < 1048576.0)) {
+  if (!(fabs(x) < SINCOS_NEAR)) {
     const double2 v = sincos_far(x);
     *s = v.x, *c = v.y;
     return;
   }
-  const double n = rint(x * 0.63661977236758134308);  // 2 / pi
-  double y = fma(-n, 1.57079632679489655800, x);      // pi / 2 rounded, and the rest
-  y = fma(-n, 6.12323399573676603587e-17, y);
-  const double z = y * y;
-  double p = 1.0 / 355687428096000.0;  // 1 / 17!
-  p = fma(p, z, -1.0 / 1307674368000.0);
-  p = fma(p, z, 1.0 / 6227020800.0);
-  p = fma(p, z, -1.0 / 39916800.0);
-  p = fma(p, z, 1.0 / 362880.0);
-  p = fma(p, z, -1.0 / 5040.0);
-  p = fma(p, z, 1.0 / 120.0);
-  p = fma(p, z, -1.0 / 6.0);
-  const double sn = fma(y * z, p, y);
-  double q = 1.0 / 20922789888000.0;  // 1 / 16!
-  q = fma(q, z, -1.0 / 87178291200.0);
-  q = fma(q, z, 1.0 / 479001600.0);
-  q = fma(q, z, -1.0 / 3628800.0);
-  q = fma(q, z, 1.0 / 40320.0);
-  q = fma(q, z, -1.0 / 720.0);
-  q = fma(q, z, 1.0 / 24.0);
-  const double cs = fma(z * z, q, fma(-0.5, z, 1.0));
-  const int k = static_cast<int>(n) & 3;  // quadrant
-  const double a = (k & 1) ? cs : sn, b = (k & 1) ? sn : cs;
-  *s = (k & 2) ? -a : a;
-  *c = (k == 1 || k == 2) ? -b : b;
+  sincos_near(x, s, c);
 }
 
 }  // namespace bmi

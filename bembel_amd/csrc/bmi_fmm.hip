@@ -107,8 +107,8 @@ __global__ void k_coupling_assemble(const int4* __restrict__ leaves, int nleaves
     out[base + static_cast<int64_t>(j) * cd + i] = (0.25 * M_1_PI) / r * a[3] * b[3];
   } else {
     double sn, cs;
-    sincos(kre * r, &sn, &cs);
-    const double mag = exp(kim * r) * (0.25 * M_1_PI) / r;
+    sincos_phase(kre * r, &sn, &cs);
+    const double mag = (kim == 0.0 ? 1.0 : exp(kim * r)) * (0.25 * M_1_PI) / r;
     const double kr = mag * cs, ki = -mag * sn;
     if constexpr (KIND == BMI_HELMHOLTZ_SL) {
       const int64_t idx = base + static_cast<int64_t>(j) * cd + i;

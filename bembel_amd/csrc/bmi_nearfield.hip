@@ -45,20 +45,6 @@ struct NFParams {
 
 // far-field table record: x0 x1 x2 kappa w s0 s1 pad [ds0 ds1 ds2 dt0 dt1 dt2 pad pad]
 
-// 1 / sqrt(s), s > 0: the hardware estimate (v_rsq_f64) refined by two steps of Newton's
-// iteration for 1/sqrt, y <- y + y (1 - s y^2) / 2, each of which squares the relative error
-// (the residual 1 - s y^2 formed with one rounding by an FMA); within a few ulps of the rounded
-// quotient 1 / sqrt(s), for a third of the instructions of a square root and a division
-__device__ __forceinline__ double rsqrt_newton(double s) {
-  double y = __builtin_amdgcn_rsq(s);
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const double e = fma(-(s * y), y, 1.0);
-    y = fma(0.5 * y, e, y);
-  }
-  return y;
-}
-
 // 1 / x, x != 0: the hardware estimate (v_rcp_f64) refined by two steps of Newton's iteration
 // for the reciprocal, y <- y + y (1 - x y) (residual by an FMA); within an ulp or two of the
 // rounded quotient, for half the instructions of a division
