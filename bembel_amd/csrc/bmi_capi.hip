@@ -393,8 +393,9 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
     // the backward transformation of both components
     launch_mx_prep(h->lvl_total / rows, nrhs, h->np2, rows, w.fw[0], w.fw[1], h->d_mx_tan.ptr, w.z, st);
     launch_mx_coupling(co.fp32, h->ntgt_all, nrhs, h->np2, rows, h->d_mx_order.ptr, h->d_tgt_all.ptr,
-                       h->d_crp_all.ptr, h->d_csrc.ptr,
-                       co.F, h->d_lvl_off.ptr, h->d_mx_tan.ptr, w.z, w.fw[0], w.fw[1], h->mx_qre, h->mx_qim, st);
+                       h->d_crp_all.ptr, h->d_csrc.ptr, co.F, h->d_lvl_off.ptr, w.z, w.fw[0], w.fw[1], st);
+    launch_mx_finish(h->lvl_total / rows, nrhs, h->np2, rows, h->d_mx_tan.ptr, w.fw[0], w.fw[1], h->mx_qre, h->mx_qim,
+                     st);
     apply_tree(h, false, nrhs, nullptr, w.fw[0], w.fw[1], yf, st);
     return;
   }
@@ -1143,7 +1144,7 @@ static void assemble_h2(bmi_h2* h, hipStream_t st) {
   for (int l = 0; l <= h->L; ++l) h->lvl_off[l + 1] = h->lvl_off[l] + static_cast<int64_t>(ncl_at(s, l)) * h->cd;
   h->lvl_total = h->lvl_off[h->L + 1];
   h->d_lvl_off.upload(h->lvl_off, st);
-  // ---- coupling blocks (Maxwell: the kernel values of each leaf, see k_mx_coupling)
+  // ---- coupling blocks (Maxwell: the kernel values of each leaf, see k_mx_prep)
   h->mxf = op.kind == BMI_MAXWELL_SL;
   if (h->mxf) {
     const double k2re = op.kappa_re * op.kappa_re - op.kappa_im * op.kappa_im, k2im = 2 * op.kappa_re * op.kappa_im;

@@ -31,6 +31,10 @@ struct RowsArgs {
   int64_t yseg, ycs, yks, yrs;
   int accumulate;
   int slabs, ncw;  // set by the launch: row slabs, column groups per workgroup
+  int xl = 0, yl = 0;            // factors of the level offsets of x and y (0: nrhs)
+  const int* order = nullptr;    // the order in which targets are taken (null: as listed)
+  double* y1 = nullptr;          // columns from ysplit on go to y1, counted from there
+  int ysplit = 0;
 };
 void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st);
 
@@ -79,13 +83,16 @@ bool launch_multi_cpl_t(bool cplx, bool fp32, int ntgt, int nrhs, int cd, int ld
 int fp32_coupling_ld(bool cplx, int cd);
 void convert_blocks_to_fp32(const double* src, float* dst, int64_t nb, int cd, int ld, bool cplx, hipStream_t st);
 // Maxwell far field from the kernel values of each coupling leaf: the four columns (tangent-
-// weighted value moments, summed derivative moments) of every cluster entry, then one sweep
-// that writes both components' local expansions of every cluster entry
+// weighted value moments, summed derivative moments) of every cluster entry; one sweep over the
+// kernel values, whose four columns of sums take the place of the moments; and both components'
+// local expansions from these, in place
 void launch_mx_prep(int64_t ne, int nrhs, int np2, int cd, const double* fw0, const double* fw1, const double* tan,
                     double* Z, hipStream_t st);
 void launch_mx_coupling(bool fp32, int ntgt_all, int nrhs, int np2, int cd, const int* order, const int2* tgt_all,
-                        const int* rp_all, const int* src, const void* K, const int64_t* lvl_off, const double* tan, const double* Z,
-                        double* bw0, double* bw1, double qre, double qim, hipStream_t st);
+                        const int* rp_all, const int* src, const void* K, const int64_t* lvl_off, const double* Z,
+                        double* w0, double* w1, hipStream_t st);
+void launch_mx_finish(int64_t ne, int nrhs, int np2, int cd, const double* tan, double* w0, double* w1, double qre,
+                      double qim, hipStream_t st);
 void convert_to_bf16(const double* src, unsigned short* dst, int64_t n, hipStream_t st);
 // tree transformations of column-major products (bmi_tree.hip).  upward: moments of x at level L and
 // transfers up to level 0 into the multipole arrays v0, v1 (vd components of nc np^2 rows; clear: the

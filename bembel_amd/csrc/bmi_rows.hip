@@ -59,13 +59,13 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
   const int k0 = (static_cast<int>(blockIdx.y) * ncw + cw) * (NT * CT);
   const int rc = static_cast<int>(blockIdx.z) / a.slabs;
   const int row0 = (static_cast<int>(blockIdx.z) - rc * a.slabs) * (16 * MT);
-  const int own = static_cast<int>(blockIdx.x);
-  int64_t lo = 0;
+  const int own = a.order ? a.order[blockIdx.x] : static_cast<int>(blockIdx.x);
+  int64_t lo = 0, ylo = 0;  // level offsets
   int cl = own;
   if (a.tgt) {
     const int2 T = a.tgt[own];
     cl = T.y;
-    lo = a.lvl_off[T.x] * a.nrhs;
+    lo = a.lvl_off[T.x] * a.xl, ylo = a.lvl_off[T.x] * a.yl;
   }
   // first row of this lane in every row group, moved back where its load would pass the last row
   int rb[MT / RV];
@@ -190,8 +190,10 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
           vr += t[0];
         }
       }
-      double* y = a.y + S * (lo + rc * a.yseg + static_cast<int64_t>(cl) * a.ycs + static_cast<int64_t>(j) * a.yks +
-                             static_cast<int64_t>(row) * a.yrs);
+      const bool second = a.y1 && j >= a.ysplit;
+      double* y = (second ? a.y1 : a.y) + S * (ylo + rc * a.yseg + static_cast<int64_t>(cl) * a.ycs +
+                                               static_cast<int64_t>(second ? j - a.ysplit : j) * a.yks +
+                                               static_cast<int64_t>(row) * a.yrs);
       if (a.accumulate) {
         vr += y[0];
         if constexpr (C) vi += y[1];
@@ -213,6 +215,8 @@ void launch_rows(const RowsArgs& a, dim3 grid, int nw, hipStream_t st) {
 
 void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st) {
   if (a.nown <= 0 || a.nrhs <= 0) return;
+  if (a.xl == 0) a.xl = a.nrhs;
+  if (a.yl == 0) a.yl = a.nrhs;
   const int tiles = (a.n + 15) / 16;
   const int ct = cplx ? 8 : 16;
   const int nt = a.nrhs > ct ? 2 : 1;

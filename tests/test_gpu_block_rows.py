@@ -68,3 +68,18 @@ def test_gpu_block_rows_fp32_blocks(gpu, op):
     # FP32 copies of the coupling blocks, columns padded to whole vectors: 1e-8 from the FP64 operator
     H, oh, n, scalar = _pair(op, 3, 1, 9, precision=B.MIXED)
     _check(H, oh, n, scalar, (1, 3, 20), tol=1e-6)
+
+
+@pytest.mark.parametrize("precision", [B.FP64, B.MIXED])
+@pytest.mark.parametrize("n_cheb", [2, 5, 9])
+def test_gpu_block_rows_maxwell_columns(gpu, n_cheb, precision):
+    # four columns of kernel sums per right-hand side, in two halves: the columns of a product are
+    # those of single products (the same sums over the same blocks), against the oracle in test_gpu_maxwell
+    op = B.MaxwellSingleLayerOperator()
+    op.set_wavenumber(2.0 - 0.1j)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), 3, 1, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb, precision=precision)
+    X = _columns(ps.number_of_dofs, 5, op.scalar, 7)
+    one = np.stack([H @ X[:, k] for k in range(5)], 1)
+    for c in (2, 3, 5):
+        assert np.linalg.norm(H @ X[:, :c] - one[:, :c]) <= 1e-13 * np.linalg.norm(one[:, :c]), c
