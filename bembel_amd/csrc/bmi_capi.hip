@@ -249,6 +249,10 @@ struct bmi_h2 {
   DevBuf<int> d_srp, d_ssrc, d_sblk, d_sgrp, d_sgslot;
   DevBuf<double> d_part;
   bmi::SymList sl{};
+  // without fused upper sweeps: the same lists for block-row sweeps of a few columns (0: none), over
+  // every cluster; part then grows with the workspace
+  int64_t npairs_far = 0;
+  int ngather_far = 0;
   // workspace (grown on demand)
   int ws_rhs = 0;
   DevBuf<double> d_xs, d_ys, d_fw[2], d_bw, d_xin, d_yout;
@@ -322,6 +326,17 @@ static CouplingOperand coupling_operand(const bmi_h2* h, bool reduced) {
   return {false, h->d_coup.ptr, nullptr, 0, h->cd, static_cast<int64_t>(h->cd) * h->cd};
 }
 
+// Far field from one block of every pair: columns of one tile (the partial sums of one more would cost a
+// second pass over the blocks).  Rows of a block from which it pays: see PAIR_MIN_ROWS.
+static bool pair_columns(const bmi_h2* h, int nrhs) {
+  return h->npairs_far > 0 && (h->mxf ? 4 : 1) * nrhs <= block_rows_tile(h->cplx);
+}
+// scalars of partial sums per pair
+static int64_t pair_partial(const bmi_h2* h, int nrhs) {
+  const int n = h->mxf ? h->np2 : h->cd, cols = (h->mxf ? 4 : 1) * nrhs;
+  return static_cast<int64_t>(block_rows_slabs(h->cplx, n, h->ntgt_all)) * cols * n;
+}
+
 static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
   (void)st;
   if (nrhs <= h->ws_rhs) return;
@@ -334,6 +349,11 @@ static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
   h->d_bw.alloc(S * h->lvl_total * nrhs);
   h->d_yf.alloc(S * N * nrhs);
   if (h->mxf) h->d_mxz.alloc(2 * S * h->lvl_total * nrhs);  // 4 np2 columns per entry = 2 cd
+  if (h->npairs_far > 0) {
+    // for as many of the columns as one tile takes (a later product of fewer columns uses them)
+    const int most = block_rows_tile(h->cplx) / (h->mxf ? 4 : 1);
+    h->d_part.alloc(S * h->npairs_far * pair_partial(h, std::min(nrhs, most)));
+  }
   h->ws_rhs = nrhs;
 }
 
@@ -387,13 +407,19 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
   const int rows = h->cd;
   const CouplingOperand co = coupling_operand(h, reduced);
   apply_tree(h, true, nrhs, xs, w.fw[0], w.fw[1], nullptr, st);
+  PairSweep pairs{};
+  const bool use_pairs = w.own && h->sweep_mode != 0 && pair_columns(h, nrhs) && !co.Fc;
+  if (use_pairs)
+    pairs = PairSweep{h->d_srp.ptr, h->d_ssrc.ptr, h->d_sblk.ptr, h->d_sgslot.ptr, h->d_part.ptr, h->ngather_far,
+                      h->d_sgtgt.ptr, h->d_sgrp.ptr};
+  const PairSweep* ps = use_pairs ? &pairs : nullptr;
   if (h->mxf) {
     // four columns per cluster entry from both components' moments, one sweep over the kernel
     // values writing both components' local expansions (into the moment buffers, consumed), then
     // the backward transformation of both components
     launch_mx_prep(h->lvl_total / rows, nrhs, h->np2, rows, w.fw[0], w.fw[1], h->d_mx_tan.ptr, w.z, st);
     launch_mx_coupling(co.fp32, h->ntgt_all, nrhs, h->np2, rows, h->d_mx_order.ptr, h->d_tgt_all.ptr,
-                       h->d_crp_all.ptr, h->d_csrc.ptr, co.F, h->d_lvl_off.ptr, w.z, w.fw[0], w.fw[1], st);
+                       h->d_crp_all.ptr, h->d_csrc.ptr, co.F, h->d_lvl_off.ptr, w.z, w.fw[0], w.fw[1], ps, st);
     launch_mx_finish(h->lvl_total / rows, nrhs, h->np2, rows, h->d_mx_tan.ptr, w.fw[0], w.fw[1], h->mx_qre, h->mx_qim,
                      st);
     apply_tree(h, false, nrhs, nullptr, w.fw[0], w.fw[1], yf, st);
@@ -402,7 +428,7 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
   // every cluster of every level is a target (zero where there are no blocks)
   launch_coupling_apply(C, co.fp32, std::max(h->cpl_variant, 0), h->ntgt_all, nrhs, rows, h->d_tgt_all.ptr,
                         h->d_crp_all.ptr, h->d_csrc.ptr, co.F, co.blk, 0, h->d_lvl_off.ptr, w.fw[0], w.bw, 0, st,
-                        co.Fc, co.ncoarse, co.ld);
+                        co.Fc, co.ncoarse, co.ld, ps);
   apply_tree(h, false, nrhs, nullptr, w.bw, nullptr, yf, st);
 }
 
@@ -886,114 +912,124 @@ static NFPair classify_pair(const bmi_space* s, int kind, int ff, int e1, int e2
   return p;
 }
 
-// Coupling blocks of a symmetric kernel pair up: (level, c2, c1) is the transpose of (level, c1,
-// c2) (same kernel values; the two weights multiply in the other order). For single-RHS sweeps
-// list one block per pair under its smaller cluster c1 (the upper block (c1, c2) for real
-// kernels, the lower block (c2, c1) for complex ones), and per cluster c2 the entries whose
-// partials it receives. Leaves the handle unchanged when a block has no partner.
-static void build_symmetric_lists(bmi_h2* h, const std::vector<int2>& tgt, const std::vector<int>& crp,
-                                  const std::vector<int>& csrc, hipStream_t st) {
-  const int nt = static_cast<int>(tgt.size());
-  auto find_target = [&](int level, int c) {
-    const auto it = std::lower_bound(tgt.begin(), tgt.end(), make_int2(level, c), [](const int2& a, const int2& b) {
-      return a.x != b.x ? a.x < b.x : a.y < b.y;
-    });
-    return (it != tgt.end() && it->x == level && it->y == c) ? static_cast<int>(it - tgt.begin()) : -1;
-  };
-  std::vector<int2> utgt;
-  std::vector<int> urp(1, 0), usrc, ublk;
-  std::vector<int2> ucol;  // (target index of the column cluster, upper entry)
-  for (int t = 0; t < nt; ++t) {
-    const int level = tgt[t].x, c1 = tgt[t].y;
-    bool any = false;
-    for (int p = crp[t]; p < crp[t + 1]; ++p) {
-      const int c2 = csrc[p];
-      const int t2 = find_target(level, c2);
-      if (c2 == c1 || t2 < 0 || !std::binary_search(csrc.begin() + crp[t2], csrc.begin() + crp[t2 + 1], c1)) return;
-      if (c2 < c1) continue;
-      if (!any) utgt.push_back(tgt[t]), urp.push_back(urp.back()), any = true;
-      ucol.push_back(make_int2(t2, static_cast<int>(usrc.size())));
-      usrc.push_back(c2);
-      // complex kernels: the lower block (c2, c1), whose row products are the partials and whose
-      // column products sum into the rows of c1
-      ublk.push_back(h->cplx ? static_cast<int>(std::lower_bound(csrc.begin() + crp[t2], csrc.begin() + crp[t2 + 1], c1) -
-                                                csrc.begin())
-                             : p);
-      urp.back()++;
+// The blocks of a symmetric kernel pair up: block (s, t) is the transpose of (t, s) (same kernel values; the
+// two weights multiply in the other order).  One block of each pair is listed, under its row, and per
+// row the pairs listed under the other one, whose transposed products are due to it, with their partial
+// sums in (row, entry) order.  Rows are (level, cluster) with the sources of a row ascending in src; a row
+// r of cluster c belongs to a level whose rows start at r - c.
+struct PairRows {
+  std::vector<int> rp{0}, src, blk, slot;  // of every row; slot -1: a block that is its own transpose
+  std::vector<int2> gtgt;                  // rows receiving partial sums and the ranges of their slots
+  std::vector<int> grp{0};
+  int64_t nslots = 0;
+};
+enum class PairOrder {
+  upper,  // under the smaller row, block (s, t), s < t
+  lower,  // under the smaller row, block (t, s)
+  even,   // under either row by the parity of s + t, so that all rows have about the same number
+};
+// false if a block has no partner (or, without diag, is its own)
+static bool pair_rows(const std::vector<int2>& rows, const std::vector<int>& rp, const std::vector<int>& src,
+                      PairOrder order, bool diag, PairRows& out) {
+  const int n = static_cast<int>(rows.size());
+  // the partner of every block: rows are taken in ascending order, so the entries below the diagonal of a
+  // row are met in their own order
+  std::vector<int> next(rp.begin(), rp.end() - 1), mate(src.size());
+  for (int r = 0; r < n; ++r) {
+    const int c = rows[r].y;
+    if (next[r] < rp[r + 1] && src[next[r]] < c) return false;
+    for (int p = next[r]; p < rp[r + 1]; ++p) {
+      const int r2 = r - c + src[p];
+      int q = p;
+      if (r2 == r) {
+        if (!diag) return false;
+      } else {
+        if (r2 >= n || rows[r2].x != rows[r].x) return false;
+        q = next[r2]++;
+        if (q >= rp[r2 + 1] || src[q] != c) return false;
+      }
+      mate[p] = q, mate[q] = p;
     }
   }
-  // gather order: column targets in (level, cluster) order, entries in list order; each entry's
-  // partial is stored at its position in this order
-  std::stable_sort(ucol.begin(), ucol.end(), [](const int2& a, const int2& b) { return a.x < b.x; });
-  std::vector<int2> gtgt;
-  std::vector<int> grp(1, 0), gslot(usrc.size());
-  for (size_t q = 0; q < ucol.size(); ++q) {
-    const int2& e = ucol[q];
-    if (gtgt.empty() || gtgt.back().x != tgt[e.x].x || gtgt.back().y != tgt[e.x].y) {
-      gtgt.push_back(tgt[e.x]);
-      grp.push_back(grp.back());
-    }
-    grp.back()++;
-    gslot[e.y] = static_cast<int>(q);
+  auto owned = [&](int c, int c2) { return (c <= c2) != (order == PairOrder::even && ((c + c2) & 1)); };
+  std::vector<int> place(src.size());  // of the blocks that are not listed: their row's slots in order
+  for (int r = 0; r < n; ++r) {
+    const int c = rows[r].y;
+    const int64_t before = out.nslots;
+    for (int p = rp[r]; p < rp[r + 1]; ++p)
+      if (mate[p] != p && !owned(c, src[p])) place[p] = static_cast<int>(out.nslots++);
+    if (out.nslots == before) continue;
+    out.gtgt.push_back(rows[r]);
+    out.grp.push_back(static_cast<int>(out.nslots));
   }
-  const int S = h->cplx ? 2 : 1;
-  h->d_stgt.upload(utgt, st);
-  h->d_srp.upload(urp, st);
-  h->d_ssrc.upload(usrc, st);
-  h->d_sblk.upload(ublk, st);
-  h->d_sgtgt.upload(gtgt, st);
-  h->d_sgrp.upload(grp, st);
-  h->d_sgslot.upload(gslot, st);
-  h->d_part.alloc(static_cast<size_t>(S) * usrc.size() * h->cd);
-  h->sl = SymList{static_cast<int>(utgt.size()), h->d_stgt.ptr, h->d_srp.ptr, h->d_ssrc.ptr, h->d_sblk.ptr,
-                  h->d_part.ptr, h->d_sgslot.ptr, static_cast<int>(gtgt.size()), h->d_sgtgt.ptr, h->d_sgrp.ptr};
-  h->sym = true;
+  for (int r = 0; r < n; ++r) {
+    for (int p = rp[r]; p < rp[r + 1]; ++p) {
+      if (mate[p] != p && !owned(rows[r].y, src[p])) continue;
+      out.src.push_back(src[p]);
+      out.blk.push_back(order == PairOrder::lower ? mate[p] : p);
+      out.slot.push_back(mate[p] == p ? -1 : place[mate[p]]);
+    }
+    out.rp.push_back(static_cast<int>(out.src.size()));
+  }
+  return true;
+}
+
+// lists of the fused single-column sweeps (rows with entries only): the upper block (c1, c2) for real
+// kernels, the lower block (c2, c1) for complex ones, whose row products are the partial sums and whose
+// column products add up to the rows of c1.  With pairs, lists of the block-row sweeps of a few columns:
+// every cluster, either block of a pair.
+static void build_symmetric_lists(bmi_h2* h, const std::vector<int2>& all, const std::vector<int>& rp_all,
+                                  const std::vector<int>& csrc, bool pairs, hipStream_t st) {
+  PairRows pr;
+  if (pairs && csrc.size() < 2 * static_cast<size_t>(PAIR_MIN_COUNT)) return;
+  const PairOrder order = pairs ? PairOrder::even : h->cplx ? PairOrder::lower : PairOrder::upper;
+  if (!pair_rows(all, rp_all, csrc, order, false, pr) || pr.nslots == 0) return;
+  h->d_ssrc.upload(pr.src, st);
+  h->d_sblk.upload(pr.blk, st);
+  h->d_sgtgt.upload(pr.gtgt, st);
+  h->d_sgrp.upload(pr.grp, st);
+  h->d_sgslot.upload(pr.slot, st);
+  if (pairs) {
+    h->d_srp.upload(pr.rp, st);
+    h->npairs_far = pr.nslots;
+    h->ngather_far = static_cast<int>(pr.gtgt.size());
+  } else {
+    std::vector<int2> utgt;
+    std::vector<int> urp(1, 0);
+    for (size_t r = 0; r < all.size(); ++r)
+      if (pr.rp[r + 1] > pr.rp[r]) utgt.push_back(all[r]), urp.push_back(pr.rp[r + 1]);
+    h->d_stgt.upload(utgt, st);
+    h->d_srp.upload(urp, st);
+    h->d_part.alloc(static_cast<size_t>(h->cplx ? 2 : 1) * pr.src.size() * h->cd);
+    h->sl = SymList{static_cast<int>(utgt.size()), h->d_stgt.ptr, h->d_srp.ptr, h->d_ssrc.ptr, h->d_sblk.ptr,
+                    h->d_part.ptr, h->d_sgslot.ptr, static_cast<int>(pr.gtgt.size()), h->d_sgtgt.ptr, h->d_sgrp.ptr};
+    h->sym = true;
+  }
   BMI_CHECK_HIP(hipStreamSynchronize(st));
 }
 
-// Near-field leaves of a symmetric kernel pair up as well: leaf (c2, c1) is the transpose of
-// (c1, c2) (the assembly copies it so).  For single-RHS sweeps list, per row cluster, its
-// diagonal leaf and the leaves (c, c2) with c2 > c; each of the latter also gives the transposed
-// product for the rows of c2, gathered per column cluster in list order.  Leaves the handle
-// unchanged when a leaf has no partner.
+// Near-field leaves of a symmetric kernel pair up as well (the assembly copies leaf (c2, c1) from
+// (c1, c2)): per row cluster its diagonal leaf and the leaves (c, c2) with c2 > c, each of which also
+// gives the transposed product for the rows of c2.
 static void build_near_symmetric_lists(bmi_h2* h, const std::vector<int>& drp, const std::vector<int>& dsrc,
                                        hipStream_t st) {
   const int ncl = h->ncl_leaf;
-  std::vector<int2> tg(ncl), col;  // col: (column cluster, entry)
-  std::vector<int> rp(1, 0), src, blk, slot;
-  for (int c = 0; c < ncl; ++c) {
-    tg[c] = make_int2(0, c);
-    for (int p = drp[c]; p < drp[c + 1]; ++p) {
-      const int c2 = dsrc[p];
-      if (c2 < c) continue;
-      if (c2 > c && !std::binary_search(dsrc.begin() + drp[c2], dsrc.begin() + drp[c2 + 1], c)) return;
-      if (c2 > c) col.push_back(make_int2(c2, static_cast<int>(src.size())));
-      src.push_back(c2);
-      blk.push_back(p);
-      slot.push_back(-1);
-    }
-    rp.push_back(static_cast<int>(src.size()));
-  }
-  std::stable_sort(col.begin(), col.end(), [](const int2& a, const int2& b) { return a.x < b.x; });
-  std::vector<int2> gtgt;
-  std::vector<int> grp(1, 0);
-  for (size_t q = 0; q < col.size(); ++q) {
-    if (gtgt.empty() || gtgt.back().y != col[q].x) gtgt.push_back(make_int2(0, col[q].x)), grp.push_back(grp.back());
-    grp.back()++;
-    slot[col[q].y] = static_cast<int>(q);
-  }
+  std::vector<int2> tg(ncl);
+  for (int c = 0; c < ncl; ++c) tg[c] = make_int2(0, c);
+  PairRows pr;
+  if (!pair_rows(tg, drp, dsrc, PairOrder::upper, true, pr)) return;
   const int S = h->cplx ? 2 : 1;
   h->d_ntgt.upload(tg, st);
-  h->d_nrp.upload(rp, st);
-  h->d_nsrc.upload(src, st);
-  h->d_nblk.upload(blk, st);
-  h->d_nslot.upload(slot, st);
-  h->d_ngtgt.upload(gtgt, st);
-  h->d_ngrp.upload(grp, st);
+  h->d_nrp.upload(pr.rp, st);
+  h->d_nsrc.upload(pr.src, st);
+  h->d_nblk.upload(pr.blk, st);
+  h->d_nslot.upload(pr.slot, st);
+  h->d_ngtgt.upload(pr.gtgt, st);
+  h->d_ngrp.upload(pr.grp, st);
   h->d_zero.upload(std::vector<int64_t>(1, 0), st);
-  h->d_npart.alloc(static_cast<size_t>(S) * std::max<size_t>(col.size(), 1) * h->dd);
+  h->d_npart.alloc(static_cast<size_t>(S) * std::max<int64_t>(pr.nslots, 1) * h->dd);
   h->nsl = SymList{ncl, h->d_ntgt.ptr, h->d_nrp.ptr, h->d_nsrc.ptr, h->d_nblk.ptr, h->d_npart.ptr, h->d_nslot.ptr,
-                   static_cast<int>(gtgt.size()), h->d_ngtgt.ptr, h->d_ngrp.ptr, h->d_zero.ptr};
+                   static_cast<int>(pr.gtgt.size()), h->d_ngtgt.ptr, h->d_ngrp.ptr, h->d_zero.ptr};
   h->nsym = true;
   BMI_CHECK_HIP(hipStreamSynchronize(st));
 }
@@ -1246,9 +1282,11 @@ static void assemble_h2(bmi_h2* h, hipStream_t st) {
                        [&](int a, int b) { return rp_all[a + 1] - rp_all[a] > rp_all[b + 1] - rp_all[b]; });
       h->d_mx_order.upload(order, st);
     }
+    if (vd == 1 && (op.kind == BMI_LAPLACE_SL || op.kind == BMI_HELMHOLTZ_SL) && sym_sweep_supported(h->cplx, h->dd, h->cd))
+      build_symmetric_lists(h, all, rp_all, csrc, false, st);
+    else if (op.kind != BMI_DUMMY && (h->mxf || vd == 1) && (h->mxf ? h->np2 : h->cd) >= PAIR_MIN_ROWS)
+      build_symmetric_lists(h, all, rp_all, csrc, true, st);
   }
-  if (vd == 1 && (op.kind == BMI_LAPLACE_SL || op.kind == BMI_HELMHOLTZ_SL) && sym_sweep_supported(h->cplx, h->dd, h->cd))
-    build_symmetric_lists(h, tgt, crp, csrc, st);
   // FP32 coupling copy: MIXED pads the columns to whole 16-byte row vectors (the sweeps read rows
   // as vectors); MIXED_BF16 keeps the FP64 layout, shared with its BF16 blocks
   h->ld32 = h->mxf ? h->np2 : op.precision == BMI_PRECISION_MIXED ? fp32_coupling_ld(h->cplx, h->cd) : h->cd;
@@ -1660,6 +1698,12 @@ bmi_status bmi_h2_estimate_bytes(const bmi_space* s, const bmi_op_desc* op, int 
     if (S == 1) b += lvl_total * 16 + lvl_total / cd * 32;            // node tables
   }
   b += (int64_t(dense.size()) + int64_t(lowrank.size())) * 8;                           // CSR indices
+  const int64_t pn = mxf ? np2 : cd, pc = mxf ? 4 : 1;  // lists and partial sums of paired coupling blocks
+  if (op->kind != BMI_DUMMY && (mxf || vd == 1) && pn >= PAIR_MIN_ROWS &&
+      int64_t(lowrank.size()) >= 2 * PAIR_MIN_COUNT)
+    b += int64_t(lowrank.size()) / 2 *
+         (12 + S * 8 * block_rows_slabs(S == 2, static_cast<int>(pn), lvl_total / cd) * pn * pc *
+                   std::min<int64_t>(std::max(nrhs, 1), block_rows_tile(S == 2) / pc));
   if (cd > 0) b += lvl_total / cd * 12;                                                  // all-cluster list
   b += std::max(nrhs, 1) * S * (3 * int64_t(s->nsuper) + (vd + 1) * lvl_total) * 8;   // workspace
   b += int64_t(s->nel) * 25 * 16 * 8 + int64_t(s->val.size()) * 24;                    // tables, T

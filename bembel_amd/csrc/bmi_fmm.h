@@ -35,7 +35,36 @@ struct RowsArgs {
   const int* order = nullptr;    // the order in which targets are taken (null: as listed)
   double* y1 = nullptr;          // columns from ysplit on go to y1, counted from there
   int ysplit = 0;
+  // symmetric pairs (one of the blocks (t, s), (s, t) per entry, vd = 1, columns of one tile): the block
+  // of every entry and the place of F^T x_t, which is due to s, among the partial sums
+  const int* blk = nullptr;
+  const int* slot = nullptr;
+  double* part = nullptr;
 };
+// The lists of a symmetric far field (one block per pair, over every cluster; see RowsArgs) and the targets
+// that receive partial sums.
+struct PairSweep {
+  const int* rp;
+  const int* src;
+  const int* blk;
+  const int* slot;
+  double* part;
+  int ngather;
+  const int2* gtgt;
+  const int* grp;
+};
+// From this many rows of a block and this many pairs on.  Pairs against every block, one column / four:
+// 36 rows, 34,000 pairs (real) 302 / 335 against 318 / 342 us; 49 rows, 7,300 pairs (complex) 245 / 278
+// against 294 / 308; 81 rows, 1,900 pairs (real) 156 / 163 against 165 / 166; with 25 rows four columns gain
+// 3 %, and the partial sums of a few columns come near the size of the blocks.
+constexpr int PAIR_MIN_ROWS = 36;
+constexpr int PAIR_MIN_COUNT = 1024;
+// row slabs of a launch: parts of the rows with partial sums of their own
+int block_rows_slabs(bool cplx, int n, int64_t owners);
+// columns of one tile
+constexpr int block_rows_tile(bool cplx) { return cplx ? 8 : 16; }
+// the sweep of a's targets from their pairs: block rows, then the partial sums
+void launch_pair_rows(bool cplx, bool fp32, RowsArgs a, const PairSweep& ps, hipStream_t st);
 void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st);
 
 void launch_cluster_points(const bmi_space* s, int level, int np, const double* d_cheb, double* out,
@@ -55,7 +84,8 @@ bool wave_coupling_supported(bool cplx, int cd);
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,
                            const int* rp, const int* src, const void* F, int64_t fstride, int64_t fcomp,
                            const int64_t* lvl_off, const double* fw, double* bw, int accumulate, hipStream_t st,
-                           const unsigned short* Fc = nullptr, int ncoarse = 0, int ld = 0);
+                           const unsigned short* Fc = nullptr, int ncoarse = 0, int ld = 0,
+                           const PairSweep* pairs = nullptr);
 // many right-hand sides: internal vectors with the RHS index fastest (see bmi_fmm.hip)
 void launch_spmv_tin(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, const double* v, const double* X,
                      int64_t ldx, double* Yt, hipStream_t st);
@@ -90,7 +120,7 @@ void launch_mx_prep(int64_t ne, int nrhs, int np2, int cd, const double* fw0, co
                     double* Z, hipStream_t st);
 void launch_mx_coupling(bool fp32, int ntgt_all, int nrhs, int np2, int cd, const int* order, const int2* tgt_all,
                         const int* rp_all, const int* src, const void* K, const int64_t* lvl_off, const double* Z,
-                        double* w0, double* w1, hipStream_t st);
+                        double* w0, double* w1, const PairSweep* pairs, hipStream_t st);
 void launch_mx_finish(int64_t ne, int nrhs, int np2, int cd, const double* tan, double* w0, double* w1, double qre,
                       double qim, hipStream_t st);
 void convert_to_bf16(const double* src, unsigned short* dst, int64_t n, hipStream_t st);

@@ -2310,20 +2310,18 @@ bool wave_coupling_supported(bool cplx, int cd) { return cd == 16 || cd == 25 ||
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,
                            const int* rp, const int* src, const void* F, int64_t fstride, int64_t fcomp,
                            const int64_t* lvl_off, const double* fw, double* bw, int accumulate, hipStream_t st,
-                           const unsigned short* Fc, int ncoarse, int ld) {
+                           const unsigned short* Fc, int ncoarse, int ld, const PairSweep* pairs) {
   if (ld <= 0) ld = cd;
   const int64_t n = static_cast<int64_t>(ntgt) * nrhs * cd;
   if (n == 0) return;
   TimedScope ts("coupling_apply", st);
   // several columns, and single columns of block sizes without a wave-per-target kernel (the BF16
   // blocks of the coarsest levels are read by the wave kernels only)
-  auto rows = [&] {
-    launch_block_rows(cplx, fp32,
-                      RowsArgs{ntgt, nrhs, cd, ld, 1, tgt, lvl_off, rp, src, F, fstride, fw, 0,
-                               static_cast<int64_t>(nrhs) * cd, cd, 1, bw, 0, static_cast<int64_t>(nrhs) * cd, cd, 1,
-                               accumulate, 1, 1},
-                      st);
-  };
+  const RowsArgs ra{ntgt, nrhs, cd, ld, 1, tgt, lvl_off, rp, src, F, fstride, fw, 0,
+                    static_cast<int64_t>(nrhs) * cd, cd, 1, bw, 0, static_cast<int64_t>(nrhs) * cd, cd, 1,
+                    accumulate, 1, 1};
+  if (pairs) return launch_pair_rows(cplx, fp32, ra, *pairs, st);
+  auto rows = [&] { launch_block_rows(cplx, fp32, ra, st); };
   if (nrhs > 1 && (!Fc || ncoarse == 0)) return rows();
   const dim3 wgrid(static_cast<unsigned>((ntgt + 3) / 4));
   // wave-per-target kernels for the block sizes of the configurations (np 4, 5)
@@ -2846,7 +2844,7 @@ void launch_mx_prep(int64_t ne, int nrhs, int np2, int cd, const double* fw0, co
 // column): 872 -> 662 us.
 void launch_mx_coupling(bool fp32, int ntgt_all, int nrhs, int np2, int cd, const int* order, const int2* tgt_all,
                         const int* rp_all, const int* src, const void* K, const int64_t* lvl_off, const double* Z,
-                        double* w0, double* w1, hipStream_t st) {
+                        double* w0, double* w1, const PairSweep* pairs, hipStream_t st) {
   if (ntgt_all <= 0 || nrhs <= 0) return;
   if (np2 > 256) throw Error(BMI_UNSUPPORTED, "Maxwell far field with more than 16x16 Chebyshev nodes");
   TimedScope ts("coupling_apply", st);
@@ -2856,7 +2854,10 @@ void launch_mx_coupling(bool fp32, int ntgt_all, int nrhs, int np2, int cd, cons
   a.xl = 2 * nrhs, a.yl = nrhs;
   a.order = order;
   a.y1 = w1, a.ysplit = 2 * nrhs;
-  launch_block_rows(true, fp32, a, st);
+  if (pairs)
+    launch_pair_rows(true, fp32, a, *pairs, st);
+  else
+    launch_block_rows(true, fp32, a, st);
 }
 
 void launch_mx_finish(int64_t ne, int nrhs, int np2, int cd, const double* tan, double* w0, double* w1, double qre,

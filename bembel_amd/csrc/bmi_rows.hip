@@ -16,6 +16,15 @@
 // come from the caches), and their sums are added in wave order through LDS: the same bits on
 // every run.
 //
+// Symmetric kernels (PAIR): the block (s, t) is the transpose of (t, s), so one block of each pair is
+// read for both products, half the bytes.  A chunk's entries are also laid into LDS (a wave's own tiles)
+// and read back with rows and columns exchanged, as the right operand of x_t^T F; the sums over this
+// workgroup's rows are complete per chunk and go to the pair's place among the partial sums of s, which
+// k_pair_gather adds in a fixed order.  Pairs are listed under either row by parity: under the smaller
+// one the first rows have twice the mean and the last none (81 rows, 34,000 pairs: 779 us so, 681 us by
+// parity, 886 us reading every block).  Products on an ellipsoid, 9x9 nodes: Helmholtz, 1,536 elements, five
+// columns 566 -> 478 us; Maxwell, 1,536 elements, P 2 644 -> 519 us; Helmholtz, 6,144 elements, P 2 1.90 -> 1.31 ms.
+//
 // Measured against one thread per row (generic sizes) and one wave per target (16 and 25 rows, two
 // complex columns per pass): Laplace product, 6,144 elements, 9x9 nodes, one column 2160 -> 954 us;
 // Helmholtz product, 1,536 elements, P 1, 9x9 nodes, five columns 2469 -> 735 us; Helmholtz GMRES
@@ -41,7 +50,17 @@ struct Entry {
   __device__ void load(const FT* p) { __builtin_memcpy(v, p, sizeof(v)); }
 };
 
-template <bool C, typename FT, int RV, int MT, int NT>
+// orders a wave's LDS writes before its own reads of them
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+constexpr int PAIR_LD = 18;               // doubles per column of a staged tile: 16 rows, 16-byte reads without conflicts
+constexpr int PAIR_TILE = 16 * PAIR_LD;  // one row tile of one plane
+
+template <bool C, typename FT, int RV, int MT, int NT, bool PAIR>
 __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
   constexpr int S = C ? 2 : 1, PL = C ? 2 : 1;
   constexpr int CT = C ? 8 : 16;  // right-hand sides per column tile
@@ -90,6 +109,23 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int u = 0; u < NT; ++u) acc[p][m][u] = rows_d4{0.0, 0.0, 0.0, 0.0};
+  // PAIR: x of the target as the left operand of x_t^T F, lane = column li (complex: Re | Im) of row
+  // 4 lk + s of every row tile; rows past the block count as zero
+  double x1[PAIR ? MT : 1][4];
+  rows_d4 acc2[PL];
+  double* stage = red + w * (MT * PL * PAIR_TILE);
+  if constexpr (PAIR) {
+    const int j = C ? (li & 7) : li;
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int i = 4 * lk + s;
+        const int row = row0 + (RV == 1 ? 16 * m + i : 16 * RV * (m / RV) + RV * i + m % RV);
+        x1[m][s] = row < n && j < a.nrhs ? a.x[xcol[0] + S * (static_cast<int64_t>(cl) * a.xcs + static_cast<int64_t>(row) * a.xrs)]
+                                         : 0.0;
+      }
+  }
   // the wave's blocks: q = p * vd + (column component)
   const int q1 = a.rp[own + 1] * vd;
   int q = a.rp[own] * vd + bw;
@@ -99,15 +135,15 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
     double x[NT][KU];
   };
   const FT* __restrict__ F = static_cast<const FT*>(a.F);
-  // the sources in the constant address space: scalar loads, which do not take part in the count of the
+  // the lists in the constant address space: scalar loads, which do not take part in the count of the
   // vector loads below
-  typedef const int __attribute__((address_space(4)))* SrcPtr;
-  const SrcPtr src = (SrcPtr)(a.src);
+  typedef const int __attribute__((address_space(4)))* ListPtr;
+  const ListPtr src = (ListPtr)(a.src), blk = (ListPtr)(a.blk), slot = (ListPtr)(a.slot);
   const FT* f = nullptr;  // the block being loaded and the source's values
   const double* xs = nullptr;
   auto take = [&](int q2) {
     const int p = vd == 1 ? q2 : q2 / vd, cc = q2 - p * vd;
-    f = F + S * ((static_cast<int64_t>(p) * vd + rc) * vd + cc) * a.fblk;
+    f = F + S * ((static_cast<int64_t>(PAIR ? blk[p] : p) * vd + rc) * vd + cc) * a.fblk;
     xs = a.x + S * (cc * a.xseg + static_cast<int64_t>(src[p]) * a.xcs);
   };
   auto load = [&](Chunk& c, int kb) {
@@ -134,6 +170,15 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
         const double v0 = in ? static_cast<double>(c.f[g][s].v[0]) : 0.0;
         double v1 = 0.0;
         if constexpr (C || RV == 2) v1 = in ? static_cast<double>(c.f[g][s].v[1]) : 0.0;
+        if constexpr (PAIR) {
+          double* t = stage + (4 * s + lk) * PAIR_LD + li;
+          if constexpr (C || RV == 2) {
+            t[2 * g * PAIR_TILE] = !C && last[g] ? v1 : v0;
+            t[(2 * g + 1) * PAIR_TILE] = v1;
+          } else {
+            t[g * PAIR_TILE] = v0;
+          }
+        }
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
           if constexpr (C) {
@@ -148,6 +193,41 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
       }
     }
   };
+  // PAIR: the chunk's columns of x_t^T F over this slab's rows, complete: lane = column kb + li of
+  // right-hand sides 4 v + lk
+  auto transposed = [&]() {
+    wave_lds_fence();
+#pragma unroll
+    for (int pl = 0; pl < PL; ++pl) acc2[pl] = rows_d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int pl = 0; pl < PL; ++pl) {
+        const double2* t = reinterpret_cast<const double2*>(stage + (m * PL + pl) * PAIR_TILE + li * PAIR_LD + 4 * lk);
+        const double2 t0 = t[0], t1 = t[1];
+        acc2[pl] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1[PAIR ? m : 0][0], t0.x, acc2[pl], 0, 0, 0);
+        acc2[pl] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1[PAIR ? m : 0][1], t0.y, acc2[pl], 0, 0, 0);
+        acc2[pl] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1[PAIR ? m : 0][2], t1.x, acc2[pl], 0, 0, 0);
+        acc2[pl] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1[PAIR ? m : 0][3], t1.y, acc2[pl], 0, 0, 0);
+      }
+    wave_lds_fence();
+  };
+  auto store_partial = [&](int p, int kb) {
+    const int col = kb + li;
+    double* o = a.part + S * ((static_cast<int64_t>(slot[p]) * a.slabs + row0 / (16 * MT)) * a.nrhs * n + col);
+#pragma unroll
+    for (int v = 0; v < (C ? 2 : 4); ++v) {
+      const int j = 4 * v + lk;
+      if (4 * v >= a.nrhs) break;
+      if (col < n && j < a.nrhs) {
+        if constexpr (C)
+          *reinterpret_cast<double2*>(o + static_cast<int64_t>(2) * j * n) =
+              make_double2(acc2[0][v] - acc2[PL - 1][v + 2], acc2[0][v + 2] + acc2[PL - 1][v]);
+        else
+          o[static_cast<int64_t>(j) * n] = acc2[0][v];
+      }
+    }
+  };
   if (q < q1) {
     // Two chunks in turn: the loads of one are in flight while the other is multiplied.  They are issued
     // without a condition (past the last chunk: its columns again, counted as zero), and each chunk is
@@ -157,9 +237,10 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
     constexpr int LOADS = KU * (MT / RV + NT);
     static_assert(LOADS < 64, "loads of a chunk within the counter");
     Chunk c0, c1;
-    int kb = 0;  // first column of the chunk loaded last; n: past the end
+    int kb = 0;              // first column of the chunk loaded last; n: past the end
+    int done = -1, kdone = 0;  // PAIR: the chunk whose transposed product waits to be stored
     auto step = [&](const Chunk& now, Chunk& next) {
-      const int kn = kb;
+      const int kn = kb, qn = q;
       kb += 4 * KU;
       if (kb >= n) {
         kb = n;
@@ -168,7 +249,15 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
       load(next, kb);
       // vmcnt(LOADS), the other counters unbounded
       __builtin_amdgcn_s_waitcnt((LOADS & 15) | ((LOADS >> 4) << 14) | 0x0f70);
+      if constexpr (PAIR) {
+        // stores of the chunk before: behind this wait, which would otherwise wait for them too
+        if (done >= 0) store_partial(done, kdone);
+      }
       multiply(now, kn);
+      if constexpr (PAIR) {
+        if (kn < n) transposed();
+        done = kn < n ? qn : -1, kdone = kn;
+      }
     };
     const int chunks = (q1 - q + nbw - 1) / nbw * ((n + 4 * KU - 1) / (4 * KU));
     take(q);
@@ -176,6 +265,9 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
     for (int t = 0; t < chunks; t += 2) {
       step(c0, c1);
       step(c1, c0);
+    }
+    if constexpr (PAIR) {
+      if (done >= 0) store_partial(done, kdone);
     }
   }
   // sums over the waves of a column group, one row tile at a time: tile entry (row 4 v + lk, column
@@ -226,45 +318,90 @@ __global__ __launch_bounds__(512) void k_block_rows(RowsArgs a) {
   }
 }
 
-template <bool C, typename FT, int RV, int MT, int NT>
+template <bool C, typename FT, int RV, int MT, int NT, bool PAIR>
 void launch_rows(const RowsArgs& a, dim3 grid, int nw, hipStream_t st) {
-  const size_t lds = static_cast<size_t>(nw) * (C ? 2 : 1) * NT * 256 * sizeof(double);
-  hipLaunchKernelGGL((k_block_rows<C, FT, RV, MT, NT>), grid, dim3(static_cast<unsigned>(64 * nw)), lds, st, a);
+  const int planes = C ? 2 : 1;
+  const size_t lds = static_cast<size_t>(nw) * planes * std::max(NT * 256, PAIR ? MT * PAIR_TILE : 0) * sizeof(double);
+  hipLaunchKernelGGL((k_block_rows<C, FT, RV, MT, NT, PAIR>), grid, dim3(static_cast<unsigned>(64 * nw)), lds, st, a);
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+// thread per (target, column, row): the target's partial sums in slot order
+template <bool C>
+__global__ __launch_bounds__(256) void k_pair_gather(RowsArgs a, int ng, const int2* __restrict__ gtgt,
+                                                     const int* __restrict__ grp) {
+  constexpr int S = C ? 2 : 1;
+  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int per = a.nrhs * a.n;
+  if (gid >= static_cast<int64_t>(ng) * per) return;
+  const int g = static_cast<int>(gid / per), e = static_cast<int>(gid - static_cast<int64_t>(g) * per);
+  const int j = e / a.n, row = e - j * a.n;
+  const int64_t q0 = static_cast<int64_t>(grp[g]) * a.slabs, q1 = static_cast<int64_t>(grp[g + 1]) * a.slabs;
+  const double* p = a.part + S * (q0 * per + e);
+  double vr = 0.0, vi = 0.0;
+#pragma unroll 4
+  for (int64_t q = q0; q < q1; ++q, p += S * per) {
+    if constexpr (C) {
+      const double2 t = *reinterpret_cast<const double2*>(p);
+      vr += t.x, vi += t.y;
+    } else {
+      vr += p[0];
+    }
+  }
+  const int2 T = gtgt[g];
+  const bool second = a.y1 && j >= a.ysplit;
+  double* y = (second ? a.y1 : a.y) + S * (a.lvl_off[T.x] * a.yl + static_cast<int64_t>(T.y) * a.ycs +
+                                           static_cast<int64_t>(second ? j - a.ysplit : j) * a.yks +
+                                           static_cast<int64_t>(row) * a.yrs);
+  y[0] += vr;
+  if constexpr (C) y[1] += vi;
+}
+
 }  // namespace
+
+// row tiles per workgroup: at most six real or three complex ones (registers: two waves per SIMD);
+// few targets get workgroups of fewer rows, so that more of the chip takes part
+static int rows_tiles(bool cplx, int n, int64_t owners) {
+  const int tiles = (n + 15) / 16;
+  const int most = cplx ? 3 : 6, unit = cplx || n < 2 ? 1 : 2;
+  int slabs = (tiles + most - 1) / most;
+  while (owners * slabs < 512 && slabs * unit < tiles) ++slabs;
+  const int mt = (tiles + slabs - 1) / slabs;
+  return (mt + unit - 1) / unit * unit;
+}
+int block_rows_slabs(bool cplx, int n, int64_t owners) {
+  const int mt = rows_tiles(cplx, n, owners);
+  return ((n + 15) / 16 + mt - 1) / mt;
+}
 
 void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st) {
   if (a.nown <= 0 || a.nrhs <= 0) return;
   if (a.xl == 0) a.xl = a.nrhs;
   if (a.yl == 0) a.yl = a.nrhs;
-  const int tiles = (a.n + 15) / 16;
-  const int ct = cplx ? 8 : 16;
+  const int ct = block_rows_tile(cplx);
   const int nt = a.nrhs > ct ? 2 : 1;
-  // row tiles per workgroup: at most six real or three complex ones (registers: two waves per SIMD);
-  // few targets get workgroups of fewer rows, so that more of the chip takes part
-  const int rv = cplx || a.n < 2 ? 1 : 2;
-  const int most = cplx ? 3 : 6, unit = rv;
-  int slabs = (tiles + most - 1) / most;
+  const bool pair = a.part != nullptr;
+  BMI_REQUIRE(!pair || (nt == 1 && a.vd == 1 && a.tgt && a.n > 1), BMI_INVALID_ARG, "pairs of blocks: one column tile");
   const int64_t owners = static_cast<int64_t>(a.nown) * a.vd;
-  while (owners * slabs < 512 && slabs * unit < tiles) ++slabs;
-  int mt = (tiles + slabs - 1) / slabs;
-  mt = (mt + unit - 1) / unit * unit;
-  a.slabs = (tiles + mt - 1) / mt;
+  const int rv = cplx || a.n < 2 ? 1 : 2;
+  const int mt = rows_tiles(cplx, a.n, owners);
+  a.slabs = block_rows_slabs(cplx, a.n, owners);
   // column groups of a workgroup share its blocks through the caches; the rest of its waves take
   // blocks in turn
   const int groups = (a.nrhs + nt * ct - 1) / (nt * ct);
   a.ncw = groups >= 4 ? 4 : groups >= 2 ? 2 : 1;
-  const int nw = owners * a.slabs < 2048 ? 8 : 4;
+  // (eight waves where their staged tiles fit 64 KB)
+  const int nw = owners * a.slabs < 2048 && (!pair || mt * (cplx ? 2 : 1) <= 3) ? 8 : 4;
   const dim3 grid(static_cast<unsigned>(a.nown), static_cast<unsigned>((groups + a.ncw - 1) / a.ncw),
                   static_cast<unsigned>(a.slabs * a.vd));
 #define BMI_ROWS(CC, FT, RVV, MTT)                                                        \
   if (cplx == CC && fp32 == std::is_same<FT, float>::value && rv == RVV && mt == MTT) { \
-    if (nt == 1)                                                                        \
-      launch_rows<CC, FT, RVV, MTT, 1>(a, grid, nw, st);                                \
+    if (pair)                                                                           \
+      launch_rows<CC, FT, RVV, MTT, 1, true>(a, grid, nw, st);                          \
+    else if (nt == 1)                                                                   \
+      launch_rows<CC, FT, RVV, MTT, 1, false>(a, grid, nw, st);                         \
     else                                                                                \
-      launch_rows<CC, FT, RVV, MTT, 2>(a, grid, nw, st);                                \
+      launch_rows<CC, FT, RVV, MTT, 2, false>(a, grid, nw, st);                         \
     return;                                                                             \
   }
   BMI_ROWS(false, double, 1, 1)
@@ -283,6 +420,21 @@ void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st) {
   BMI_ROWS(true, float, 1, 3)
 #undef BMI_ROWS
   throw Error(BMI_UNSUPPORTED, "no block-row sweep of this tile count");
+}
+
+void launch_pair_rows(bool cplx, bool fp32, RowsArgs a, const PairSweep& ps, hipStream_t st) {
+  if (a.nown <= 0 || a.nrhs <= 0) return;
+  a.rp = ps.rp, a.src = ps.src, a.blk = ps.blk, a.slot = ps.slot, a.part = ps.part;
+  launch_block_rows(cplx, fp32, a, st);
+  if (a.yl == 0) a.yl = a.nrhs;
+  a.slabs = block_rows_slabs(cplx, a.n, a.nown);
+  const int64_t nt = static_cast<int64_t>(ps.ngather) * a.nrhs * a.n;
+  const dim3 grid(static_cast<unsigned>((nt + 255) / 256));
+  if (cplx)
+    hipLaunchKernelGGL(k_pair_gather<true>, grid, dim3(256), 0, st, a, ps.ngather, ps.gtgt, ps.grp);
+  else
+    hipLaunchKernelGGL(k_pair_gather<false>, grid, dim3(256), 0, st, a, ps.ngather, ps.gtgt, ps.grp);
+  BMI_CHECK_HIP(hipGetLastError());
 }
 
 }  // namespace bmi

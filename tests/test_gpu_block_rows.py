@@ -83,3 +83,28 @@ def test_gpu_block_rows_maxwell_columns(gpu, n_cheb, precision):
     one = np.stack([H @ X[:, k] for k in range(5)], 1)
     for c in (2, 3, 5):
         assert np.linalg.norm(H @ X[:, :c] - one[:, :c]) <= 1e-13 * np.linalg.norm(one[:, :c]), c
+
+
+@pytest.mark.parametrize("precision", [B.FP64, B.MIXED])
+@pytest.mark.parametrize("kind,P,n_cheb", [("laplace", 1, 6), ("laplace", 2, 7), ("helmholtz", 1, 6), ("helmholtz", 2, 9),
+                                           ("maxwell", 1, 6), ("maxwell", 1, 9)])
+def test_gpu_block_rows_pairs(gpu, kind, P, n_cheb, precision):
+    # one block of each symmetric pair against every block: the same terms summed in another order, and
+    # the two weights of a coupling entry multiplied in the other order (an ulp of the entry).  Columns up
+    # to the tile and past it; the workspace first grown by a product that does not use pairs
+    op = {"laplace": B.LaplaceSingleLayerOperator, "helmholtz": B.HelmholtzSingleLayerOperator,
+          "maxwell": B.MaxwellSingleLayerOperator}[kind]()
+    if kind != "laplace":
+        op.set_wavenumber(2.0 - 0.1j)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), 3, P, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb, precision=precision)
+    X = _columns(ps.number_of_dofs, 20, op.scalar, 11)
+    for c in (20, 1, 2, 3, 7):
+        H.set_sweep(None)
+        got = H @ X[:, :c]
+        again = H @ X[:, :c]
+        H.set_sweep("full")
+        want = H @ X[:, :c]
+        assert np.array_equal(got, again), c
+        tol = 1e-13 if precision == B.FP64 else 1e-6
+        assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want), c
