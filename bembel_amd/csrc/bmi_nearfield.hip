@@ -22,6 +22,9 @@
 // 0.71, vertex 0.65, regular 0.60).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "bmi_internal.h"
 #include "bmi_device.h"
 
@@ -32,6 +35,9 @@ struct NFParams {
   int poly_stride;
   double h;        // element width in the parameter domain
   double rh, rh2;  // 1 / h, 1 / h^2 (powers of two)
+  // powers of two with the size l of the geometry in them, about l^-4 and (l / h)^2: squared measures of line
+  // points times ms are of order one at any unit of length, and mr takes the factor back
+  double ms, mr;
   double kre, kim;  // wavenumber
   int dummy_fn;
   const double* ffield;  // far-field table, FF_STRIDE doubles per point
@@ -397,13 +403,16 @@ __device__ __forceinline__ void line_contract(PolyPtr G, bool fix_u, double f, d
 }
 
 // A point of a contracted line.  The surface measure stays split as sqrt(cc) m, m with the weight: the
-// kernel takes sqrt(cc / |x - y|^2) by one reciprocal square root of the product.
+// kernel takes sqrt(cc / |x - y|^2) by one reciprocal square root of the product.  cc is scaled by
+// NFParams::ms: the product of two of them and |x - y|^2 would else leave the range of a double
+// where lengths do by the power of ten.
 struct LinePt {
   double x0, x1, x2, cc, m, s0, s1;
 };
 
-// the smallest cc used: a vanishing measure (a collapsed edge) then gives zero, not 0 / 0
-constexpr double MIN_CC = 1e-200;
+// the smallest cc |x - y|^2 whose root is taken: a vanishing measure of either point (an element without
+// area) then gives cc times a finite number, zero, and not 0 / 0
+constexpr double MIN_CCS = 1e-300;
 
 template <int PD, int KIND>
 __device__ __forceinline__ LinePt line_point(const double* L, const NFParams& prm, bool fix_u, double u, double v,
@@ -434,7 +443,7 @@ __device__ __forceinline__ LinePt line_point(const double* L, const NFParams& pr
   if constexpr (KIND == BMI_DUMMY) {
     q.cc = 1.0, q.m = w;
   } else {
-    q.cc = fmax(cross_square(E1, E2), MIN_CC), q.m = (bot * bot) * (prm.rh2 * w);
+    q.cc = cross_square(E1, E2) * prm.ms, q.m = (bot * bot) * (prm.mr * w);
   }
   return q;
 }
@@ -473,7 +482,7 @@ __device__ __forceinline__ void line_points(const double* L, const NFParams& prm
       E2[k] = fma(-X[k], d2[m][3], d2[m][k]);
     }
     q[m].x0 = X[0], q[m].x1 = X[1], q[m].x2 = X[2];
-    q[m].cc = fmax(cross_square(E1, E2), MIN_CC), q[m].m = (bot * bot) * prm.rh2;
+    q[m].cc = cross_square(E1, E2) * prm.ms, q[m].m = (bot * bot) * prm.mr;
     // computed here: moved behind the branches of the phases, the points would keep both lines'
     // coefficients in registers
     asm volatile("" : "+v"(q[m].x0), "+v"(q[m].x1), "+v"(q[m].x2), "+v"(q[m].cc), "+v"(q[m].m));
@@ -557,7 +566,7 @@ __device__ __forceinline__ void kernel_scaled(double d0, double d1, double d2, d
                                               double& kr, double& ki) {
   // f sqrt(cc) exp(-i kappa r) / (4 pi r)
   const double s = d0 * d0 + d1 * d1 + d2 * d2;
-  const double mag = (f * (0.25 * M_1_PI)) * (cc * rsqrt_newton(cc * s));
+  const double mag = (f * (0.25 * M_1_PI)) * (cc * rsqrt_newton(fmax(cc * s, MIN_CCS)));
   if constexpr (KIND == BMI_LAPLACE_SL) {
     kr = mag, ki = 0.0;
   } else {
@@ -1612,6 +1621,18 @@ static const double* element_polynomials(const bmi_space* s, DevBuf<double>& buf
   return buf.ptr;
 }
 
+// element widths, and the scaling of the line points' measures by the radius of the largest patch
+static void set_lengths(const bmi_space* s, NFParams& prm) {
+  double l = 0.0;
+  for (const double r : s->crad[0]) l = std::max(l, r);
+  const int k = l > 0.0 && std::isfinite(l) ? std::max(-250, std::min(250, std::ilogb(l))) : 0;
+  prm.h = 1.0 / s->n;
+  prm.rh = s->n;
+  prm.rh2 = static_cast<double>(s->n) * s->n;
+  prm.ms = std::ldexp(1.0, -4 * k);
+  prm.mr = std::ldexp(prm.rh2, 2 * k);
+}
+
 // dynamic LDS of one workgroup of class CLS at quadrature degree deg (each workgroup sizes its
 // point tables from its own pair's degree)
 template <int P, int KIND, int PD, int CLS, int NT>
@@ -1735,9 +1756,7 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
   NFParams prm;
   prm.poly = element_polynomials(s, d_poly, st);
   prm.poly_stride = 4 * s->pd * s->pd;
-  prm.h = 1.0 / s->n;
-  prm.rh = s->n;
-  prm.rh2 = static_cast<double>(s->n) * s->n;
+  set_lengths(s, prm);
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;
   prm.dummy_fn = op.dummy_fn;
@@ -1786,9 +1805,7 @@ void launch_integrate_jobs(const bmi_space* s, const bmi_op_desc& op, const std:
   NFParams prm;
   prm.poly = element_polynomials(s, d_poly, st);
   prm.poly_stride = 4 * s->pd * s->pd;
-  prm.h = 1.0 / s->n;
-  prm.rh = s->n;
-  prm.rh2 = static_cast<double>(s->n) * s->n;
+  set_lengths(s, prm);
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;
   prm.dummy_fn = op.dummy_fn;
