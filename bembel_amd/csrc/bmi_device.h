@@ -122,6 +122,13 @@ __device__ __forceinline__ double rsqrt_newton_any(double s) {
   return __builtin_amdgcn_class(y0, 0x240) ? y0 : rsqrt_newton(s);  // +infinity, +0
 }
 
+// sqrt(s) from y = rsqrt_newton(s): s y corrected once by its residual.  s y alone is off by up to two ulps,
+// which a phase kappa r multiplies by its size
+__device__ __forceinline__ double sqrt_newton(double s, double y) {
+  const double r = s * y;
+  return fma(0.5 * y, fma(-r, r, s), r);
+}
+
 // a b + c with the constant c in scalar registers: from vector registers the compiler copies it first,
 // into the accumulator of the two-operand form
 __device__ __forceinline__ double fma_const(double a, double b, double c) {

@@ -98,56 +98,62 @@ __global__ __launch_bounds__(256) void k_pot_sources(const double* __restrict__ 
 template <int KIND, bool FAR, bool DECAY, int DIM>
 __device__ __forceinline__ void pot_tile(const double* tile, int cnt, double x0, double x1, double x2, double kre,
                                          double kim, double (&sr)[DIM], double (&si)[DIM]) {
-  // the tile's own sums, added at the end: fewer roundings at the size of the whole sum
-  double ar[DIM], ai[DIM];
+  // 64 sources have sums of their own, added at the end: a multiply-add of complex factors rounds twice at
+  // the size of the sum, which one sum per tile showed as 1.4 times the error (864 sources: 5.9e-16 with
+  // products rounded first, 8.5e-16 without)
+  for (int j0 = 0; j0 < cnt; j0 += 64) {
+    double ar[DIM], ai[DIM];
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) ar[d] = 0.0, ai[d] = 0.0;
-  for (int j = 0; j < cnt; ++j) {
-    const double* sj = tile + j * PotSrc<KIND>::N;
-    const double d0 = x0 - sj[0], d1 = x1 - sj[1], d2 = x2 - sj[2];
-    const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-    const double ir = rsqrt_newton_any(r2);  // infinite where the target is the source
-    if constexpr (KIND == BMI_LAPLACE_SL) {
-      ar[0] += ir * sj[3];
-    } else {
-      // exp(-i kappa r) / r = exp(kim r) (cos(kre r) - i sin(kre r)) / r
-      const double r = r2 * ir;
-      double sn, cs;
-      if constexpr (FAR)
-        sincos_phase(kre * r, &sn, &cs);
-      else
-        sincos_near(kre * r, &sn, &cs);
-      const double mag = DECAY ? exp(kim * r) * ir : ir;
-      const double Kr = mag * cs, Ki = -mag * sn;
-      if constexpr (KIND == BMI_HELMHOLTZ_SL) {
-        ar[0] = fma(-Ki, sj[4], fma(Kr, sj[3], ar[0]));
-        ai[0] = fma(Ki, sj[3], fma(Kr, sj[4], ai[0]));
+    for (int d = 0; d < DIM; ++d) ar[d] = 0.0, ai[d] = 0.0;
+    const int j1 = j0 + 64 < cnt ? j0 + 64 : cnt;
+    for (int j = j0; j < j1; ++j) {
+      const double* sj = tile + j * PotSrc<KIND>::N;
+      const double d0 = x0 - sj[0], d1 = x1 - sj[1], d2 = x2 - sj[2];
+      const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+      const double ir = rsqrt_newton_any(r2);  // infinite where the target is the source
+      if constexpr (KIND == BMI_LAPLACE_SL) {
+        ar[0] += ir * sj[3];
       } else {
-        // grad_x K = K (-1 - i kappa r) / r^2 (x - y)
-        const double fr = -1.0 + kim * r, fi = -kre * r;
-        const double ir2 = ir * ir;
-        const double Gr = (Kr * fr - Ki * fi) * ir2, Gi = (Kr * fi + Ki * fr) * ir2;
-        const double dd[3] = {d0, d1, d2};
-        // G * div (complex)
-        const double gdr = Gr * sj[9] - Gi * sj[10], gdi = Gr * sj[10] + Gi * sj[9];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          ar[k] += Kr * sj[3 + k] - Ki * sj[6 + k] + gdr * dd[k];
-          ai[k] += Kr * sj[6 + k] + Ki * sj[3 + k] + gdi * dd[k];
+        // exp(-i kappa r) / r = exp(kim r) (cos(kre r) - i sin(kre r)) / r
+        const double r = sqrt_newton(r2, ir);
+        double sn, cs;
+        if constexpr (FAR)
+          sincos_phase(kre * r, &sn, &cs);
+        else
+          sincos_near(kre * r, &sn, &cs);
+        const double mag = DECAY ? exp(kim * r) * ir : ir;
+        const double Kr = mag * cs, Ki = -mag * sn;
+        if constexpr (KIND == BMI_HELMHOLTZ_SL) {
+          ar[0] = fma(-Ki, sj[4], fma(Kr, sj[3], ar[0]));
+          ai[0] = fma(Ki, sj[3], fma(Kr, sj[4], ai[0]));
+        } else {
+          // grad_x K = K (-1 - i kappa r) / r^2 (x - y)
+          const double fr = -1.0 + kim * r, fi = -kre * r;
+          const double ir2 = ir * ir;
+          const double Gr = (Kr * fr - Ki * fi) * ir2, Gi = (Kr * fi + Ki * fr) * ir2;
+          const double dd[3] = {d0, d1, d2};
+          // G * div (complex)
+          const double gdr = Gr * sj[9] - Gi * sj[10], gdi = Gr * sj[10] + Gi * sj[9];
+  #pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            ar[k] += Kr * sj[3 + k] - Ki * sj[6 + k] + gdr * dd[k];
+            ai[k] += Kr * sj[6 + k] + Ki * sj[3 + k] + gdi * dd[k];
+          }
         }
       }
     }
-  }
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) sr[d] += ar[d], si[d] += ai[d];
+    for (int d = 0; d < DIM; ++d) sr[d] += ar[d], si[d] += ai[d];
+  }
 }
 
 // partial[chunk][comp][point] (complex interleaved for C) = sum over the chunk's sources.  Bound by the
 // FP64 vector units: the distance and its reciprocal root, the phase's sine and cosine and the complex
-// multiply-add, 65 instructions per target and source of the Helmholtz layer (with the library's sqrt,
+// multiply-add, 68 instructions per target and source of the Helmholtz layer (with the library's sqrt,
 // division, sincos and exp it was 185).  The phase's range is checked once per tile, from |x| and |y|
-// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.42 ms; error
-// 1.7e-15 -> 0.8e-15 (the tiles' own sums).
+// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.49 ms; error
+// 1.7e-15 -> 0.7e-15, and below the former for few sources too (the roots and sums rounded for speed alone,
+// 1.44 ms, were up to 1.45 times further off than it for 864 to 6,144 sources).
 template <int KIND>
 __global__ __launch_bounds__(POT_TILE) void k_pot_sum(const double* __restrict__ src, int64_t nsrc, int64_t chunk,
                                                       const double* __restrict__ pts, int npts, double kre,

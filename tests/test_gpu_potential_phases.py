@@ -4,12 +4,14 @@ meets a source or lies beyond the range of r^2.
 The kernel chooses its sine and cosine for 256 targets and 256 sources at a time from |x| and |y|: a
 target far away moves its neighbours in the call to the general form, with and without which they must
 agree (both within 3e-16 per sine; the sums of up to 1,536 sources with signs within 1e-12 of the
-largest value).  Values themselves are compared with the oracle in test_gpu_potential.py.
+largest value).  Values themselves are compared with the oracle in test_gpu_potential.py, their rounding
+with extended precision here.
 """
 import numpy as np
 import pytest
 
 import bembel_amd as B
+import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +49,83 @@ def test_gpu_laplace_potential_beyond_the_range(gpu):
     dp = _potential("laplace", 0j)
     got = np.asarray(dp.evaluate(np.array([[1e200, 0.0, 0.0], [2.0, 0.0, 0.0]])))
     assert got[0] == 0.0 and np.isfinite(got[1]) and got[1] != 0.0  # r^2 overflows: 1 / r is 0
+
+
+def _sphere_sum(T, pts, sup, elements, kappa, M):
+    """The Helmholtz potential at pts of a P = 1 density (element functions' coefficients sup, four per
+    element) with numpy in the type T, every operation rounded once: the 3 x 3 Gauss points of each element
+    as sources."""
+    with open(B.SPHERE_DAT) as f:
+        lines = f.read().splitlines()[5:]
+    cp = np.array([[np.array(lines[9 * p + 5 + m].split(), dtype=float).reshape(5, 5).T for m in range(4)]
+                   for p in range(6)]).transpose(0, 2, 3, 1).astype(T)  # (patch, s, t, xyzw)
+    half, h = T(1) / 2, T(1) / 2 ** M
+    x = half + half * np.sqrt(T(3) / 5) * np.array([-1, 0, 1], dtype=T)
+    w = np.array([5, 8, 5], dtype=T) / 18
+    binom = {3: (1, 3, 3, 1), 4: (1, 4, 6, 4, 1)}
+
+    def bern(p, t):
+        return np.stack([binom[p][k] * t ** k * (1 - t) ** (p - k) for k in range(p + 1)], -1)
+
+    def der(t):
+        b = bern(3, t)
+        z = np.zeros_like(b[..., :1])
+        return 4 * (np.concatenate([z, b], -1) - np.concatenate([b, z], -1))
+
+    s, t = (elements["llc"].astype(T)[:, None, None, k] + h * (x[:, None] if k == 0 else x[None, :]) for k in (0, 1))
+    s, t = np.broadcast_arrays(s, t)
+    c = cp[elements["patch"]][:, None, None]
+
+    def form(a, b):
+        return ((a[..., :, None, None] * c).sum(-3) * b[..., :, None]).sum(-2)
+
+    v, vs, vt = form(bern(4, s), bern(4, t)), form(der(s), bern(4, t)), form(bern(4, s), der(t))
+    X = v[..., :3] / v[..., 3:]
+    ds, dt = ((d[..., :3] - X * d[..., 3:]) / v[..., 3:] for d in (vs, vt))
+    area = np.sqrt((np.cross(ds, dt) ** 2).sum(-1))
+    b = np.stack([1 - x, x], -1)  # degree 1
+    rho = np.einsum("eyx,ux,vy->euv", sup.reshape(-1, 2, 2), b, b)
+    q = (rho * (area * h * w[:, None] * w[None, :])).reshape(-1)
+    d = pts.astype(T)[:, None, :] - X.reshape(1, -1, 3)
+    r = np.sqrt((d ** 2).sum(-1))
+    four_pi = 4 * (T(4) * np.arctan(T(1)))
+    K = (np.cos(T(kappa) * r) - 1j * np.sin(T(kappa) * r)) / r / four_pi
+    return (K * q).sum(-1)
+
+
+@pytest.mark.parametrize("kappa", [8.0, 16.0])
+def test_gpu_potential_rounds_as_its_operations(gpu, kappa):
+    # few sources (864), where the phases carry most of the error: the distance to extended precision is that of
+    # pairwise sums in doubles whose roots, sines and quotients are rounded once.  An eighth more is left for the
+    # running sums over 64 sources (2 roundings of 2^-53 / sqrt(3) a source at the size of a partial sum, about
+    # 2.5e-16 of the result here, beside 6.4e-16 and 25e-16 of the plain sums).  Roots within two ulps and
+    # running sums over 256 sources were at 1.49 and 1.21 times the plain sums.
+    if np.finfo(np.longdouble).eps > 2e-19:
+        pytest.skip("no extended precision on this host")
+    M = 2
+    op = B.HelmholtzSingleLayerOperator()
+    ps = B.AnsatzSpace(B.Geometry(), M, 1, op)
+    rng = np.random.default_rng(11)
+    rho = rng.uniform(-1, 1, ps.number_of_dofs) + 1j * rng.uniform(-1, 1, ps.number_of_dofs)
+    d = rng.normal(size=(2000, 3))
+    pts = d / np.linalg.norm(d, axis=1, keepdims=True) * rng.uniform(2, 4, (2000, 1))
+    pot = B.HelmholtzSingleLayerPotential()
+    pot.set_wavenumber(complex(kappa))
+    dp = B.DiscretePotential(pot, ps)
+    dp.set_cauchy_data(rho)
+    got = np.asarray(dp.evaluate(pts))
+    rp, col, val = O.Space(O.Geometry(), M, 1).T()
+    rows = np.repeat(np.arange(len(rp) - 1), np.diff(rp))
+
+    def total(T):
+        sup = np.zeros(len(rp) - 1, dtype=np.result_type(T, np.complex128))
+        np.add.at(sup, rows, val.astype(T) * rho[col])
+        return _sphere_sum(T, pts, sup, ps.elements(), kappa, M)
+
+    exact = total(np.longdouble)
+
+    def error(y):
+        return float(np.linalg.norm(y - exact) / np.linalg.norm(exact))
+
+    print("error here", error(got), "of plain sums", error(total(np.float64)))
+    assert error(got) <= 1.125 * error(total(np.float64))
