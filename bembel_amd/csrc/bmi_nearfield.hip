@@ -82,10 +82,32 @@ struct Pt<BMI_MAXWELL_SL> {
 // of the Bernstein form (no basis to evaluate), and |u - 1/2| <= 1/2 keeps the sums as well
 // conditioned.  With x = p / w the tangents are (p_u - x w_u) / w, (p_v - x w_v) / w; derivatives
 // in the patch parameters are 1 / h times those in u, v.
+// The coordinates are those about the element's centre, rounded to single precision (the table's last entries;
+// zero for the test operator, whose values depend on the place): what all points of an element share, the
+// rounding of its coefficients, is then small against the element and not against the body, and the distances
+// of touching elements keep it.  Blocks of edge neighbours of 6,144 elements, P 2, against extended precision:
+// coefficients summed in doubles about the origin 1.5e-15 (points in Bernstein form, each rounded for itself,
+// 5.2e-16), so 4.5e-16.
 // element polynomials, written by an earlier kernel only: in the constant address space, so that
 // wave-uniform loads go through the scalar cache wherever they stand (as plain global memory the
 // compiler gave that up in the longer rules)
 typedef const __attribute__((address_space(4))) double* PolyPtr;
+
+// a point of one element about the centre of the other; the centres are read where they are used, as the
+// coefficients
+struct Shift {
+  PolyPtr o1, o2;
+  template <class PT>
+  __device__ __forceinline__ static PT moved(PT p, PolyPtr from, PolyPtr to) {
+    asm volatile("" : "+s"(from), "+s"(to));
+    p.x0 += from[0] - to[0], p.x1 += from[1] - to[1], p.x2 += from[2] - to[2];
+    return p;
+  }
+  template <class PT>
+  __device__ __forceinline__ PT to_second(const PT& p) const { return moved(p, o1, o2); }
+  template <class PT>
+  __device__ __forceinline__ PT to_first(const PT& p) const { return moved(p, o2, o1); }
+};
 
 // Sums over wave-uniform coefficients (scalar registers) take powers of the coordinate: of the operands
 // of a multiply-add one may be scalar, and a Horner chain starts with two (moves into vector registers
@@ -887,6 +909,8 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
   const int lane = tid & 63;
   const PolyPtr g1 = (PolyPtr)(prm.poly + static_cast<int64_t>(pr.e1) * prm.poly_stride);
   const PolyPtr g2 = (PolyPtr)(prm.poly + static_cast<int64_t>(pr.e2) * prm.poly_stride);
+  // points are about the centre of their element; of two elements' points the one of the outer loop is moved
+  const Shift sh{g1 + prm.poly_stride - 4, g2 + prm.poly_stride - 4};
   const double h = prm.h;
   const int n = pr.deg + 1;
   const int nq = n * n;
@@ -957,7 +981,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
       VecSum<P, CPLX> vs;
       vs.zero();
       if (act) {
-        const PtK F = q1[unit];
+        const PtK F = sh.to_second(q1[unit]);
 #pragma unroll 1
         for (int j = sub; j < nq; j += S) {
           const PtK b = q2[j];
@@ -1000,7 +1024,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
     PtK* q2 = q1 + nq;
     for (int k = tid; k < nq; k += NT) {
       const double u = gx[k / n], v = gx[k % n], w = h * (gw[k / n] * gw[k % n]);
-      q1[k] = make_point<PD, KIND>(g1, prm, u, v, w);
+      q1[k] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, w));
       q2[k] = make_point<PD, KIND>(g2, prm, u, v, w);
     }
     __syncthreads();
@@ -1240,7 +1264,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
         {
           double u, v;
           tau(odd ? 1 - t1 : t1, e0, r1, u, v);
-          const PtK F = make_point<PD, KIND>(g1, prm, u, v, fa);
+          const PtK F = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, fa));
           const double xc = moved(r2, odd ? 1 - t2 : t2);
           auto col = [&](int j1) { return colt[odd * per + j1]; };
           if (r2 & 1)
@@ -1251,7 +1275,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
         const double x = odd ? 1 - t4 : t4;
         // g = 1, 2: the rotation, uniform in the workgroup, fixed at compile time (tau and the line
         // evaluation without selects)
-        const LinePt F1 = on_line(0, odd ? 1 - t3 : t3);
+        const LinePt F1 = sh.to_second(on_line(0, odd ? 1 - t3 : t3));
         with_rotation(r2, [&](auto R) {
           constexpr int RC = decltype(R)::value;
           constexpr bool FS = (RC & 1) == 0;
@@ -1264,7 +1288,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
             return line_point<PD, KIND>(L, prm, FS, u, v, gw[j1]);
           });
         });
-        const LinePt F2 = on_line(1, odd ? 1 - t3 : t3);
+        const LinePt F2 = sh.to_first(on_line(1, odd ? 1 - t3 : t3));
         with_rotation(r1, [&](auto R) {
           constexpr int RC = decltype(R)::value;
           constexpr bool FS = (RC & 1) == 0;
@@ -1335,10 +1359,10 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
       const PtK* p6 = tin + (cn + c0) * nq;
 #pragma unroll 1
       for (int k = 0; k < 2; ++k)  // rows q0, q1 (element 1), columns p5 (element 2)
-        factor_pass<P, KIND, true>(acc, q[4 * i + k], role, act, sub, S, nq, prm, [&](int j) { return p5[j]; });
+        factor_pass<P, KIND, true>(acc, sh.to_second(q[4 * i + k]), role, act, sub, S, nq, prm, [&](int j) { return p5[j]; });
 #pragma unroll 1
       for (int k = 2; k < 4; ++k)  // rows p6 (element 1), columns q2, q3 (element 2)
-        factor_pass<P, KIND, false>(acc, q[4 * i + k], role, act, sub, S, nq, prm, [&](int j) { return p6[j]; });
+        factor_pass<P, KIND, false>(acc, sh.to_first(q[4 * i + k]), role, act, sub, S, nq, prm, [&](int j) { return p6[j]; });
     }
     __syncthreads();
   } else if constexpr (CLS == 3) {
@@ -1366,11 +1390,11 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
         if (kind < 2) {  // g = 0, a: (t1, e0) on element 1
           const double t1 = xi0 * (1 - xi1);
           tau(odd ? 1 - t1 : t1, xi1 * xj, r1, u, v);
-          tab[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
+          tab[e] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, 1.0));
         } else if (kind < 4) {  // g = 1, a: (t3, xi1) on element 1
           const double t3 = xi0 * (1 - xi1 * xj);
           tau(odd ? 1 - t3 : t3, xi1, r1, u, v);
-          tab[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
+          tab[e] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, 1.0));
         } else if (kind < 6) {  // g = 2, b: (t3, xi1) on element 2
           const double t3 = xi0 * (1 - xi1 * xj);
           tau(odd ? 1 - t3 : t3, xi1, r2, u, v);
@@ -1412,7 +1436,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
           } else {
             double u, v;
             tau(odd ? 1 - t4 : t4, e1, r1, u, v);
-            a = make_point<PD, KIND>(g1, prm, u, v, 1.0);
+            a = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, 1.0));
             b = tab[(4 + odd) * per + ta];
           }
           a.W *= w;
@@ -1435,9 +1459,9 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
       const double w = h * h * wi * (xi0 * xi0 * xi0);
       double u, v;
       tau(xi0, xi1, r1, u, v);
-      q[4 * i + 0] = make_point<PD, KIND>(g1, prm, u, v, w);
+      q[4 * i + 0] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, w));
       tau(xi1, xi0, r1, u, v);
-      q[4 * i + 1] = make_point<PD, KIND>(g1, prm, u, v, w);
+      q[4 * i + 1] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, w));
       tau(xi0, xi1, r2, u, v);
       q[4 * i + 2] = make_point<PD, KIND>(g2, prm, u, v, w);
       tau(xi1, xi0, r2, u, v);
@@ -1458,7 +1482,7 @@ __global__ __launch_bounds__(NT, nf_waves(KIND, CLS)) void k_nearfield(const NFP
           tin[e] = make_point<PD, KIND>(g2, prm, u, v, 1.0);
         } else {
           tau(e0, e1, r1, u, v);
-          tin[e] = make_point<PD, KIND>(g1, prm, u, v, 1.0);
+          tin[e] = sh.to_second(make_point<PD, KIND>(g1, prm, u, v, 1.0));
         }
       }
       __syncthreads();
@@ -1563,12 +1587,27 @@ void launch_ffield_table(const bmi_space* s, int n, int fs, double* out, hipStre
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+// an unevaluated sum hi + lo: hi the rounded sum, lo the rounding errors of its additions and products
+struct TwoSum {
+  double hi = 0.0, lo = 0.0;
+  __device__ __forceinline__ void add_product(double a, double b) {
+#pragma clang fp contract(off)
+    const double p = a * b, s = hi + p, t = s - hi;
+    lo += fma(a, b, -p) + ((hi - (s - t)) + (p - t));
+    hi = s;
+  }
+};
+
 // the homogeneous coordinates of every element in powers of u - 1/2, v - 1/2 (poly_point): coefficient
 // (a, b) is h^(a + b) / (a! b!) times the derivative at the element's centre, from differences of the
-// control points in Bernstein form; one thread per (element, a, b)
+// control points in Bernstein form; one thread per (element, a, b).  An error of a coefficient is one of all
+// points of the element, of which a block's sum leaves the whole where it averages those of the points: each is
+// rounded once.  The weights are exact (element corners are multiples of 2^-M, M <= 10: 44 bits), and the sums
+// over the control points carry their rounding errors along.
 template <int PD>
 __global__ void k_element_poly(const double* __restrict__ cp, int cp_stride, const int* __restrict__ elem_patch,
-                               const double* __restrict__ elem_llc, int nel, double h, double* __restrict__ out) {
+                               const double* __restrict__ elem_llc, int nel, double h, int centre, int stride,
+                               double* __restrict__ out) {
   const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (gid >= static_cast<int64_t>(nel) * PD * PD) return;
   const int e = static_cast<int>(gid / (PD * PD)), q = static_cast<int>(gid % (PD * PD));
@@ -1592,29 +1631,52 @@ __global__ void k_element_poly(const double* __restrict__ cp, int cp_stride, con
     }
   };
   double ws[PD], wt[PD];
+  double O[3] = {0, 0, 0};  // the same in every thread of the element
+  if (centre) {
+    weights(0, elem_llc[2 * e] + 0.5 * h, ws);
+    weights(0, elem_llc[2 * e + 1] + 0.5 * h, wt);
+    double p[4] = {0, 0, 0, 0};
+    for (int j = 0; j < PD; ++j)
+      for (int i = 0; i < PD; ++i)
+        for (int k = 0; k < 4; ++k) p[k] += wt[j] * ws[i] * c[4 * (i * PD + j) + k];
+    for (int k = 0; k < 3; ++k) O[k] = static_cast<float>(p[k] / p[3]);
+  }
   weights(q / PD, elem_llc[2 * e] + 0.5 * h, ws);
   weights(q % PD, elem_llc[2 * e + 1] + 0.5 * h, wt);
-  double v[4] = {0, 0, 0, 0};
+  TwoSum v[4];
   for (int j = 0; j < PD; ++j) {
-    double r[4] = {0, 0, 0, 0};
+    TwoSum r[4];
     for (int i = 0; i < PD; ++i)
-      for (int k = 0; k < 4; ++k) r[k] += ws[i] * c[4 * (i * PD + j) + k];
-    for (int k = 0; k < 4; ++k) v[k] += wt[j] * r[k];
+      for (int k = 0; k < 4; ++k) r[k].add_product(ws[i], c[4 * (i * PD + j) + k]);
+    for (int k = 0; k < 4; ++k) {
+      v[k].add_product(wt[j], r[k].hi);
+      v[k].lo += wt[j] * r[k].lo;
+    }
   }
-  for (int k = 0; k < 4; ++k) out[gid * 4 + k] = v[k];
+  for (int k = 0; k < 3; ++k) {  // about O: the weight times O taken off
+    v[k].add_product(-O[k], v[3].hi);
+    v[k].lo -= O[k] * v[3].lo;
+  }
+  double* o = out + static_cast<int64_t>(e) * stride;
+  for (int k = 0; k < 4; ++k) o[4 * q + k] = v[k].hi + v[k].lo;
+  if (q == 0)
+    for (int k = 0; k < 4; ++k) o[stride - 4 + k] = k < 3 ? O[k] : 0.0;
 }
 
-static const double* element_polynomials(const bmi_space* s, DevBuf<double>& buf, hipStream_t st) {
+// doubles of an element's polynomials and centre
+static int poly_stride(const bmi_space* s) { return 4 * s->pd * s->pd + 4; }
+
+static const double* element_polynomials(const bmi_space* s, bool centre, DevBuf<double>& buf, hipStream_t st) {
   const int64_t n = static_cast<int64_t>(s->nel) * s->pd * s->pd;
-  buf.alloc(static_cast<size_t>(4 * n));
+  buf.alloc(static_cast<size_t>(s->nel) * poly_stride(s));
   const dim3 grid(static_cast<unsigned>((n + 255) / 256));
   const int stride = 4 * s->pd * s->pd;
   if (s->pd == 2)
     hipLaunchKernelGGL(k_element_poly<2>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
-                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, buf.ptr);
+                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), buf.ptr);
   else if (s->pd == 5)
     hipLaunchKernelGGL(k_element_poly<5>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
-                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, buf.ptr);
+                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), buf.ptr);
   else
     throw Error(BMI_UNSUPPORTED, "patch degree not supported on the device");
   BMI_CHECK_HIP(hipGetLastError());
@@ -1754,8 +1816,8 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
   }
   DevBuf<double> d_poly;
   NFParams prm;
-  prm.poly = element_polynomials(s, d_poly, st);
-  prm.poly_stride = 4 * s->pd * s->pd;
+  prm.poly = element_polynomials(s, op.kind != BMI_DUMMY, d_poly, st);
+  prm.poly_stride = poly_stride(s);
   set_lengths(s, prm);
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;
@@ -1803,8 +1865,8 @@ void launch_integrate_jobs(const bmi_space* s, const bmi_op_desc& op, const std:
   d_pairs.upload(pairs, st);
   DevBuf<double> d_poly;
   NFParams prm;
-  prm.poly = element_polynomials(s, d_poly, st);
-  prm.poly_stride = 4 * s->pd * s->pd;
+  prm.poly = element_polynomials(s, op.kind != BMI_DUMMY, d_poly, st);
+  prm.poly_stride = poly_stride(s);
   set_lengths(s, prm);
   prm.kre = op.kappa_re;
   prm.kim = op.kappa_im;

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 import bembel_amd as B
+import extended_lib as X
 import oracle_lib as O
 
 pytestmark = pytest.mark.gpu
@@ -55,38 +56,12 @@ def _sphere_sum(T, pts, sup, elements, kappa, M):
     """The Helmholtz potential at pts of a P = 1 density (element functions' coefficients sup, four per
     element) with numpy in the type T, every operation rounded once: the 3 x 3 Gauss points of each element
     as sources."""
-    with open(B.SPHERE_DAT) as f:
-        lines = f.read().splitlines()[5:]
-    cp = np.array([[np.array(lines[9 * p + 5 + m].split(), dtype=float).reshape(5, 5).T for m in range(4)]
-                   for p in range(6)]).transpose(0, 2, 3, 1).astype(T)  # (patch, s, t, xyzw)
-    half, h = T(1) / 2, T(1) / 2 ** M
-    x = half + half * np.sqrt(T(3) / 5) * np.array([-1, 0, 1], dtype=T)
-    w = np.array([5, 8, 5], dtype=T) / 18
-    binom = {3: (1, 3, 3, 1), 4: (1, 4, 6, 4, 1)}
-
-    def bern(p, t):
-        return np.stack([binom[p][k] * t ** k * (1 - t) ** (p - k) for k in range(p + 1)], -1)
-
-    def der(t):
-        b = bern(3, t)
-        z = np.zeros_like(b[..., :1])
-        return 4 * (np.concatenate([z, b], -1) - np.concatenate([b, z], -1))
-
-    s, t = (elements["llc"].astype(T)[:, None, None, k] + h * (x[:, None] if k == 0 else x[None, :]) for k in (0, 1))
-    s, t = np.broadcast_arrays(s, t)
-    c = cp[elements["patch"]][:, None, None]
-
-    def form(a, b):
-        return ((a[..., :, None, None] * c).sum(-3) * b[..., :, None]).sum(-2)
-
-    v, vs, vt = form(bern(4, s), bern(4, t)), form(der(s), bern(4, t)), form(bern(4, s), der(t))
-    X = v[..., :3] / v[..., 3:]
-    ds, dt = ((d[..., :3] - X * d[..., 3:]) / v[..., 3:] for d in (vs, vt))
-    area = np.sqrt((np.cross(ds, dt) ** 2).sum(-1))
-    b = np.stack([1 - x, x], -1)  # degree 1
+    x, w = X.gauss(3, T)
+    Y, area = X.sphere_points(T, elements, M, x)
+    b = X.linear(x)
     rho = np.einsum("eyx,ux,vy->euv", sup.reshape(-1, 2, 2), b, b)
-    q = (rho * (area * h * w[:, None] * w[None, :])).reshape(-1)
-    d = pts.astype(T)[:, None, :] - X.reshape(1, -1, 3)
+    q = (rho * (area * w[:, None] * w[None, :])).reshape(-1)
+    d = pts.astype(T)[:, None, :] - Y.reshape(1, -1, 3)
     r = np.sqrt((d ** 2).sum(-1))
     four_pi = 4 * (T(4) * np.arctan(T(1)))
     K = (np.cos(T(kappa) * r) - 1j * np.sin(T(kappa) * r)) / r / four_pi
@@ -100,7 +75,7 @@ def test_gpu_potential_rounds_as_its_operations(gpu, kappa):
     # running sums over 64 sources (2 roundings of 2^-53 / sqrt(3) a source at the size of a partial sum, about
     # 2.5e-16 of the result here, beside 6.4e-16 and 25e-16 of the plain sums).  Roots within two ulps and
     # running sums over 256 sources were at 1.49 and 1.21 times the plain sums.
-    if np.finfo(np.longdouble).eps > 2e-19:
+    if not X.HAS_EXTENDED:
         pytest.skip("no extended precision on this host")
     M = 2
     op = B.HelmholtzSingleLayerOperator()
