@@ -87,7 +87,7 @@ struct Pt<BMI_MAXWELL_SL> {
 // rounding of its coefficients, is then small against the element and not against the body, and the distances
 // of touching elements keep it.  Blocks of edge neighbours of 6,144 elements, P 2, against extended precision:
 // coefficients summed in doubles about the origin 1.5e-15 (points in Bernstein form, each rounded for itself,
-// 5.2e-16), so 4.5e-16.
+// 5.2e-16), so 4.5e-16, 1.7e-16 with the sums of add_products.
 // element polynomials, written by an earlier kernel only: in the constant address space, so that
 // wave-uniform loads go through the scalar cache wherever they stand (as plain global memory the
 // compiler gave that up in the longer rules)
@@ -681,7 +681,9 @@ typedef double nf_d4 __attribute__((ext_vector_type(4)));
 // vector, (P+1)^2 entries each; the pairs put them in the wave's own part of LDS (three arrays of 32
 // vectors: fixed, real, imaginary) and eight 16x16x4 steps add the 32 products to the wave's block.  The
 // block takes 8 registers (16 complex) instead of a share of it per lane (90 and 162 for P = 2), which
-// kept the rules at one wave per SIMD.
+// kept the rules at one wave per SIMD.  The 32 products have a sum of their own (one part of a complex block
+// after the other: the registers of one): thousands of terms in one running sum rounded the blocks to 4.5e-16
+// where the points leave 1.6e-16 (identical rule, 6,144 elements, P 2).
 template <int I2>
 __host__ __device__ constexpr int stage_doubles(bool cplx) {
   return 32 * (cplx ? 3 : 2) * I2;
@@ -696,14 +698,18 @@ template <int I2, bool CPLX, bool COLS>
 __device__ __forceinline__ void add_products(const double* stage, int lane, nf_d4& dr, nf_d4& di) {
   const int li = lane & 15, lk = lane >> 4, row = li < I2 ? li : I2 - 1;  // entries past the block are not read back
 #pragma unroll
-  for (int st = 0; st < 8; ++st) {
-    const int m = (4 * st + lk) * I2 + row;
-    const double f = stage[m], r = stage[32 * I2 + m];
-    dr = __builtin_amdgcn_mfma_f64_16x16x4f64(COLS ? f : r, COLS ? r : f, dr, 0, 0, 0);
-    if constexpr (CPLX) {
-      const double i = stage[64 * I2 + m];
-      di = __builtin_amdgcn_mfma_f64_16x16x4f64(COLS ? f : i, COLS ? i : f, di, 0, 0, 0);
+  for (int part = 0; part < (CPLX ? 2 : 1); ++part) {
+    nf_d4 d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      const int m = (4 * st + lk) * I2 + row;
+      const double f = stage[m], v = stage[(part + 1) * 32 * I2 + m];
+      d = __builtin_amdgcn_mfma_f64_16x16x4f64(COLS ? f : v, COLS ? v : f, d, 0, 0, 0);
     }
+    if (part == 0)
+      dr += d;
+    else
+      di += d;
   }
 }
 

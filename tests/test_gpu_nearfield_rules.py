@@ -171,9 +171,8 @@ def test_gpu_rules_round_touching_pairs(gpu, tmp_path, kappa):
     # A body whose control points have 21 bits, in its own unit and in a third of it: every length is exactly three
     # times the other, and what a block differs by from 27 times the other's is its rounding (either's, so by the
     # root of two).  Each of the 11^4 points of a rule is within a few ulps (2^-53) of its element's size, and their
-    # errors average out; what is left is the rounding of running sums of a thousand terms and more (a wave's units):
-    # sqrt(1000 / 3) times 2^-53 / sqrt(3), 1.2e-15 in one wave's, 6e-16 in the four waves'.  Coefficients rounded
-    # against the body were at 2.2e-15.
+    # errors average out: what is left is of the order of one ulp, 1.1e-16 to 3e-16 a block.  Coefficients rounded
+    # against the body and sums of thousands of terms were at 2e-15.
     with open(B.SPHERE_DAT) as f:
         lines = f.read().splitlines()
     for p in range(6):
@@ -199,4 +198,4 @@ def test_gpu_rules_round_touching_pairs(gpu, tmp_path, kappa):
         norm = np.linalg.norm(one, axis=(1, 2))
         rms = np.sqrt(np.mean((np.linalg.norm(three / 27 - one, axis=(1, 2)) / norm) ** 2) / 2)
         print("rule", rule, len(todo), "root mean square error", rms)
-        assert rms <= 8e-16, rule
+        assert rms <= 4e-16, rule
