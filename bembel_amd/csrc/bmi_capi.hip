@@ -164,6 +164,50 @@ void launch_times_t(bool cplx, int64_t N, int64_t D, const int* trp, const int* 
   BMI_CHECK_HIP(hipGetLastError());
 }
 
+// T^T A T of a small symmetric matrix in one launch, from the half of A (N x N) on and above the diagonal: 16 lanes
+// per entry (i, j), each a share of row i of T^T against the whole of row j
+template <int S>
+__global__ __launch_bounds__(256) void k_ttat_small(int64_t N, int D, const int* __restrict__ trp,
+                                                    const int* __restrict__ tcol, const double* __restrict__ tval,
+                                                    const double* __restrict__ A, double* __restrict__ R) {
+  const int64_t id = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) >> 4;
+  const int lane = threadIdx.x & 15;
+  const bool on = id < static_cast<int64_t>(D) * D;
+  const int j = on ? static_cast<int>(id / D) : 0, i = on ? static_cast<int>(id - static_cast<int64_t>(j) * D) : 0;
+  double v[S];
+#pragma unroll
+  for (int c = 0; c < S; ++c) v[c] = 0.0;
+  for (int p = trp[i] + lane; p < trp[i + 1]; p += 16) {
+    const int64_t r = tcol[p];
+    double w[S];
+#pragma unroll
+    for (int c = 0; c < S; ++c) w[c] = 0.0;
+#pragma unroll 8
+    for (int q = trp[j]; q < trp[j + 1]; ++q) {
+      const int64_t k = tcol[q], at = S * (r <= k ? k * N + r : r * N + k);
+#pragma unroll
+      for (int c = 0; c < S; ++c) w[c] += tval[q] * A[at + c];
+    }
+#pragma unroll
+    for (int c = 0; c < S; ++c) v[c] += tval[p] * w[c];
+  }
+#pragma unroll
+  for (int c = 0; c < S; ++c) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1) v[c] += __shfl_xor(v[c], o, 16);
+    if (on && lane == 0) R[S * id + c] = v[c];
+  }
+}
+void launch_ttat_small(bool cplx, int64_t N, int64_t D, const int* trp, const int* tcol, const double* tval, const double* A,
+                       double* R, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>((D * D * 16 + 255) / 256));
+  if (cplx)
+    hipLaunchKernelGGL(k_ttat_small<2>, grid, dim3(256), 0, st, N, static_cast<int>(D), trp, tcol, tval, A, R);
+  else
+    hipLaunchKernelGGL(k_ttat_small<1>, grid, dim3(256), 0, st, N, static_cast<int>(D), trp, tcol, tval, A, R);
+  BMI_CHECK_HIP(hipGetLastError());
+}
+
 __global__ void k_fill(double* p, int64_t n, double v) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1602,6 +1646,11 @@ bmi_status bmi_integrate_jobs(const bmi_space* s, const bmi_op_desc* op, int njo
   BMI_API_END
 }
 
+// super rows up to which the whole of T^T A T is one launch: with the copy of the half and two products the launches
+// are a sixth of the time of 24 elements, P 1 (Laplace 116 -> 102 us, 104 with the product on the host), and 96
+// elements, P 2, the 864 rows here, are still 1 to 4 % faster so; its reads grow as the square of a row of T^T
+constexpr int64_t DENSE_SMALL = 864;
+
 bmi_status bmi_dense_assemble(const bmi_space* s, const bmi_op_desc* op, int super_only, double* out, int mem,
                               void* stream) {
   BMI_API_BEGIN
@@ -1613,8 +1662,8 @@ bmi_status bmi_dense_assemble(const bmi_space* s, const bmi_op_desc* op, int sup
   const int64_t N = s->nsuper, D = s->ndof;
   const int ff = farfield_degree(op->kind, s->P);
   // The super matrix of a single layer is symmetric (as for the H2 leaves): the pairs e1 <= e2 are
-  // integrated and the other half is copied; the test operator's is not.  384 elements, P = 1: 6.2 ms with
-  // every pair and T^T A T on the host, 1.7 ms so.
+  // integrated and the other half is copied; the test operator's is not.  384 elements, P = 1: 6.4 ms with
+  // every pair and T^T A T on the host, 1.6 ms so.
   const bool sym = op->kind != BMI_DUMMY;
   const int64_t ne = s->nel, np = sym ? ne * (ne + 1) / 2 : ne * ne;
   std::vector<NFPair> v(np);
@@ -1629,26 +1678,26 @@ bmi_status bmi_dense_assemble(const bmi_space* s, const bmi_op_desc* op, int sup
         v[slot++] = classify_pair(s, op->kind, ff, static_cast<int>(e1), static_cast<int>(e2), e2 * s->I2 * N + e1 * s->I2);
     }
   });
-  DevBuf<double> A;
-  A.alloc(static_cast<size_t>(S) * N * N);
+  // the super matrix A, C = A T (N x D) and T^T C (D x D), in one allocation
+  const int64_t na = S * N * N, nc = super_only ? 0 : S * N * D, nr = super_only ? na : S * D * D;
+  DevBuf<double> buf;
+  buf.alloc(static_cast<size_t>(na + nc + (super_only || mem == BMI_MEM_DEVICE ? 0 : nr)));
+  double *A = buf.ptr, *C = A + na, *R = super_only ? A : mem == BMI_MEM_DEVICE ? out : C + nc;
   // super-space rows and columns are component-major: component c starts at c * nel * I2
   const int64_t vcs = static_cast<int64_t>(s->nel) * s->I2;
-  launch_nearfield(s, *op, v, A.ptr, 1, N, vcs, vcs * N, st);
-  if (sym) launch_mirror_dense(cplx, N, vcs, s->I2, A.ptr, st);
-  const hipMemcpyKind to = mem == BMI_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
-  if (super_only) {
-    BMI_CHECK_HIP(hipMemcpyAsync(out, A.ptr, A.bytes(), to, st));
+  launch_nearfield(s, *op, v, A, 1, N, vcs, vcs * N, st);
+  if (sym && !super_only && s->vd == 1 && N <= DENSE_SMALL) {
+    launch_ttat_small(cplx, N, D, s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, A, R, st);
   } else {
-    // C = A T (N x D), then T^T C (D x D)
-    DevBuf<double> C, R;
-    C.alloc(static_cast<size_t>(S) * N * D);
-    R.alloc(static_cast<size_t>(S) * D * D);
-    launch_times_t(cplx, N, D, s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, A.ptr, C.ptr, st);
-    launch_spmv(cplx, static_cast<int>(D), static_cast<int>(D), s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, C.ptr, N,
-                R.ptr, D, nullptr, nullptr, st);
-    BMI_CHECK_HIP(hipMemcpyAsync(out, R.ptr, R.bytes(), to, st));
-    BMI_CHECK_HIP(hipStreamSynchronize(st));
+    if (sym) launch_mirror_dense(cplx, N, vcs, s->I2, A, st);
+    if (!super_only) {
+      launch_times_t(cplx, N, D, s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, A, C, st);
+      launch_spmv(cplx, static_cast<int>(D), static_cast<int>(D), s->d_trowptr.ptr, s->d_tcol.ptr, s->d_tval.ptr, C, N, R,
+                  D, nullptr, nullptr, st);
+    }
   }
+  if (R != out)
+    BMI_CHECK_HIP(hipMemcpyAsync(out, R, nr * sizeof(double), mem == BMI_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st));
   BMI_CHECK_HIP(hipStreamSynchronize(st));
   BMI_API_END
 }

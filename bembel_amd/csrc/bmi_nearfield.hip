@@ -1602,91 +1602,107 @@ struct TwoSum {
     lo += fma(a, b, -p) + ((hi - (s - t)) + (p - t));
     hi = s;
   }
+  __device__ __forceinline__ void add_product(double a, const double2& b) {  // a (hi, lo)
+    add_product(a, b.x);
+    lo = fma(a, b.y, lo);
+  }
 };
 
 // the homogeneous coordinates of every element in powers of u - 1/2, v - 1/2 (poly_point): coefficient
 // (a, b) is h^(a + b) / (a! b!) times the derivative at the element's centre, from differences of the
-// control points in Bernstein form; one thread per (element, a, b).  An error of a coefficient is one of all
-// points of the element, of which a block's sum leaves the whole where it averages those of the points: each is
-// rounded once.  The weights are exact (element corners are multiples of 2^-M, M <= 10: 44 bits), and the sums
-// over the control points carry their rounding errors along.
+// control points in Bernstein form.  An error of a coefficient is one of all points of the element, of which a
+// block's sum leaves the whole where it averages those of the points: each is rounded once.  The weights are
+// exact (element corners are multiples of 2^-M, M <= 10: 44 bits), and the sums over the control points carry
+// their rounding errors along.
+// Bound: latency.  A workgroup holds an element, one direction after the other, a thread per sum of PD products
+// (a thread per coefficient, with sums of PD^2 products and weights of its own in scratch memory: 24 elements
+// 15.0 us, 3.3 so; 24,576 elements 83 -> 27 us).
+constexpr int POLY_NT = 128;
 template <int PD>
-__global__ void k_element_poly(const double* __restrict__ cp, int cp_stride, const int* __restrict__ elem_patch,
-                               const double* __restrict__ elem_llc, int nel, double h, int centre, int stride,
-                               double* __restrict__ out) {
-  const int64_t gid = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (gid >= static_cast<int64_t>(nel) * PD * PD) return;
-  const int e = static_cast<int>(gid / (PD * PD)), q = static_cast<int>(gid % (PD * PD));
-  const double* c = cp + static_cast<int64_t>(elem_patch[e]) * cp_stride;
-  // weights of the control points in the a-th power coefficient of one direction about x:
-  // h^a binom(p, a) sum over r of (-1)^(a - r) binom(a, r) B_(i - r) of degree p - a
-  auto weights = [&](int a, double x, double* w) {
-    constexpr int p = PD - 1;
-    double B[PD];
-    for (int i = 0; i < PD; ++i) w[i] = 0.0, B[i] = 0.0;
-    B[0] = 1.0;
-    for (int d = 1; d <= p - a; ++d)  // Bernstein recurrence up to degree p - a
-      for (int i = d; i >= 0; --i) B[i] = (i > 0 ? x * B[i - 1] : 0.0) + (i < d ? (1 - x) * B[i] : 0.0);
+__global__ __launch_bounds__(POLY_NT) void k_element_poly(const double* __restrict__ cp, int cp_stride,
+                                                          const int* __restrict__ elem_patch,
+                                                          const double* __restrict__ elem_llc, double h, int centre,
+                                                          int stride, double* __restrict__ out) {
+  constexpr int p = PD - 1;
+  static_assert(4 * PD * PD <= POLY_NT && 2 * PD <= POLY_NT, "a thread per sum");
+  __shared__ double w[2][PD][PD];  // weights of the control points: direction, power, point
+  __shared__ double2 r[PD][PD][4], v[PD][PD][4];  // sums (hi, lo)
+  const int e = blockIdx.x, t = threadIdx.x;
+  if (t < 2 * PD) {
+    // the a-th power coefficient of one direction about the centre x: h^a binom(p, a) sum over q of
+    // (-1)^(a - q) binom(a, q) B_(i - q) of degree p - a
+    const int dir = t / PD, a = t % PD;
+    const double x = elem_llc[2 * e + dir] + 0.5 * h;
+    double B[PD], c[PD];
+#pragma unroll
+    for (int i = 0; i < PD; ++i) B[i] = i == 0 ? 1.0 : 0.0, c[i] = 0.0;
+#pragma unroll
+    for (int d = 1; d <= p; ++d)  // Bernstein recurrence up to degree p - a
+      if (d <= p - a)
+#pragma unroll
+        for (int i = d; i >= 0; --i) B[i] = (i > 0 ? x * B[i > 0 ? i - 1 : 0] : 0.0) + (i < d ? (1 - x) * B[i] : 0.0);
     double f = 1.0;
-    for (int k = 0; k < a; ++k) f = f * (p - k) / (k + 1) * h;
-    double bin = 1.0;
-    for (int r = 0; r <= a; ++r) {
-      const double g = ((a - r) & 1) ? -f * bin : f * bin;
-      for (int i = 0; i + a <= p; ++i) w[i + r] += g * B[i];
-      bin = bin * (a - r) / (r + 1);
-    }
-  };
-  double ws[PD], wt[PD];
-  double O[3] = {0, 0, 0};  // the same in every thread of the element
-  if (centre) {
-    weights(0, elem_llc[2 * e] + 0.5 * h, ws);
-    weights(0, elem_llc[2 * e + 1] + 0.5 * h, wt);
-    double p[4] = {0, 0, 0, 0};
-    for (int j = 0; j < PD; ++j)
-      for (int i = 0; i < PD; ++i)
-        for (int k = 0; k < 4; ++k) p[k] += wt[j] * ws[i] * c[4 * (i * PD + j) + k];
-    for (int k = 0; k < 3; ++k) O[k] = static_cast<float>(p[k] / p[3]);
+    int bin = 1;
+#pragma unroll
+    for (int k = 0; k < p; ++k)
+      if (k < a) bin = bin * (p - k) / (k + 1), f *= h;
+    f *= bin;
+    bin = 1;
+#pragma unroll
+    for (int q = 0; q <= p; ++q)
+      if (q <= a) {
+        const double g = ((a - q) & 1) ? -f * bin : f * bin;
+#pragma unroll
+        for (int i = 0; i + q <= p; ++i) c[i + q] += g * B[i];  // B is zero beyond degree p - a
+        bin = bin * (a - q) / (q + 1);
+      }
+#pragma unroll
+    for (int i = 0; i < PD; ++i) w[dir][a][i] = c[i];
   }
-  weights(q / PD, elem_llc[2 * e] + 0.5 * h, ws);
-  weights(q % PD, elem_llc[2 * e + 1] + 0.5 * h, wt);
-  TwoSum v[4];
-  for (int j = 0; j < PD; ++j) {
-    TwoSum r[4];
-    for (int i = 0; i < PD; ++i)
-      for (int k = 0; k < 4; ++k) r[k].add_product(ws[i], c[4 * (i * PD + j) + k]);
-    for (int k = 0; k < 4; ++k) {
-      v[k].add_product(wt[j], r[k].hi);
-      v[k].lo += wt[j] * r[k].lo;
-    }
+  __syncthreads();
+  const int k = t & 3, j = (t >> 2) % PD, a = (t >> 2) / PD;
+  const bool on = t < 4 * PD * PD;
+  if (on) {
+    const double* c = cp + static_cast<int64_t>(elem_patch[e]) * cp_stride + 4 * j + k;
+    TwoSum s;
+#pragma unroll
+    for (int i = 0; i < PD; ++i) s.add_product(w[0][a][i], c[4 * PD * i]);
+    r[a][j][k] = make_double2(s.hi, s.lo);
   }
-  for (int k = 0; k < 3; ++k) {  // about O: the weight times O taken off
-    v[k].add_product(-O[k], v[3].hi);
-    v[k].lo -= O[k] * v[3].lo;
+  __syncthreads();
+  TwoSum s;
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < PD; ++i) s.add_product(w[1][j][i], r[a][i][k]);
+    v[a][j][k] = make_double2(s.hi, s.lo);
   }
+  __syncthreads();
+  if (!on) return;
+  // about the centre: the weight times it taken off
   double* o = out + static_cast<int64_t>(e) * stride;
-  for (int k = 0; k < 4; ++k) o[4 * q + k] = v[k].hi + v[k].lo;
-  if (q == 0)
-    for (int k = 0; k < 4; ++k) o[stride - 4 + k] = k < 3 ? O[k] : 0.0;
+  const double O = centre && k < 3 ? static_cast<double>(static_cast<float>(v[0][0][k].x / v[0][0][3].x)) : 0.0;
+  s.add_product(-O, v[a][j][3]);
+  o[t] = s.hi + s.lo;
+  if (t < 4) o[stride - 4 + t] = O;
 }
 
 // doubles of an element's polynomials and centre
 static int poly_stride(const bmi_space* s) { return 4 * s->pd * s->pd + 4; }
 
-static const double* element_polynomials(const bmi_space* s, bool centre, DevBuf<double>& buf, hipStream_t st) {
-  const int64_t n = static_cast<int64_t>(s->nel) * s->pd * s->pd;
-  buf.alloc(static_cast<size_t>(s->nel) * poly_stride(s));
-  const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+static int64_t poly_doubles(const bmi_space* s) { return static_cast<int64_t>(s->nel) * poly_stride(s); }
+
+static void element_polynomials(const bmi_space* s, bool centre, double* out, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(s->nel));
   const int stride = 4 * s->pd * s->pd;
   if (s->pd == 2)
-    hipLaunchKernelGGL(k_element_poly<2>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
-                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), buf.ptr);
+    hipLaunchKernelGGL(k_element_poly<2>, grid, dim3(POLY_NT), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
+                       s->d_elem_llc.ptr, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), out);
   else if (s->pd == 5)
-    hipLaunchKernelGGL(k_element_poly<5>, grid, dim3(256), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
-                       s->d_elem_llc.ptr, s->nel, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), buf.ptr);
+    hipLaunchKernelGGL(k_element_poly<5>, grid, dim3(POLY_NT), 0, st, s->d_cp.ptr, stride, s->d_elem_patch.ptr,
+                       s->d_elem_llc.ptr, 1.0 / s->n, centre ? 1 : 0, poly_stride(s), out);
   else
     throw Error(BMI_UNSUPPORTED, "patch degree not supported on the device");
   BMI_CHECK_HIP(hipGetLastError());
-  return buf.ptr;
 }
 
 // element widths, and the scaling of the line points' measures by the radius of the largest patch
@@ -1802,7 +1818,6 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
   ensure_device_space(s, st);
   const int ff = farfield_degree(op.kind, s->P);
   const FFTable* tab = ensure_ffield(s, ff, st, op.kind == BMI_MAXWELL_SL);
-  DevBuf<NFPair> d_pairs;
   {
     // stable counting sort by class, then by decreasing degree (degrees < 50): the launches take
     // one class each, its pairs with the largest rules first
@@ -1818,11 +1833,18 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
     std::vector<NFPair> sorted(pairs.size());
     for (const NFPair& p : pairs) sorted[start[p.cls * ND + (ND - 1 - p.deg)]++] = p;
     pairs.swap(sorted);
-    d_pairs.upload(pairs, st);
   }
-  DevBuf<double> d_poly;
+  // polynomials and pairs in one allocation (its cost counts for a few dozen elements)
+  static_assert(sizeof(NFPair) % sizeof(double) == 0, "pairs behind doubles");
+  DevBuf<double> buf;
+  buf.alloc(static_cast<size_t>(poly_doubles(s)) + pairs.size() * (sizeof(NFPair) / sizeof(double)));
+  const NFPair* d_pairs = reinterpret_cast<const NFPair*>(buf.ptr + poly_doubles(s));
+  if (!pairs.empty())
+    BMI_CHECK_HIP(hipMemcpyAsync(buf.ptr + poly_doubles(s), pairs.data(), pairs.size() * sizeof(NFPair),
+                                 hipMemcpyHostToDevice, st));
+  element_polynomials(s, op.kind != BMI_DUMMY, buf.ptr, st);
   NFParams prm;
-  prm.poly = element_polynomials(s, op.kind != BMI_DUMMY, d_poly, st);
+  prm.poly = buf.ptr;
   prm.poly_stride = poly_stride(s);
   set_lengths(s, prm);
   prm.kre = op.kappa_re;
@@ -1846,7 +1868,7 @@ void launch_nearfield(const bmi_space* s, const bmi_op_desc& op, std::vector<NFP
     prm.qre = -k2r / den;
     prm.qim = k2i / den;
   }
-  dispatch(s, op.kind, s->P, pairs, d_pairs.ptr, prm, st);
+  dispatch(s, op.kind, s->P, pairs, d_pairs, prm, st);
   BMI_CHECK_HIP(hipStreamSynchronize(st));
 }
 
@@ -1867,11 +1889,11 @@ void launch_integrate_jobs(const bmi_space* s, const bmi_op_desc& op, const std:
     p.off = k;
     pairs.push_back(p);
   }
-  DevBuf<NFPair> d_pairs;
-  d_pairs.upload(pairs, st);
   DevBuf<double> d_poly;
+  d_poly.alloc(static_cast<size_t>(poly_doubles(s)));
+  element_polynomials(s, op.kind != BMI_DUMMY, d_poly.ptr, st);
   NFParams prm;
-  prm.poly = element_polynomials(s, op.kind != BMI_DUMMY, d_poly, st);
+  prm.poly = d_poly.ptr;
   prm.poly_stride = poly_stride(s);
   set_lengths(s, prm);
   prm.kre = op.kappa_re;

@@ -46,3 +46,17 @@ def test_gpu_dense_halves_and_projection(gpu, kind, M, P):
     want, mag = T.T @ A @ T, np.abs(T).T @ np.abs(A) @ np.abs(T)
     m = int((T != 0).sum(0).max())
     assert (np.abs(G - want) <= 4 * m * 2.0 ** -52 * mag).all()
+
+
+# 864 super rows, the last whose product is one launch, and 1,536
+@pytest.mark.parametrize("M,P", [(2, 2), (3, 1)])
+@pytest.mark.parametrize("kind", ["laplace", "helmholtz"])
+def test_gpu_dense_projection_sizes(gpu, kind, M, P):
+    op = _operator(kind)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), M, P, op)
+    A = np.asarray(B.DenseMatrix(ps, op, super_only=True).matrix)
+    rp, col, val = ps.get_transformation_matrix()
+    T = scipy.sparse.csr_matrix((val, col, rp), shape=(len(A), ps.number_of_dofs)).toarray()
+    G = np.asarray(B.DenseMatrix(ps, op).matrix)
+    m = int((T != 0).sum(0).max())
+    assert (np.abs(G - T.T @ A @ T) <= 4 * m * 2.0 ** -52 * (np.abs(T).T @ np.abs(A) @ np.abs(T))).all()
