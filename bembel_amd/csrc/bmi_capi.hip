@@ -401,7 +401,8 @@ static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
   h->ws_rhs = nrhs;
 }
 
-static bool has_far(const bmi_h2* h) { return h->L >= 0 && h->lvl_total > 0; }
+// (the coarsest meshes have no admissible pair of clusters: their products are the near field alone)
+static bool has_far(const bmi_h2* h) { return h->ntgt > 0; }
 
 // Workspace of one product: the handle's own buffers (bmi_h2_matvec, the solvers), or a region of
 // the per-device scratch array (bmi_h2_matvec_noalloc).  Only products on the handle's own
