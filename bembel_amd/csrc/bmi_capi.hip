@@ -370,15 +370,11 @@ static CouplingOperand coupling_operand(const bmi_h2* h, bool reduced) {
   return {false, h->d_coup.ptr, nullptr, 0, h->cd, static_cast<int64_t>(h->cd) * h->cd};
 }
 
-// Far field from one block of every pair: columns of one tile (the partial sums of one more would cost a
-// second pass over the blocks).  Rows of a block from which it pays: see PAIR_MIN_ROWS.
-static bool pair_columns(const bmi_h2* h, int nrhs) {
-  return h->npairs_far > 0 && (h->mxf ? 4 : 1) * nrhs <= block_rows_tile(h->cplx);
-}
-// scalars of partial sums per pair
-static int64_t pair_partial(const bmi_h2* h, int nrhs) {
-  const int n = h->mxf ? h->np2 : h->cd, cols = (h->mxf ? 4 : 1) * nrhs;
-  return static_cast<int64_t>(block_rows_slabs(h->cplx, n, h->ntgt_all)) * cols * n;
+// far field from one block of every pair (pairs_pay)
+static int pair_rows_of(const bmi_h2* h) { return h->mxf ? h->np2 : h->cd; }
+static bool use_pairs(const bmi_h2* h, int nrhs, bool fp32) {
+  return h->npairs_far > 0 &&
+         pairs_pay(h->cplx, fp32, pair_rows_of(h), h->ntgt_all, h->npairs_far, (h->mxf ? 4 : 1) * nrhs);
 }
 
 static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
@@ -396,7 +392,8 @@ static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
   if (h->npairs_far > 0) {
     // for as many of the columns as one tile takes (a later product of fewer columns uses them)
     const int most = block_rows_tile(h->cplx) / (h->mxf ? 4 : 1);
-    h->d_part.alloc(S * h->npairs_far * pair_partial(h, std::min(nrhs, most)));
+    h->d_part.alloc(S * h->npairs_far *
+                    pair_partial(h->cplx, pair_rows_of(h), h->ntgt_all, (h->mxf ? 4 : 1) * std::min(nrhs, most)));
   }
   h->ws_rhs = nrhs;
 }
@@ -453,11 +450,11 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
   const CouplingOperand co = coupling_operand(h, reduced);
   apply_tree(h, true, nrhs, xs, w.fw[0], w.fw[1], nullptr, st);
   PairSweep pairs{};
-  const bool use_pairs = w.own && h->sweep_mode != 0 && pair_columns(h, nrhs) && !co.Fc;
-  if (use_pairs)
+  const bool paired = w.own && h->sweep_mode != 0 && use_pairs(h, nrhs, co.fp32) && !co.Fc;
+  if (paired)
     pairs = PairSweep{h->d_srp.ptr, h->d_ssrc.ptr, h->d_sblk.ptr, h->d_sgslot.ptr, h->d_part.ptr, h->ngather_far,
                       h->d_sgtgt.ptr, h->d_sgrp.ptr};
-  const PairSweep* ps = use_pairs ? &pairs : nullptr;
+  const PairSweep* ps = paired ? &pairs : nullptr;
   if (h->mxf) {
     // four columns per cluster entry from both components' moments, one sweep over the kernel
     // values writing both components' local expansions (into the moment buffers, consumed), then
@@ -1026,7 +1023,10 @@ static bool pair_rows(const std::vector<int2>& rows, const std::vector<int>& rp,
 static void build_symmetric_lists(bmi_h2* h, const std::vector<int2>& all, const std::vector<int>& rp_all,
                                   const std::vector<int>& csrc, bool pairs, hipStream_t st) {
   PairRows pr;
-  if (pairs && csrc.size() < 2 * static_cast<size_t>(PAIR_MIN_COUNT)) return;
+  // (pairs: for the fewest columns, which gain the most)
+  if (pairs && !pairs_pay(h->cplx, false, pair_rows_of(h), static_cast<int64_t>(all.size()),
+                          static_cast<int64_t>(csrc.size() / 2), h->mxf ? 4 : 1))
+    return;
   const PairOrder order = pairs ? PairOrder::even : h->cplx ? PairOrder::lower : PairOrder::upper;
   if (!pair_rows(all, rp_all, csrc, order, false, pr) || pr.nslots == 0) return;
   h->d_ssrc.upload(pr.src, st);
@@ -1329,7 +1329,7 @@ static void assemble_h2(bmi_h2* h, hipStream_t st) {
     }
     if (vd == 1 && (op.kind == BMI_LAPLACE_SL || op.kind == BMI_HELMHOLTZ_SL) && sym_sweep_supported(h->cplx, h->dd, h->cd))
       build_symmetric_lists(h, all, rp_all, csrc, false, st);
-    else if (op.kind != BMI_DUMMY && (h->mxf || vd == 1) && (h->mxf ? h->np2 : h->cd) >= PAIR_MIN_ROWS)
+    else if (op.kind != BMI_DUMMY && (h->mxf || vd == 1))
       build_symmetric_lists(h, all, rp_all, csrc, true, st);
   }
   // FP32 coupling copy: MIXED pads the columns to whole 16-byte row vectors (the sweeps read rows
@@ -1748,12 +1748,12 @@ bmi_status bmi_h2_estimate_bytes(const bmi_space* s, const bmi_op_desc* op, int 
     if (S == 1) b += lvl_total * 16 + lvl_total / cd * 32;            // node tables
   }
   b += (int64_t(dense.size()) + int64_t(lowrank.size())) * 8;                           // CSR indices
-  const int64_t pn = mxf ? np2 : cd, pc = mxf ? 4 : 1;  // lists and partial sums of paired coupling blocks
-  if (op->kind != BMI_DUMMY && (mxf || vd == 1) && pn >= PAIR_MIN_ROWS &&
-      int64_t(lowrank.size()) >= 2 * PAIR_MIN_COUNT)
-    b += int64_t(lowrank.size()) / 2 *
-         (12 + S * 8 * block_rows_slabs(S == 2, static_cast<int>(pn), lvl_total / cd) * pn * pc *
-                   std::min<int64_t>(std::max(nrhs, 1), block_rows_tile(S == 2) / pc));
+  const int64_t pn = mxf ? np2 : cd;
+  const int pc = mxf ? 4 : 1;  // lists and partial sums of paired coupling blocks
+  const int64_t npairs = int64_t(lowrank.size()) / 2, ncl = lvl_total / cd;
+  if (op->kind != BMI_DUMMY && (mxf || vd == 1) && pairs_pay(S == 2, false, static_cast<int>(pn), ncl, npairs, pc))
+    b += npairs * (12 + S * 8 * pair_partial(S == 2, static_cast<int>(pn), ncl,
+                                             pc * std::min(std::max(nrhs, 1), block_rows_tile(S == 2) / pc)));
   if (cd > 0) b += lvl_total / cd * 12;                                                  // all-cluster list
   b += std::max(nrhs, 1) * S * (3 * int64_t(s->nsuper) + (vd + 1) * lvl_total) * 8;   // workspace
   b += int64_t(s->nel) * 25 * 16 * 8 + int64_t(s->val.size()) * 24;                    // tables, T

@@ -53,16 +53,29 @@ struct PairSweep {
   const int2* gtgt;
   const int* grp;
 };
-// From this many rows of a block and this many pairs on.  Pairs against every block, one column / four:
-// 36 rows, 34,000 pairs (real) 302 / 335 against 318 / 342 us; 49 rows, 7,300 pairs (complex) 245 / 278
-// against 294 / 308; 81 rows, 1,900 pairs (real) 156 / 163 against 165 / 166; with 25 rows four columns gain
-// 3 %, and the partial sums of a few columns come near the size of the blocks.
+// blocks of fewer rows are not paired: with 25 the partial sums of a few columns come near the size of the
+// blocks, and four columns gain 3 %
 constexpr int PAIR_MIN_ROWS = 36;
-constexpr int PAIR_MIN_COUNT = 1024;
 // row slabs of a launch: parts of the rows with partial sums of their own
 int block_rows_slabs(bool cplx, int n, int64_t owners);
 // columns of one tile
 constexpr int block_rows_tile(bool cplx) { return cplx ? 8 : 16; }
+// scalars of partial sums of one pair
+inline int64_t pair_partial(bool cplx, int n, int64_t owners, int cols) {
+  return static_cast<int64_t>(block_rows_slabs(cplx, n, owners)) * cols * n;
+}
+// whether a sweep of cols columns over npairs pairs (n rows, owners clusters) is the faster one: the bytes of the
+// blocks that are not read, less three quarters of those of the partial sums, written and read (some stay in the
+// caches), are 100 MB or more, the 20 us that the second pass through LDS and the gather take.  Over 191 cases of 36
+// to 81 rows, 1 to 16 columns, 384 to 6,144 elements, FP64 and FP32 the pairs it takes are 0.97 to 1.49 times as
+// fast as every block and the ones it leaves 0.84 to 1.04: 6,144 elements, 81 rows, one column 861 us by every block,
+// 638 by pairs, 16 columns 1,079 and 970; 1,536 elements, 36 rows, 16 columns 166 and 193.
+inline bool pairs_pay(bool cplx, bool fp32, int n, int64_t owners, int64_t npairs, int cols) {
+  if (n < PAIR_MIN_ROWS || cols > block_rows_tile(cplx)) return false;
+  const int64_t S = cplx ? 2 : 1;
+  const int64_t blocks = S * n * n * (fp32 ? 4 : 8), partial = 2 * S * 8 * pair_partial(cplx, n, owners, cols);
+  return npairs * (4 * blocks - 3 * partial) >= 400 * 1000 * 1000;
+}
 // the sweep of a's targets from their pairs: block rows, then the partial sums
 void launch_pair_rows(bool cplx, bool fp32, RowsArgs a, const PairSweep& ps, hipStream_t st);
 void launch_block_rows(bool cplx, bool fp32, RowsArgs a, hipStream_t st);

@@ -108,3 +108,48 @@ def test_gpu_block_rows_pairs(gpu, kind, P, n_cheb, precision):
         assert np.array_equal(got, again), c
         tol = 1e-13 if precision == B.FP64 else 1e-6
         assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want), c
+
+
+# Row tiles of a workgroup by rows and clusters: real 2 (36 and 64 rows, 510 clusters), 4 (81 rows, 510; 36, 2,046) and 6
+# (81 rows, 2,046), complex 1 (64 rows, 126), 2 (36 rows, 510) and 3 (81 rows, 510; 36 rows, 2,046); one to four row slabs
+@pytest.mark.parametrize("kind,M,n_cheb,paired", [
+    ("laplace", 4, 6, (1,)), ("laplace", 4, 8, (1, 8, 9)), ("laplace", 4, 9, (1, 3, 12)), ("laplace", 5, 6, (1, 8, 9, 15, 16)),
+    ("laplace", 5, 9, (1, 9, 16)), ("helmholtz", 3, 8, (1,)), ("helmholtz", 4, 6, (1, 2, 3)),
+    ("helmholtz", 4, 9, (1, 5, 7, 8)), ("helmholtz", 5, 6, (1, 7, 8)), ("maxwell", 4, 6, (1,)), ("maxwell", 4, 9, (1, 2))])
+def test_gpu_block_rows_pair_tiles(gpu, kind, M, n_cheb, paired):
+    # as above, the workspace growing from product to product; a product that reads every block gives the bits of
+    # the forced one, and one column past the tile does
+    op = {"laplace": B.LaplaceSingleLayerOperator, "helmholtz": B.HelmholtzSingleLayerOperator,
+          "maxwell": B.MaxwellSingleLayerOperator}[kind]()
+    if kind != "laplace":
+        op.set_wavenumber(2.0 - 0.1j)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), M, 1, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb)
+    past = {"laplace": 17, "helmholtz": 9, "maxwell": 3}[kind]
+    X = _columns(ps.number_of_dofs, past, op.scalar, 13)
+    for c in paired + (past,):
+        H.set_sweep(None)
+        got = H @ X[:, :c]
+        H.set_sweep("full")
+        want = H @ X[:, :c]
+        assert np.array_equal(got, want) == (c == past), c
+        assert np.linalg.norm(got - want) <= 1e-13 * np.linalg.norm(want), c
+
+
+@pytest.mark.parametrize("kind,M,n_cheb,precision,cols", [
+    ("laplace", 3, 6, B.FP64, (1, 4, 16)), ("laplace", 4, 6, B.FP64, (12, 16)), ("laplace", 4, 6, B.MIXED, (2, 4, 16)),
+    ("helmholtz", 4, 6, B.MIXED, (4, 8)), ("helmholtz", 3, 7, B.FP64, (2, 8)), ("maxwell", 3, 6, B.FP64, (1, 2))])
+def test_gpu_block_rows_pairs_that_do_not_pay(gpu, kind, M, n_cheb, precision, cols):
+    # few or small pairs, many columns, FP32 blocks: partial sums and gather cost more than the blocks saved
+    op = {"laplace": B.LaplaceSingleLayerOperator, "helmholtz": B.HelmholtzSingleLayerOperator,
+          "maxwell": B.MaxwellSingleLayerOperator}[kind]()
+    if kind != "laplace":
+        op.set_wavenumber(2.0 - 0.1j)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), M, 1, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb, precision=precision)
+    X = _columns(ps.number_of_dofs, max(cols), op.scalar, 13)
+    for c in cols:
+        H.set_sweep(None)
+        got = H @ X[:, :c]
+        H.set_sweep("full")
+        assert np.array_equal(got, H @ X[:, :c]), c
