@@ -294,7 +294,7 @@ struct bmi_h2 {
   DevBuf<double> d_part;
   bmi::SymList sl{};
   // without fused upper sweeps: the same lists for block-row sweeps of a few columns (0: none), over
-  // every cluster; part then grows with the workspace
+  // every cluster; part is then made by the first product that uses them (ensure_partials)
   int64_t npairs_far = 0;
   int ngather_far = 0;
   // workspace (grown on demand)
@@ -376,9 +376,33 @@ static bool use_pairs(const bmi_h2* h, int nrhs, bool fp32) {
   return h->npairs_far > 0 &&
          pairs_pay(h->cplx, fp32, pair_rows_of(h), h->ntgt_all, h->npairs_far, (h->mxf ? 4 : 1) * nrhs);
 }
+static int64_t partial_doubles(const bmi_h2* h, int nrhs) {
+  return (h->cplx ? 2 : 1) * h->npairs_far *
+         pair_partial(h->cplx, pair_rows_of(h), h->ntgt_all, (h->mxf ? 4 : 1) * nrhs);
+}
 
-static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
-  (void)st;
+// Partial sums of a product of nrhs columns, when such a product comes first.  Without them it reads every block:
+// when there is no memory for them, and on a stream that a caller captures.
+static void ensure_partials(bmi_h2* h, int nrhs, bool reduced, hipStream_t st) {
+  const CouplingOperand co = coupling_operand(h, reduced);
+  if (co.Fc || !use_pairs(h, nrhs, co.fp32)) return;
+  const size_t n = static_cast<size_t>(partial_doubles(h, nrhs));
+  if (n <= h->d_part.n) return;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  BMI_CHECK_HIP(hipStreamIsCapturing(st, &cs));
+  if (cs != hipStreamCaptureStatusNone) return;
+  h->drop_graphs();
+  try {
+    h->d_part.alloc(n);
+  } catch (const Error& e) {
+    if (e.status != BMI_OUT_OF_MEMORY) throw;
+    (void)hipGetLastError();
+    h->npairs_far = 0;
+  }
+}
+
+static void ensure_workspace(bmi_h2* h, int nrhs, bool reduced, hipStream_t st) {
+  ensure_partials(h, nrhs, reduced, st);
   if (nrhs <= h->ws_rhs) return;
   h->drop_graphs();
   const int S = h->cplx ? 2 : 1;
@@ -389,12 +413,6 @@ static void ensure_workspace(bmi_h2* h, int nrhs, hipStream_t st) {
   h->d_bw.alloc(S * h->lvl_total * nrhs);
   h->d_yf.alloc(S * N * nrhs);
   if (h->mxf) h->d_mxz.alloc(2 * S * h->lvl_total * nrhs);  // 4 np2 columns per entry = 2 cd
-  if (h->npairs_far > 0) {
-    // for as many of the columns as one tile takes (a later product of fewer columns uses them)
-    const int most = block_rows_tile(h->cplx) / (h->mxf ? 4 : 1);
-    h->d_part.alloc(S * h->npairs_far *
-                    pair_partial(h->cplx, pair_rows_of(h), h->ntgt_all, (h->mxf ? 4 : 1) * std::min(nrhs, most)));
-  }
   h->ws_rhs = nrhs;
 }
 
@@ -450,7 +468,8 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
   const CouplingOperand co = coupling_operand(h, reduced);
   apply_tree(h, true, nrhs, xs, w.fw[0], w.fw[1], nullptr, st);
   PairSweep pairs{};
-  const bool paired = w.own && h->sweep_mode != 0 && use_pairs(h, nrhs, co.fp32) && !co.Fc;
+  const bool paired = w.own && h->sweep_mode != 0 && !co.Fc && use_pairs(h, nrhs, co.fp32) &&
+                      static_cast<int64_t>(h->d_part.n) >= partial_doubles(h, nrhs);
   if (paired)
     pairs = PairSweep{h->d_srp.ptr, h->d_ssrc.ptr, h->d_sblk.ptr, h->d_sgslot.ptr, h->d_part.ptr, h->ngather_far,
                       h->d_sgtgt.ptr, h->d_sgrp.ptr};
@@ -844,7 +863,7 @@ static void apply_dof(bmi_h2* h, const Work& w, int nrhs, const double* X, int64
 
 void h2_apply_device(bmi_h2* h, int nrhs, const double* X, int64_t ldx, double* Y, int64_t ldy, const double* alpha,
                      const double* beta, hipStream_t st, bool reduced) {
-  ensure_workspace(h, nrhs, st);
+  ensure_workspace(h, nrhs, reduced, st);
   apply_dof(h, handle_work(h), nrhs, X, ldx, Y, ldy, alpha, beta, st, reduced);
 }
 
@@ -1751,9 +1770,12 @@ bmi_status bmi_h2_estimate_bytes(const bmi_space* s, const bmi_op_desc* op, int 
   const int64_t pn = mxf ? np2 : cd;
   const int pc = mxf ? 4 : 1;  // lists and partial sums of paired coupling blocks
   const int64_t npairs = int64_t(lowrank.size()) / 2, ncl = lvl_total / cd;
-  if (op->kind != BMI_DUMMY && (mxf || vd == 1) && pairs_pay(S == 2, false, static_cast<int>(pn), ncl, npairs, pc))
-    b += npairs * (12 + S * 8 * pair_partial(S == 2, static_cast<int>(pn), ncl,
-                                             pc * std::min(std::max(nrhs, 1), block_rows_tile(S == 2) / pc)));
+  if (op->kind != BMI_DUMMY && (mxf || vd == 1) && pairs_pay(S == 2, false, static_cast<int>(pn), ncl, npairs, pc)) {
+    b += npairs * 12;
+    const int cols = pc * std::max(nrhs, 1);
+    if (pairs_pay(S == 2, op->precision != BMI_PRECISION_FP64, static_cast<int>(pn), ncl, npairs, cols))
+      b += npairs * S * 8 * pair_partial(S == 2, static_cast<int>(pn), ncl, cols);
+  }
   if (cd > 0) b += lvl_total / cd * 12;                                                  // all-cluster list
   b += std::max(nrhs, 1) * S * (3 * int64_t(s->nsuper) + (vd + 1) * lvl_total) * 8;   // workspace
   b += int64_t(s->nel) * 25 * 16 * 8 + int64_t(s->val.size()) * 24;                    // tables, T
@@ -1922,7 +1944,7 @@ bmi_status bmi_h2_matvec_super(const bmi_h2* hc, int nrhs, const double* Xs, dou
   bmi_h2* h = const_cast<bmi_h2*>(hc);
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (nrhs == 0) return BMI_OK;
-  ensure_workspace(h, nrhs, st);
+  ensure_workspace(h, nrhs, h2_is_mixed(h), st);
   apply_super(h, handle_work(h), nrhs, Xs, Ys, h->d_yf.ptr, h2_is_mixed(h), st);
   const int S = h->cplx ? 2 : 1;
   if (has_far(h)) device_add(Ys, h->d_yf.ptr, static_cast<int64_t>(S) * h->s->nsuper * nrhs, st);

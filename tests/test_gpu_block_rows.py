@@ -153,3 +153,44 @@ def test_gpu_block_rows_pairs_that_do_not_pay(gpu, kind, M, n_cheb, precision, c
         got = H @ X[:, :c]
         H.set_sweep("full")
         assert np.array_equal(got, H @ X[:, :c]), c
+
+
+@pytest.mark.parametrize("kind,precision,n_cheb,cols,sums", [
+    ("laplace", B.FP64, 9, (17, 12, 1), (0, 12, 12)), ("laplace", B.FP64, 9, (1, 12, 17), (1, 12, 12)),
+    ("laplace", B.FP64, 6, (16, 1), (0, 1)), ("laplace", B.MIXED, 6, (1,), (0,)), ("helmholtz", B.MIXED, 9, (9, 4), (0, 4)),
+    ("maxwell", B.FP64, 9, (3, 2), (0, 2))])
+def test_gpu_partial_sums_held(gpu, kind, precision, n_cheb, cols, sums):
+    # a handle holds partial sums for the largest product that used them, and none for others; the estimate
+    # counts those of its product
+    op = {"laplace": B.LaplaceSingleLayerOperator, "helmholtz": B.HelmholtzSingleLayerOperator,
+          "maxwell": B.MaxwellSingleLayerOperator}[kind]()
+    if kind != "laplace":
+        op.set_wavenumber(2.0 - 0.1j)
+    ps = B.AnsatzSpace(B.Geometry(scale=(1.0, 0.7, 0.5)), 4, 1, op)
+    H = B.H2Matrix(ps, op, n_cheb=n_cheb, precision=precision)
+    S = 1 if kind == "laplace" else 2
+    vd = 2 if kind == "maxwell" else 1
+    clusters, pairs = 510, int((H.leaves()[:, 0] != 2).sum()) // 2
+
+    def held():
+        info = np.zeros(16, dtype=np.int64)
+        B._check(B.library().bmi_h2_info(H._h, info.ctypes.data_as(B.C.POINTER(B.C.c_int64))))
+        return int(info[8])
+
+    def workspace(c):  # three super vectors, multipole and local coefficients, Maxwell's four columns
+        coefficients = clusters * n_cheb ** 2 * vd
+        return 8 * S * c * (3 * ps.number_of_super_dofs + (vd + 1) * coefficients + (2 * coefficients if vd == 2 else 0))
+
+    base, most = held(), 0
+    X = _columns(ps.number_of_dofs, max(cols), op.scalar, 3)
+    for c, s in zip(cols, sums):
+        H @ X[:, :c]
+        most = max(most, c)
+        partial = 8 * S * pairs * 2 * s * (4 if kind == "maxwell" else 1) * n_cheb ** 2  # two row slabs
+        assert held() - base - workspace(most) == partial, (c, held() - base - workspace(most), partial)
+        d = op.desc(n_cheb=n_cheb, eta=1.6, min_cluster_level=1, precision=precision)
+        est = np.zeros(1, dtype=np.int64)
+        B._check(B.library().bmi_h2_estimate_bytes(ps._h, B.C.byref(d), c,
+                                                   est.ctypes.data_as(B.C.POINTER(B.C.c_int64))))
+        if c == cols[0]:
+            assert 1.0 <= est[0] / held() <= 1.05, c
