@@ -488,7 +488,7 @@ static void apply_far(bmi_h2* h, const Work& w, int nrhs, const double* xs, doub
   }
   // every cluster of every level is a target (zero where there are no blocks)
   launch_coupling_apply(C, co.fp32, std::max(h->cpl_variant, 0), h->ntgt_all, nrhs, rows, h->d_tgt_all.ptr,
-                        h->d_crp_all.ptr, h->d_csrc.ptr, co.F, co.blk, 0, h->d_lvl_off.ptr, w.fw[0], w.bw, 0, st,
+                        h->d_crp_all.ptr, h->d_csrc.ptr, co.F, co.blk, h->d_lvl_off.ptr, w.fw[0], w.bw, st,
                         co.Fc, co.ncoarse, co.ld, ps);
   apply_tree(h, false, nrhs, nullptr, w.bw, nullptr, yf, st);
 }
@@ -667,11 +667,11 @@ static void autotune(bmi_h2* h, const double* xs, bool reduced, hipStream_t st) 
                                       apply_near(h, 1, xs, h->d_ys.ptr, st);
                                       return true;
                                     }).first);
-    if (far && wave_coupling_supported(h->cplx, h->cd))
+    if (far && wave_coupling_supported(h->cd))
       h->cpl_variant = std::max(0, pick({0, 1}, 1, 0, [&](int v, int) {
                                      launch_coupling_apply(h->cplx, co.fp32, v, h->ntgt, 1, h->cd, h->d_tgt.ptr,
-                                                           h->d_crp.ptr, h->d_csrc.ptr, co.F, co.blk, 0,
-                                                           h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, 0, st,
+                                                           h->d_crp.ptr, h->d_csrc.ptr, co.F, co.blk,
+                                                           h->d_lvl_off.ptr, h->d_fw[0].ptr, h->d_bw.ptr, st,
                                                            co.Fc, co.ncoarse, co.ld);
                                      return true;
                                    }).first);

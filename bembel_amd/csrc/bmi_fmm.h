@@ -91,14 +91,13 @@ void launch_spmv(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, c
                  const double* x2 = nullptr, bool long_rows = false);
 // block sizes whose single columns run one wave per cluster, in two variants
 bool wave_leaf_supported(int dd);
-bool wave_coupling_supported(bool cplx, int cd);
+bool wave_coupling_supported(int cd);
 // variant: 0 = one block per lane group per iteration, 1 = two (chosen by the autotuner)
 // Fc/ncoarse: BF16 copies of the first ncoarse blocks (fp32 only); ld: column stride of F (0: cd)
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,
-                           const int* rp, const int* src, const void* F, int64_t fstride, int64_t fcomp,
-                           const int64_t* lvl_off, const double* fw, double* bw, int accumulate, hipStream_t st,
-                           const unsigned short* Fc = nullptr, int ncoarse = 0, int ld = 0,
-                           const PairSweep* pairs = nullptr);
+                           const int* rp, const int* src, const void* F, int64_t fstride, const int64_t* lvl_off,
+                           const double* fw, double* bw, hipStream_t st, const unsigned short* Fc = nullptr,
+                           int ncoarse = 0, int ld = 0, const PairSweep* pairs = nullptr);
 // many right-hand sides: internal vectors with the RHS index fastest (see bmi_fmm.hip)
 void launch_spmv_tin(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, const double* v, const double* X,
                      int64_t ldx, double* Yt, hipStream_t st);

@@ -339,22 +339,19 @@ __global__ void k_mx_finish(int64_t ne, int nrhs, int np2, int cd, const double*
 // wave owns one row cluster (near field) or one target cluster (coupling): lane i owns row i,
 // issues all DD (CD) column loads of a block before its first multiply-add, so each wave keeps a
 // whole block in flight, and reads the source segment of the input, which is wave-uniform, via
-// scalar loads.  RT right-hand sides share each block load.
+// scalar loads.  One column; with BF16 copies of the coarsest coupling blocks RT right-hand sides share each
+// block load.
 
-// near field: ys[seg + c*DD + i, k] (+)= sum_blocks F (DD x DD) xs[c2*DD + .., k].  UB blocks
-// are loaded per iteration (their products are still added in block order, so every UB gives the
-// same bits).
+// near field: ys[c*DD + i] = sum_blocks F (DD x DD) xs[c2*DD + ..].  UB blocks are loaded per iteration
+// (their products are still added in block order, so every UB gives the same bits).
 struct LeafArgs {
-  int ncl, nrhs;
+  int ncl;
   const int* rp;
   const int* src;
   const void* F;  // double, or float for the reduced-precision copy
-  int64_t fstride, fcomp;
+  int64_t fstride;
   const double* xs;
-  int64_t ldxs, xseg;
   double* ys;
-  int64_t ldys, yseg;
-  int accumulate;
 };
 
 // wave-uniform double from lane l of v
@@ -363,7 +360,7 @@ __device__ __forceinline__ double lane_double(double v, int l) {
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
-template <bool C, int DD, int RT, int UB, typename FT = double>
+template <bool C, int DD, int UB, typename FT = double>
 __device__ __forceinline__ void leaf_wave(int c, const LeafArgs& a) {
   constexpr int S = C ? 2 : 1;
   static_assert(DD <= 64, "leaf rows exceed a wave");
@@ -372,101 +369,78 @@ __device__ __forceinline__ void leaf_wave(int c, const LeafArgs& a) {
   const int p0 = a.rp[c], p1 = a.rp[c + 1];
   const FT* __restrict__ F = static_cast<const FT*>(a.F);
   const double* __restrict__ xs = a.xs;
-  for (int k0 = 0; k0 < a.nrhs; k0 += RT) {
-    double ar[RT], ai[RT];
+  double ar = 0.0, ai = 0.0;
+  // the source clusters of 64 entries at a time, one per lane: the block loop reads them with
+  // lane reads instead of a dependent load per block
+  for (int q0 = p0; q0 < p1; q0 += 64) {
+    const int srcv = q0 + lane < p1 ? a.src[q0 + lane] : 0;
+    const int q1 = p1 - q0 < 64 ? p1 : q0 + 64;
+    for (int p = q0; p < q1; p += UB) {
+      const int nb = q1 - p < UB ? q1 - p : UB;
+      FT fr[UB][DD], fi[UB][C ? DD : 1];
+      // the source vectors: one coalesced load per lane (lane j: entry j), issued before the
+      // blocks and handed to every lane with lane reads.  Read straight from global memory, each
+      // entry would be a load of one address by the whole wave, and these wait on each other
+      double xr0[UB], xi0[UB];
 #pragma unroll
-    for (int r = 0; r < RT; ++r) ar[r] = 0.0, ai[r] = 0.0;
-    // the source clusters of 64 entries at a time, one per lane: the block loop reads them with
-    // lane reads instead of a dependent load per block
-    for (int q0 = p0; q0 < p1; q0 += 64) {
-      const int srcv = q0 + lane < p1 ? a.src[q0 + lane] : 0;
-      const int q1 = p1 - q0 < 64 ? p1 : q0 + 64;
-      for (int p = q0; p < q1; p += UB) {
-        const int nb = q1 - p < UB ? q1 - p : UB;
-        FT fr[UB][DD], fi[UB][C ? DD : 1];
-        // the source vectors: one coalesced load per lane (lane j: entry j), issued before the
-        // blocks and handed to every lane with lane reads.  Read straight from global memory, each
-        // entry would be a load of one address by the whole wave, and these wait on each other
-        double xr0[UB][RT], xi0[UB][RT];
-#pragma unroll
-        for (int u = 0; u < UB; ++u) {
-          if (UB > 1 && u >= nb) break;
-          const int s2 = __builtin_amdgcn_readlane(srcv, p + u - q0);
-#pragma unroll
-          for (int r = 0; r < RT; ++r) {
-            const int k = k0 + r;
-            if (RT > 1 && k >= a.nrhs) break;
-            const double* x = xs + S * (static_cast<int64_t>(k) * a.ldxs + a.xseg + static_cast<int64_t>(s2) * DD + i);
-            if constexpr (C) {
-              const double2 v = *reinterpret_cast<const double2*>(x);
-              xr0[u][r] = v.x, xi0[u][r] = v.y;
-            } else {
-              xr0[u][r] = x[0];
-            }
-          }
+      for (int u = 0; u < UB; ++u) {
+        if (UB > 1 && u >= nb) break;
+        const double* x = xs + S * (static_cast<int64_t>(__builtin_amdgcn_readlane(srcv, p + u - q0)) * DD + i);
+        if constexpr (C) {
+          const double2 v = *reinterpret_cast<const double2*>(x);
+          xr0[u] = v.x, xi0[u] = v.y;
+        } else {
+          xr0[u] = x[0];
         }
+      }
 #pragma unroll
-        for (int u = 0; u < UB; ++u) {
-          if (UB > 1 && u >= nb) break;
-          const FT* f = F + S * (static_cast<int64_t>(p + u) * a.fstride + a.fcomp);
+      for (int u = 0; u < UB; ++u) {
+        if (UB > 1 && u >= nb) break;
+        const FT* f = F + S * (static_cast<int64_t>(p + u) * a.fstride);
 #pragma unroll
-          for (int j = 0; j < DD; ++j) {
-            if constexpr (C && std::is_same<FT, double>::value) {
-              const double2 v = *reinterpret_cast<const double2*>(f + 2 * (j * DD + i));
-              fr[u][j] = v.x, fi[u][j] = v.y;
-            } else if constexpr (C) {
-              const float2 v = *reinterpret_cast<const float2*>(f + 2 * (j * DD + i));
-              fr[u][j] = v.x, fi[u][j] = v.y;
-            } else {
-              fr[u][j] = f[j * DD + i];
-            }
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < UB; ++u) {
-          if (UB > 1 && u >= nb) break;
-#pragma unroll
-          for (int r = 0; r < RT; ++r) {
-            if (RT > 1 && k0 + r >= a.nrhs) break;
-#pragma unroll
-            for (int j = 0; j < DD; ++j) {
-              const double f_r = static_cast<double>(fr[u][j]);
-              const double xr = lane_double(xr0[u][r], j);
-              if constexpr (C) {
-                const double f_i = static_cast<double>(fi[u][j]);
-                const double xi = lane_double(xi0[u][r], j);
-                ar[r] += f_r * xr - f_i * xi;
-                ai[r] += f_r * xi + f_i * xr;
-              } else {
-                ar[r] += f_r * xr;
-              }
-            }
+        for (int j = 0; j < DD; ++j) {
+          if constexpr (C && std::is_same<FT, double>::value) {
+            const double2 v = *reinterpret_cast<const double2*>(f + 2 * (j * DD + i));
+            fr[u][j] = v.x, fi[u][j] = v.y;
+          } else if constexpr (C) {
+            const float2 v = *reinterpret_cast<const float2*>(f + 2 * (j * DD + i));
+            fr[u][j] = v.x, fi[u][j] = v.y;
+          } else {
+            fr[u][j] = f[j * DD + i];
           }
         }
       }
-    }
-    if (lane < DD) {
 #pragma unroll
-      for (int r = 0; r < RT; ++r) {
-        const int k = k0 + r;
-        if (k >= a.nrhs) break;
-        double* y = a.ys + S * (static_cast<int64_t>(k) * a.ldys + a.yseg + static_cast<int64_t>(c) * DD + lane);
-        if (a.accumulate) {
-          ar[r] += y[0];
-          if constexpr (C) ai[r] += y[1];
+      for (int u = 0; u < UB; ++u) {
+        if (UB > 1 && u >= nb) break;
+#pragma unroll
+        for (int j = 0; j < DD; ++j) {
+          const double f_r = static_cast<double>(fr[u][j]);
+          const double xr = lane_double(xr0[u], j);
+          if constexpr (C) {
+            const double f_i = static_cast<double>(fi[u][j]);
+            const double xi = lane_double(xi0[u], j);
+            ar += f_r * xr - f_i * xi;
+            ai += f_r * xi + f_i * xr;
+          } else {
+            ar += f_r * xr;
+          }
         }
-        y[0] = ar[r];
-        if constexpr (C) y[1] = ai[r];
       }
     }
   }
+  if (lane < DD) {
+    double* y = a.ys + S * (static_cast<int64_t>(c) * DD + lane);
+    y[0] = ar;
+    if constexpr (C) y[1] = ai;
+  }
 }
 
-template <bool C, int DD, int RT, int UB>
+template <bool C, int DD, int UB>
 __global__ __launch_bounds__(256) void k_leaf_w(LeafArgs a) {
   const int c = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6));
   if (c >= a.ncl) return;
-  leaf_wave<C, DD, RT, UB>(c, a);
+  leaf_wave<C, DD, UB>(c, a);
 }
 
 // coupling: bw[t][k][i] (+)= sum over blocks (t, s) of F (CD x CD) fw[s][k][:], all levels in one
@@ -652,14 +626,14 @@ __device__ __forceinline__ void leaf_wave_v(int c, const LeafArgs& a) {
 #pragma unroll
       for (int u = 0; u < UB; ++u) {
         const int pu = p + u < q1 ? p + u : q1 - 1;
-        const double* x = xs + S * (a.xseg + static_cast<int64_t>(__builtin_amdgcn_readlane(srcv, pu - q0)) * DD + le);
+        const double* x = xs + S * (static_cast<int64_t>(__builtin_amdgcn_readlane(srcv, pu - q0)) * DD + le);
         if constexpr (C) {
           const double2 v = *reinterpret_cast<const double2*>(x);
           xor_[u] = v.x, xoi[u] = v.y;
         } else {
           xor_[u] = x[0], xoi[u] = 0.0;
         }
-        const FT* f = F + S * (static_cast<int64_t>(pu) * a.fstride + a.fcomp);
+        const FT* f = F + S * (static_cast<int64_t>(pu) * a.fstride);
 #pragma unroll
         for (int jj = 0; jj < JC; ++jj) {
           const int j = g * JC + jj < DD ? g * JC + jj : DD - 1;
@@ -703,16 +677,11 @@ __device__ __forceinline__ void leaf_wave_v(int c, const LeafArgs& a) {
     if constexpr (C) yi[q] = si;
   }
   if (g0 == 0) {
-    double* y = a.ys + S * (a.yseg + static_cast<int64_t>(c) * DD + RPL * l);
+    double* y = a.ys + S * (static_cast<int64_t>(c) * DD + RPL * l);
 #pragma unroll
     for (int q = 0; q < RPL; ++q) {
-      double vr = yr[q], vi = C ? yi[q] : 0.0;
-      if (a.accumulate) {
-        vr += y[S * q];
-        if constexpr (C) vi += y[S * q + 1];
-      }
-      y[S * q] = vr;
-      if constexpr (C) y[S * q + 1] = vi;
+      y[S * q] = yr[q];
+      if constexpr (C) y[S * q + 1] = yi[q];
     }
   }
 }
@@ -1374,7 +1343,7 @@ __device__ __forceinline__ void sweep_fused_body(const LeafArgs& la, const CplAr
       if constexpr (R2N)
         leaf_wave_v<C, NFT, DD, UBN>(c, la);
       else
-        leaf_wave<C, DD, 1, UBN, NFT>(c, la);
+        leaf_wave<C, DD, UBN, NFT>(c, la);
     }
   } else {
     const int t = __builtin_amdgcn_readfirstlane((b - nb_near) * 4 + w);
@@ -2230,7 +2199,7 @@ __global__ __launch_bounds__(256) void k_sweep_fly(LeafArgs la, FlyArgs fa, int 
       if constexpr (DD % RowVec<C, float>::RPL == 0)
         leaf_wave_v<C, float, DD, UBN>(c, la);
       else
-        leaf_wave<C, DD, 1, UBN, float>(c, la);
+        leaf_wave<C, DD, UBN, float>(c, la);
     }
   }
 }
@@ -2305,12 +2274,12 @@ void launch_spmv(bool cplx, int nrows, int nrhs, const int* rp, const int* ci, c
 }
 
 bool wave_leaf_supported(int dd) { return dd == 16 || dd == 36; }
-bool wave_coupling_supported(bool cplx, int cd) { return cd == 16 || cd == 25 || (cplx && cd == 32); }
+bool wave_coupling_supported(int cd) { return cd == 16 || cd == 25; }
 
 void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs, int cd, const int2* tgt,
-                           const int* rp, const int* src, const void* F, int64_t fstride, int64_t fcomp,
-                           const int64_t* lvl_off, const double* fw, double* bw, int accumulate, hipStream_t st,
-                           const unsigned short* Fc, int ncoarse, int ld, const PairSweep* pairs) {
+                           const int* rp, const int* src, const void* F, int64_t fstride, const int64_t* lvl_off,
+                           const double* fw, double* bw, hipStream_t st, const unsigned short* Fc, int ncoarse, int ld,
+                           const PairSweep* pairs) {
   if (ld <= 0) ld = cd;
   const int64_t n = static_cast<int64_t>(ntgt) * nrhs * cd;
   if (n == 0) return;
@@ -2319,7 +2288,7 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   // blocks of the coarsest levels are read by the wave kernels only)
   const RowsArgs ra{ntgt, nrhs, cd, ld, 1, tgt, lvl_off, rp, src, F, fstride, fw, 0,
                     static_cast<int64_t>(nrhs) * cd, cd, 1, bw, 0, static_cast<int64_t>(nrhs) * cd, cd, 1,
-                    accumulate, 1, 1};
+                    0, 1, 1};
   if (pairs) return launch_pair_rows(cplx, fp32, ra, *pairs, st);
   auto rows = [&] { launch_block_rows(cplx, fp32, ra, st); };
   if (nrhs > 1 && (!Fc || ncoarse == 0)) return rows();
@@ -2327,7 +2296,7 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   // wave-per-target kernels for the block sizes of the configurations (np 4, 5)
 #define BMI_CPL_W(CC, FTT, CDD)                                                                              \
   if (cplx == CC && fp32 == std::is_same<FTT, float>::value && cd == CDD) {                                  \
-    const CplArgs ca{ntgt, nrhs, tgt, rp, src, F, fstride, fcomp, lvl_off, fw, bw, accumulate, Fc, ncoarse, ld}; \
+    const CplArgs ca{ntgt, nrhs, tgt, rp, src, F, fstride, 0, lvl_off, fw, bw, 0, Fc, ncoarse, ld};  \
     if (nrhs == 1 && variant == 1)                                                                            \
       hipLaunchKernelGGL((k_coupling_w<CC, FTT, CDD, 1, 2>), wgrid, dim3(256), 0, st, ca);                    \
     else if (nrhs == 1)                                                                                       \
@@ -2345,8 +2314,6 @@ void launch_coupling_apply(bool cplx, bool fp32, int variant, int ntgt, int nrhs
   BMI_CPL_W(false, float, 25)
   BMI_CPL_W(true, double, 25)
   BMI_CPL_W(true, float, 25)
-  BMI_CPL_W(true, double, 32)
-  BMI_CPL_W(true, float, 32)
 #undef BMI_CPL_W
   rows();
 }
@@ -2364,11 +2331,11 @@ void launch_leaf(bool cplx, int variant, int ncl, int nrhs, int dd, int vd, cons
     const dim3 wgrid(static_cast<unsigned>((ncl + 3) / 4));
 #define BMI_LEAF_W(CC, DDD)                                                                                     \
   if (cplx == CC && dd == DDD) {                                                                                \
-    const LeafArgs la{ncl, nrhs, rp, src, F, dblk, 0, xs, ldxs, 0, ys, ldys, 0, 0};  /* one component */        \
+    const LeafArgs la{ncl, rp, src, F, dblk, xs, ys};                                                           \
     if (variant == 1)                                                                                           \
-      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1, 2>), wgrid, dim3(256), 0, st, la);                               \
+      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 2>), wgrid, dim3(256), 0, st, la);                               \
     else                                                                                                        \
-      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1, 1>), wgrid, dim3(256), 0, st, la);                               \
+      hipLaunchKernelGGL((k_leaf_w<CC, DDD, 1>), wgrid, dim3(256), 0, st, la);                               \
     BMI_CHECK_HIP(hipGetLastError());                                                                           \
     return;                                                                                                     \
   }
@@ -2463,7 +2430,7 @@ bool launch_sweep_fused(bool cplx, bool fp32, int leaf_variant, int cpl_variant,
                         const int2* tgt, const int* crp, const int* csrc, const void* cF, const int64_t* lvl_off,
                         const double* fw, double* bw, hipStream_t st, const unsigned short* Fc, int ncoarse,
                         bool near32, int ld, const SymList* sym, const SymList* nsym) {
-  const LeafArgs la{ncl, 1, drp, dsrc, dF, static_cast<int64_t>(dd) * dd, 0, xs, 0, 0, ys, 0, 0, 0};
+  const LeafArgs la{ncl, drp, dsrc, dF, static_cast<int64_t>(dd) * dd, xs, ys};
   if (ld <= 0) ld = cd;
   if (sym) {
     // upper blocks only: FP64 blocks, or the FP32 copy padded to whole row vectors
@@ -2518,7 +2485,7 @@ bool launch_sweep_fly(bool cplx, int variant, int ncl, int dd, const int* drp, c
                       const double* xs, double* ys, int ntgt, int cd, const int2* tgt, const int* crp,
                       const int* csrc, const int64_t* lvl_off, const float4* pts, const double4* org,
                       double kre, double kim, const double* fw, double* bw, hipStream_t st) {
-  const LeafArgs la{ncl, 1, drp, dsrc, dF32, static_cast<int64_t>(dd) * dd, 0, xs, 0, 0, ys, 0, 0, 0};
+  const LeafArgs la{ncl, drp, dsrc, dF32, static_cast<int64_t>(dd) * dd, xs, ys};
   const FlyArgs fa{ntgt, tgt, crp, csrc, lvl_off, pts, org, fw, bw, static_cast<float>(kre * 0.5 * M_1_PI),
                    static_cast<float>(kim)};
   const int nbn = (ncl + 3) / 4, nbc = (ntgt + 3) / 4;
