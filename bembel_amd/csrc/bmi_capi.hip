@@ -13,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <sstream>
+#include <system_error>
 #include <thread>
 
 #include "bmi_fmm.h"
@@ -932,7 +933,8 @@ bool h2_is_mixed(const bmi_h2* h) { return h->op.precision != BMI_PRECISION_FP64
 
 // ------------------------------------------------------------------ assembly
 // fn(thread, begin, end) over [0, n) in contiguous ranges, on up to 16 threads with at least `grain`
-// items each; an exception of any of them is rethrown here.
+// items each; an exception of any of them is rethrown here, and one of a thread that cannot be started does not
+// leave with others running.
 template <class F>
 static void parallel_ranges(int64_t n, int64_t grain, F&& fn) {
   const int nth = static_cast<int>(std::max<int64_t>(
@@ -947,8 +949,14 @@ static void parallel_ranges(int64_t n, int64_t grain, F&& fn) {
     }
   };
   std::vector<std::thread> pool;
-  for (int t = 1; t < nth; ++t) pool.emplace_back(work, t);
+  pool.reserve(nth);
+  int started = 1;  // ranges without a thread (none to be had) are done here
+  try {
+    for (; started < nth; ++started) pool.emplace_back(work, started);
+  } catch (const std::system_error&) {
+  }
   work(0);
+  for (int t = started; t < nth; ++t) work(t);
   for (auto& th : pool) th.join();
   for (const std::string& e : errors) BMI_REQUIRE(e.empty(), BMI_UNSUPPORTED, e);
 }
