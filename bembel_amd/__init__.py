@@ -588,9 +588,12 @@ class H2Matrix:
         _check(library().bmi_h2_use_graphs(self._h, 1 if enable else 0))
 
     def set_sweep(self, mode):
-        """Sweep of single-RHS products: None (timed choice, default), "full" (every block),
-        "upper" (upper coupling blocks of a symmetric kernel with the transposed products formed
-        from them) or "upper_near" (the same for the near-field leaves too)."""
+        """Which blocks products read.  None (default): single-RHS products of the block sizes with fused
+        sweeps time the forms below once and keep the fastest; other sizes, and Maxwell, read one coupling
+        block of each symmetric pair where that pays (at most 16 real, 8 complex or 2 Maxwell columns).
+        "full": every block, in all of these products.  "upper": single-RHS products read the upper
+        coupling blocks of a symmetric kernel and form the transposed products from them; "upper_near":
+        the same for the near-field leaves too (both refused for sizes without fused sweeps)."""
         m = {None: -1, "full": 0, "upper": 1, "upper_near": 2}[mode]
         _check(library().bmi_h2_set_sweep(self._h, m))
 

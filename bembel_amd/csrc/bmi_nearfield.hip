@@ -17,9 +17,9 @@
 //
 // Measured, 24,576 elements of the sphere, P 2, 13 points per direction for touching pairs, against
 // points in Bernstein form, blocks in registers and the library's sine and cosine: Laplace identical 58.0
-// -> 22.7 ms, edge 97.0 -> 40.7, vertex 18.6 -> 17.6, regular 16.6 -> 15.9; Helmholtz identical 82.5 ->
-// 30.8, edge 149.5 -> 69.8, vertex 54.7 -> 47.7, regular 35.7 -> 31.7 (VALU busy: identical 0.76, edge
-// 0.71, vertex 0.65, regular 0.60).
+// -> 22.7 ms, edge 97.0 -> 41.3, vertex 18.6 -> 17.6, regular 16.6 -> 15.9; Helmholtz identical 82.5 ->
+// 29.3, edge 149.5 -> 69.2, vertex 54.7 -> 46.4, regular 35.7 -> 30.8 (VALU busy: Laplace identical 0.77, edge
+// 0.71, vertex 0.69, regular 0.60).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -149,9 +149,9 @@ __device__ __forceinline__ void pot_tile(const double* tile, int cnt, double x0,
 
 // partial[chunk][comp][point] (complex interleaved for C) = sum over the chunk's sources.  Bound by the
 // FP64 vector units: the distance and its reciprocal root, the phase's sine and cosine and the complex
-// multiply-add, 68 instructions per target and source of the Helmholtz layer (with the library's sqrt,
-// division, sincos and exp it was 185).  The phase's range is checked once per tile, from |x| and |y|
-// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.49 ms; error
+// multiply-add, 62 instructions per target and source of the Helmholtz layer (SQ_INSTS_VALU; with the
+// library's sqrt, division, sincos and exp 185 in the loop).  The phase's range is checked once per tile, from |x| and |y|
+// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.48 ms; error
 // 1.7e-15 -> 0.7e-15, and below the former for few sources too (the roots and sums rounded for speed alone,
 // 1.44 ms, were up to 1.45 times further off than it for 864 to 6,144 sources).
 template <int KIND>

@@ -45,35 +45,42 @@ def log(*a):
     print("[bench]", *a, file=sys.stderr, flush=True)
 
 
+def seven_digits(o):
+    """o with every float at seven significant digits"""
+    if isinstance(o, dict):
+        return {k: seven_digits(v) for k, v in o.items()}
+    if isinstance(o, (list, tuple)):
+        return [seven_digits(v) for v in o]
+    return float("%.7g" % o) if isinstance(o, float) else o
+
+
 def pct(a, q):
     return float(np.percentile(np.asarray(a), q))
 
 
 def nearfield_flops(classes_deg, P, pd, cplx=False):
-    """Algorithmic FP64 flops of the Duffy pairs as the rules compute them, n Gauss points per
-    direction.  Identical: 8 n^4 surface points, 4 n^4 kernel values, each added to the block and
-    to its transpose ((P+1)^4 updates each).  Edge (factorised): 6 n^4 evaluations, each adding kernel x basis to a
-    (P+1)^2 vector, one outer product per outer point (6 n^3), 8 n^3 tabulated surface points, 4 n^3
-    contracted patch lines and 4 n^4 points on them.  Vertex (factorised): 4 n^4 evaluations into
-    vectors, 4 n^2 outer products, 4 n^2 + 2 n^3 surface points."""
-    I2 = (P + 1) ** 2
+    """FP64 flops of the Duffy pairs as the rules compute them (a multiply-add is two), n Gauss points per
+    direction.  Identical: 4 n^2 contracted lines, 8 n^4 points on them, 4 n^4 kernel values into (P+1)^2
+    sums, 2 n^3 outer products.  Edge: 6 n^4 kernel values into P+1 sums, 6 n^3 outer products, 4 n^4 + 4 n^3
+    points on 4 n^3 contracted lines, 4 n^3 surface points.  Vertex: 4 n^4 kernel values into (P+1)^2 sums,
+    4 n^2 outer products, 4 n^2 + 2 n^3 surface points."""
+    I, I2 = P + 1, (P + 1) ** 2
     c = 2 if cplx else 1
-    Fk = 40 if cplx else 20                   # kernel value (distance, 1/r, sincos)
-    Fe = 2 * I2 * I2 * c + I2                 # full block update of one evaluation
-    Fv = I2 + 2 * I2 * c + 6 * (P + 1)        # basis vector and its accumulation
+    Fk = 80 if cplx else 25                   # kernel value (distance, reciprocal root; root, sine, cosine)
     Fo = 2 * I2 * I2 * c                      # outer product of two basis vectors
-    Fg = 16 * pd * pd + 24 * pd + 90          # surface point with both tangents (2-D patch evaluation)
-    Fl = 16 * pd * pd + 20                    # patch contracted to a line (values and cross derivatives)
-    F1 = 24 * pd + 60                         # point on a contracted line
+    Fg = 16 * pd * pd + 16 * pd + 50          # surface point with both tangents and its measure
+    Fl = 16 * pd * pd - 8 * pd                # element contracted to a line (values and cross derivatives)
+    F1 = 24 * pd + 13                         # point on a contracted line
     tot = 0.0
     for cls, n, cnt in classes_deg:
         n = float(n)
         if cls == 2:
-            f = 8 * n ** 4 * (Fe + Fg) + 4 * n ** 4 * Fk
+            f = 4 * n ** 2 * Fl + 8 * n ** 4 * F1 + 4 * n ** 4 * (Fk + 2 * I2 * c + I * c) + 2 * n ** 3 * Fo
         elif cls == 3:
-            f = 6 * n ** 4 * (Fk + Fv) + 6 * n ** 3 * Fo + 8 * n ** 3 * Fg + 4 * n ** 3 * Fl + 4 * n ** 4 * F1
+            f = 6 * n ** 4 * (Fk + 2 * I * c + 3 * I) + 6 * n ** 3 * (Fo + I2 * (1 + c)) + \
+                4 * n ** 3 * (Fg + Fl) + (4 * n ** 4 + 4 * n ** 3) * F1
         else:
-            f = 4 * n ** 4 * (Fk + Fv) + 4 * n ** 2 * Fo + (4 * n ** 2 + 2 * n ** 3) * Fg
+            f = 4 * n ** 4 * (Fk + I2 + 2 * I2 * c + 6 * I) + 4 * n ** 2 * Fo + (4 * n ** 2 + 2 * n ** 3) * Fg
         tot += cnt * f
     return tot
 
@@ -453,9 +460,9 @@ def run_serving(B, torch, rng, nreq, rate=8.0, pool=12):
            "precision": "mixed (FP32 reduced operator, FP64 refinement)", "tol": 1e-6,
            "scheduling": "up to 4 batches admitted; each GMRES batch a task on its own stream, all driven by one "
                          "device thread, so the batches overlap on the device",
-           "mix": [{"M": r["M"], "P": r["P"], "helmholtz": r["helm"], "nrhs": r["nrhs"], "latency_s": i["latency_s"],
-                    "iterations": i["iterations"], "batch_requests": i["batch_requests"], "status": i["status"]}
-                   for r, i in zip(reqs, infos)]}
+           # requests by operator and refinement (one entry per request made the line longer than a log's tail)
+           "mix": {"%s M%d" % ("helmholtz" if h else "laplace", m): sum(1 for r in reqs if (r["helm"], r["M"]) == (h, m))
+                   for h, m in sorted({(r["helm"], r["M"]) for r in reqs})}}
     log("serving: %d requests (%d ok) in %.1f s, p50 %.2f s, p99 %.2f s, %.2f solves/s, %d batched, %d cache hits" % (
         nreq, ok, wall, out["p50_latency_s"], out["p99_latency_s"], out["solves_per_s"], out["batched_requests"],
         out["operator_cache_hits"]))
@@ -683,7 +690,8 @@ def cpu_serving(O, reqs, infos, rng, threads, budget_s=20.0):
     tot = sum(d["cpu_s"] for d in done)
     log("serving CPU sample: %d requests, %.1f s serial (%.2f solves/s)" % (len(done), tot, len(done) / tot))
     return {"cores": threads, "kind": "port", "requests": len(done), "serial_s": tot, "solves_per_s": len(done) / tot,
-            "p50_request_s": pct([d["cpu_s"] for d in done], 50), "sampled": done,
+            "p50_request_s": pct([d["cpu_s"] for d in done], 50),
+            "gpu_p50_of_these_s": pct([d["gpu_latency_s"] for d in done], 50),
             "sample": "requests with M <= 4 of the same stream, each solved alone by the oracle (assembly + "
                       "GMRES(100) to 1e-6 per right-hand side, FP64), until %.0f s were spent" % budget_s}
 
@@ -968,7 +976,7 @@ def main():
         "serving": serving,
         "build": B.build_info(),
     }
-    print(json.dumps(out), flush=True)
+    print(json.dumps(seven_digits(out)), flush=True)
 
 
 if __name__ == "__main__":

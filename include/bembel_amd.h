@@ -179,11 +179,15 @@ bmi_status bmi_h2_matvec(const bmi_h2* h, int nrhs, const double* X, int64_t ldx
    than its few launches save).  No counterpart in the reference (its product is CPU code);
    exposed so callers can compare both modes. */
 bmi_status bmi_h2_use_graphs(bmi_h2* h, int enable);
-/* Sweep of single-RHS products: -1 (default) lets the first product time the forms and keep
-   the fastest, 0 reads every block, 1 reads only the upper coupling blocks of a symmetric kernel
-   (Laplace, Helmholtz) and forms the transposed products from them, 2 does the same for the
-   near-field leaves as well (BMI_UNSUPPORTED where a form is not available).  No counterpart in
-   the reference (its product is CPU code); exposed so callers can compare the forms. */
+/* Which blocks products read.  -1 (default): single-RHS products of the block sizes with fused sweeps let
+   the first product time the forms and keep the fastest; other sizes, and Maxwell, read one coupling block
+   of each symmetric pair where a rule on bytes says that this pays (products of at most one column tile:
+   16 real, 8 complex, 2 Maxwell columns).  0: every block, in all of these products.  1: only the upper
+   coupling blocks of a symmetric kernel (Laplace, Helmholtz) in single-RHS products, with the transposed
+   products formed from them; 2: the same for the near-field leaves as well.  1 and 2 are BMI_UNSUPPORTED
+   for sizes without fused sweeps, also where -1 reads pairs.  Products of more columns than a tile, and
+   bmi_h2_matvec_noalloc of those other sizes, read every block in every mode.  No counterpart in the
+   reference (its product is CPU code); exposed so callers can compare the forms. */
 bmi_status bmi_h2_set_sweep(bmi_h2* h, int mode);
 /* Single-RHS products on the handle's workspace: -1 (default) lets the first product time both
    forms and keep the faster, 0 runs the near-field leaves and coupling blocks in one launch after
