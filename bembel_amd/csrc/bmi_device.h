@@ -122,11 +122,14 @@ __device__ __forceinline__ double rsqrt_newton_any(double s) {
   return __builtin_amdgcn_class(y0, 0x240) ? y0 : rsqrt_newton(s);  // +infinity, +0
 }
 
-// sqrt(s) from y = rsqrt_newton(s): s y corrected once by its residual.  s y alone is off by up to two ulps,
-// which a phase kappa r multiplies by its size
-__device__ __forceinline__ double sqrt_newton(double s, double y) {
-  const double r = s * y;
-  return fma(0.5 * y, fma(-r, r, s), r);
+// y = 1 / sqrt(s) as above and r = sqrt(s): s y corrected once by its residual, with the half of the iterate before
+// (s y alone is off by up to two ulps, which a phase kappa r multiplies by its size)
+__device__ __forceinline__ void rsqrt_sqrt_newton(double s, double& y, double& r) {
+  const double y0 = __builtin_amdgcn_rsq(s);
+  const double y1 = fma(0.5 * y0, fma(-(s * y0), y0, 1.0), y0), h = 0.5 * y1;
+  y = __builtin_amdgcn_class(y0, 0x240) ? y0 : fma(h, fma(-(s * y1), y1, 1.0), y1);
+  r = s * y;
+  r = fma(h, fma(-r, r, s), r);
 }
 
 // a b + c with the constant c in scalar registers: from vector registers the compiler copies it first,

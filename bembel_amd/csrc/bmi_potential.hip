@@ -98,24 +98,26 @@ __global__ __launch_bounds__(256) void k_pot_sources(const double* __restrict__ 
 template <int KIND, bool FAR, bool DECAY, int DIM>
 __device__ __forceinline__ void pot_tile(const double* tile, int cnt, double x0, double x1, double x2, double kre,
                                          double kim, double (&sr)[DIM], double (&si)[DIM]) {
-  // 64 sources have sums of their own, added at the end: a multiply-add of complex factors rounds twice at
-  // the size of the sum, which one sum per tile showed as 1.4 times the error (864 sources: 5.9e-16 with
-  // products rounded first, 8.5e-16 without)
-  for (int j0 = 0; j0 < cnt; j0 += 64) {
+  // the tile's own sums, added at the end; complex ones of 64 sources: a multiply-add of complex factors rounds twice
+  // at the size of the sum, which one sum per tile showed as 1.4 times the error (864 sources: 5.9e-16 with
+  // products rounded first, 8.5e-16 without).  A real one rounds once, and shorter loops would cost the Laplace
+  // layer its pipelining (192 targets, 3,456 sources: 73 us so, 85 us with 64)
+  constexpr int SUM = KIND == BMI_LAPLACE_SL ? POT_TILE : 64;
+  for (int j0 = 0; j0 < cnt; j0 += SUM) {
     double ar[DIM], ai[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; ++d) ar[d] = 0.0, ai[d] = 0.0;
-    const int j1 = j0 + 64 < cnt ? j0 + 64 : cnt;
+    const int j1 = j0 + SUM < cnt ? j0 + SUM : cnt;
     for (int j = j0; j < j1; ++j) {
       const double* sj = tile + j * PotSrc<KIND>::N;
       const double d0 = x0 - sj[0], d1 = x1 - sj[1], d2 = x2 - sj[2];
       const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      const double ir = rsqrt_newton_any(r2);  // infinite where the target is the source
       if constexpr (KIND == BMI_LAPLACE_SL) {
-        ar[0] += ir * sj[3];
+        ar[0] += rsqrt_newton_any(r2) * sj[3];  // infinite where the target is the source
       } else {
         // exp(-i kappa r) / r = exp(kim r) (cos(kre r) - i sin(kre r)) / r
-        const double r = sqrt_newton(r2, ir);
+        double ir, r;
+        rsqrt_sqrt_newton(r2, ir, r);
         double sn, cs;
         if constexpr (FAR)
           sincos_phase(kre * r, &sn, &cs);
@@ -149,9 +151,9 @@ __device__ __forceinline__ void pot_tile(const double* tile, int cnt, double x0,
 
 // partial[chunk][comp][point] (complex interleaved for C) = sum over the chunk's sources.  Bound by the
 // FP64 vector units: the distance and its reciprocal root, the phase's sine and cosine and the complex
-// multiply-add, 62 instructions per target and source of the Helmholtz layer (SQ_INSTS_VALU; with the
+// multiply-add, 61 instructions per target and source of the Helmholtz layer (SQ_INSTS_VALU; with the
 // library's sqrt, division, sincos and exp 185 in the loop).  The phase's range is checked once per tile, from |x| and |y|
-// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.48 ms; error
+// (their sum bounds r).  6,000 targets, 98,304 sources, real kappa: 3.09 -> 1.46 ms; error
 // 1.7e-15 -> 0.7e-15, and below the former for few sources too (the roots and sums rounded for speed alone,
 // 1.44 ms, were up to 1.45 times further off than it for 864 to 6,144 sources).
 template <int KIND>
